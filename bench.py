@@ -1,7 +1,8 @@
 """Benchmark: D2Q9 TRT Taylor-Green vortex, periodic 4096 x 4096, on one MI355X.
 
 A step is one time step of the lattice (collide -> stream -> BCs) over the
-whole 4096^2 lattice, i.e. one fused pull collide-stream kernel launch.
+whole 4096^2 lattice; the library's kernels advance one or several steps per
+pass over it.
 ``value`` is the plain FP64 throughput in MLUPS (million lattice updates per
 second) over K timed steps, populations resident in HBM.  The same run with
 each reduced storage (FP16/BF16 non-equilibrium records, FP16/BF16
@@ -10,8 +11,10 @@ relative L2 velocity error against the FP64 run.
 
 ``roofline`` prices the fused kernel against MI355X's 8 TB/s: algorithmic
 bytes per launch = 2 * Q * sizeof(population) * nodes (one read and one write
-of every population), divided by the kernel's average duration measured with
-HIP events on the library's stream.
+of every population per pass, however many steps the pass advances:
+``steps_per_pass``), divided by the kernel's average duration measured with
+HIP events on the library's stream.  The ``spread`` entries are of runs with
+one step per launch.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--n 4096]
 """
@@ -46,6 +49,9 @@ def tgv_populations(L, q, n, u0=0.02):
 # the Taylor-Green workload's length: the accuracy of every storage is taken
 # after this many steps, whatever --steps is
 ACCURACY_STEPS = 5000
+# time steps a kernel of the timed runs advances per pass over the lattice (the
+# library's several-step kernels at this size; the deviation storages: one)
+STEPS_PER_PASS = {"f64": 5, "f32": 6, "f16neq": 4, "bf16neq": 4, "f16dev": 1, "bf16dev": 1}
 # fused launches timed one by one for the spread of the kernel's duration
 SPREAD_LAUNCHES = 200
 # back-to-back device copies of the FP64 lattice for the copy-rate ceiling
@@ -380,7 +386,8 @@ def mrt_leg(L, steps=20):
     """Regularised MRT (mrt.jl:56-118) in FP64 on the periodic Taylor-Green
     vortex, D2Q9 at 4096^2 and D2Q17 / D2Q37 at 8192 x 2048, all relaxation
     times 0.8, beside SRT(0.8) on the same lattice: kernel time per step from
-    HIP events and the fraction of 8 TB/s at 2 Q 8 bytes per node."""
+    HIP events and the fraction of 8 TB/s at 2 Q 8 bytes per node and step (more
+    than what moves where a pass advances several steps)."""
     rows = []
     for qid, nx, ny in ((9, 4096, 4096), (17, 8192, 2048), (37, 8192, 2048)):
         q = L.Quadratures[f"D2Q{qid}"]()
@@ -414,8 +421,8 @@ def mrt_leg(L, steps=20):
 def sizes_leg(L, sizes, steps=20):
     """D2Q9 TRT(0.8, 1.1) on periodic n x n lattices (uniform flow 0.01 along
     x, equilibrium start) in FP64 and FP32: kernel time per step from HIP
-    events and algorithmic GB/s (2 Q sizeof per node).  Rows of whole 128-byte
-    lines run the row-shaped kernel, other widths the flat-index one."""
+    events and algorithmic GB/s (2 Q sizeof per node and step; several steps
+    share a pass)."""
     q = L.D2Q9()
     rows = []
     for n in sizes:
@@ -430,7 +437,6 @@ def sizes_leg(L, sizes, steps=20):
             us = ms / max(nl, 1) * 1e3
             gbs = 2 * q.Q * eb * n * n / (us * 1e-6) / 1e9
             rows.append({"lattice": [n, n], "storage": storage,
-                         "kernel": "row-shaped" if (n * eb) % 128 == 0 else "flat-index",
                          "us_per_step": round(us, 1), "achieved_GBps": round(gbs, 1),
                          "frac": round(gbs / HBM_PEAK_GBS, 4)})
             del m
@@ -562,7 +568,8 @@ def main():
     mlups64 = nodes * K / wall64 / 1e6
     bytes64 = 2 * q.Q * 8 * nodes
     kavg64 = kms64 / max(nl64, 1)
-    gbs64 = bytes64 / (kavg64 * 1e-3) / 1e9
+    spp64 = STEPS_PER_PASS["f64"]
+    gbs64 = bytes64 / (kavg64 * spp64 * 1e-3) / 1e9
     spread64 = launch_spread(L, m64)
     copy_s = copy_rate(L, m64.f_stream)
     copy_gbs = bytes64 / copy_s / 1e9
@@ -597,8 +604,9 @@ def main():
             "unit": "GB/s",
             "frac": round(gbs64 / HBM_PEAK_GBS, 4),
             "traffic": traffic_for("d2q9_trt_f64_4096"),
-            "kernel": "k_fused_v<9,TRT,F64> (128x2 blocks, 1 node/thread, non-temporal stores)",
-            "kernel_ms_avg": round(kavg64, 5),
+            "kernel": "k_march<9,TRT,F64> (marching waves, five steps per pass)",
+            "kernel_ms_avg": round(kavg64 * spp64, 5),
+            "steps_per_pass": spp64,
             "bytes_per_launch": bytes64,
             "shader_clock_mhz": _r(clk64),
             "spread": spread64,
@@ -615,13 +623,13 @@ def main():
         # record (*neq: 2 Q + 8 bytes per node), rest-state deviations (*dev),
         # and shifted FP32
         kernels = {
-            "f16neq": "k_fused_neq_rows2<9,TRT,F16Neq> (two columns x 2 rows per lane, LDS "
-                      "record window, edge nodes in its last block column)",
-            "bf16neq": "k_fused_neq_rows2<9,TRT,BF16Neq> (two columns x 2 rows per lane, LDS "
-                       "record window, edge nodes in its last block column)",
+            "f16neq": "k_march<9,TRT,F16Neq> (marching waves, two columns per lane, four steps "
+                      "per pass)",
+            "bf16neq": "k_march<9,TRT,BF16Neq> (marching waves, two columns per lane, four "
+                       "steps per pass)",
             "f16dev": "k_fused_v<9,TRT,F16Dev> (4 nodes/thread)",
             "bf16dev": "k_fused_v<9,TRT,BF16Dev> (4 nodes/thread)",
-            "f32": "k_fused_v<9,TRT,F32> (256x1 blocks, 1 node/thread)",
+            "f32": "k_march<9,TRT,F32> (marching waves, six steps per pass)",
         }
         for storage, key, per_node in (("f16neq", "fp16neq", 2 * q.Q + 8),
                                        ("f16dev", "fp16dev", 2 * q.Q),
@@ -633,7 +641,8 @@ def main():
             mlups16 = nodes * K / wall16 / 1e6
             bytes16 = 2 * per_node * nodes
             kavg16 = kms16 / max(nl16, 1)
-            gbs16 = bytes16 / (kavg16 * 1e-3) / 1e9
+            spp16 = STEPS_PER_PASS[storage]
+            gbs16 = bytes16 / (kavg16 * spp16 * 1e-3) / 1e9
             spread16 = launch_spread(L, m16)
             del m16
             result[key] = {
@@ -648,7 +657,8 @@ def main():
                              "unit": "GB/s", "frac": round(gbs16 / HBM_PEAK_GBS, 4),
                              "traffic": traffic_for(f"d2q9_trt_{storage}_4096"),
                              "kernel": kernels[storage],
-                             "kernel_ms_avg": round(kavg16, 5), "bytes_per_launch": bytes16,
+                             "kernel_ms_avg": round(kavg16 * spp16, 5),
+                             "steps_per_pass": spp16, "bytes_per_launch": bytes16,
                              "shader_clock_mhz": _r(clk16), "spread": spread16},
             }
 

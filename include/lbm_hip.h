@@ -184,13 +184,15 @@ int lbm_model_set_bcs(lbm_model m, const lbm_bc *bcs, int n);
  * distinct Hermite components; periodic lattices with nx a multiple of 16,
  * other cases return an error; parity with the oracle to 1e-12 relative
  * instead of bit for bit).  It is opt-in: on MI355X it is slower than the
- * default vector kernel.  No counterpart in the reference (a CPU loop has no
- * launch shape). */
+ * default vector kernel.  A shape other than the automatic one also selects
+ * one fused step per launch (lbm_simulate).  No counterpart in the reference
+ * (a CPU loop has no launch shape). */
 int lbm_model_set_launch(lbm_model m, int block_x, int rows_per_block, int nodes_per_thread,
                          int nontemporal);
-/* Autotuner: times every launch shape of the fused step for this model on
- * scratch copies of f_stream (the caller's fields are not advanced), keeps
- * the fastest in the model and returns it.  No counterpart in the reference. */
+/* Autotuner: times every launch shape of the fused step for this model, and
+ * the several-step kernels where lbm_simulate has them, on scratch copies of
+ * f_stream (the caller's fields are not advanced), keeps the fastest in the
+ * model and returns it (the automatic shape for the several-step kernels).  No counterpart in the reference. */
 int lbm_autotune(lbm_model m, lbm_field f_stream, int trial_steps, int *block_x,
                  int *rows_per_block, int *nodes_per_thread, int *nontemporal,
                  double *us_per_step);
@@ -207,18 +209,23 @@ int lbm_apply_bcs(lbm_model m, lbm_field f_new, lbm_field f_old);
 /* stream! then apply!, as one pass */
 int lbm_stream_bc(lbm_model m, lbm_field f, lbm_field f_new);
 /* simulate(model, t0:t0+nsteps-1) without processing -- lattice_boltzmann_model.jl:60-77:
- * nsteps x (collide! f_stream -> f_collision; stream! + apply!) with one fused
- * pull collide-stream kernel per step.  On return both buffers hold exactly
- * what the reference's model.f_stream / model.f_collision hold. */
+ * nsteps x (collide! f_stream -> f_collision; stream! + apply!) with fused pull
+ * collide-stream kernels.  With the automatic launch shape, D2Q4/5/9 models in
+ * storage F64, F32, F16NEQ or BF16NEQ advance several steps per kernel (the
+ * 16-bit storages on even widths from 800,000 nodes up; they then round to 16
+ * bits once per pass instead of once per step); everything else runs one
+ * kernel per step.  On return both buffers hold exactly what the reference's
+ * model.f_stream / model.f_collision hold. */
 int lbm_simulate(lbm_model m, lbm_field f_stream, lbm_field f_collision, int64_t nsteps);
 /* As lbm_simulate, also returning the time of the fused kernels (HIP events on
- * the library stream): *ms_total over the fused launches of the run, *nlaunch
- * their number (nsteps - 1, or nsteps - 2 where the first step runs as one
- * collide + fused pass: D2Q4/5/9 on lattices of whole 64 x 8 tiles). */
+ * the library stream): *ms_total over the fused launches of the run after the
+ * first, *nlaunch the number of steps they advance (nsteps less the steps of
+ * the first pass, which starts from the canonical state: one, or as many as a
+ * several-step pass holds). */
 int lbm_simulate_timed(lbm_model m, lbm_field f_stream, lbm_field f_collision, int64_t nsteps,
                        double *ms_total, int64_t *nlaunch);
-/* Measurement support; no counterpart in the reference.  As lbm_simulate,
- * with a HIP event before every fused launch: launch_ms[k] (nsteps - 1
+/* Measurement support; no counterpart in the reference.  As lbm_simulate with
+ * one fused step per launch and a HIP event before every fused launch: launch_ms[k] (nsteps - 1
  * entries) is the time from the start of fused launch k to the start of the
  * next (the last: to the end of the last), *nlaunch the number of entries. */
 int lbm_simulate_launch_times(lbm_model m, lbm_field f_stream, lbm_field f_collision,

@@ -61,6 +61,8 @@ def _deps(src):
                 os.path.join(REPO, "include", "lbm_hip.h")]
     if src == "lbm_dispatch.cpp":
         return [os.path.join(CSRC, "lbm_internal.h")]
+    if src.startswith("k_multi"):
+        return kern + [os.path.join(CSRC, "lbm_multi.h")]
     if src.startswith("k_adjoint"):
         return kern + [os.path.join(CSRC, "lbm_adjoint.h")]
     return kern
@@ -84,7 +86,8 @@ def build(force: bool = False, verbose: bool = False) -> str:
             continue
         jobs.append((src, [HIPCC, *COMMON, *flags, "-c", s, "-o", o]))
     # heaviest units first, at most one hipcc per CPU
-    jobs.sort(key=lambda j: (not j[0].startswith("k_"), "q37" not in j[0], j[0]))
+    jobs.sort(key=lambda j: (not j[0].startswith("k_"),
+                             "q37" not in j[0] and "multi_f" not in j[0], j[0]))
     width = max(1, min(len(jobs), os.cpu_count() or 1, 16))
     procs = []
     failed = []

@@ -1,0 +1,7 @@
+// k_multi_f64_q9.hip -- several fused steps per pass, storage f64, D2Q9.
+// Plain FP64: compiled with -ffp-contract=off (bit-exact with the CPU restatement).
+#include "lbm_multi.h"
+
+namespace lbm {
+LBM_DEFINE_MULTI(f64, StF64, 9)
+}  // namespace lbm

@@ -506,6 +506,121 @@ int run(lbm::Op op, lbm_model m, lbm_field src, lbm_field dst, bool with_bcs) {
     return 0;
 }
 
+// ---- several steps per pass ---------------------------------------------------
+// The pass sizes a run of collisions is split into (lbm_multi.h's kernels).
+struct MultiPlan {
+    int kernel = lbm::kMultiNone;
+    int max_steps = 1;
+    // relative cost of a pass of k steps (0: not available), k = 1 the single-step kernel
+    double cost[9] = {};
+};
+
+// Which kernel advances this model several steps at a time.  D2Q4/5/9, storages
+// F64, F32 and the non-equilibrium ones, automatic launch shape (a launch
+// shape set by the caller names a single-step kernel).  Measured on MI355X,
+// D2Q9 TRT, us per step (single-step kernel -> the one chosen):
+//   FP64: 64^2 4.5 -> 1.1 and 128^2 4.8 -> 1.3 (8 x 8 tiles, 8 steps);
+//     257^2 5.4 -> 2.6 (64 x 16 blocks); 512^2 10.3 -> 4.1 (64 x 32 blocks);
+//     1024^2 33.8 -> 12.3 (wide blocks; marching waves 16.1);
+//     2048^2 116 -> 41 (marching waves; wide blocks 50); 4096^2 413 -> 130;
+//   FP32: 64^2 4.0 -> 0.8; 257^2 4.5 -> 1.6; 512^2 6.0 -> 2.3; 1024^2 17.6 ->
+//     6.1 (march 7.6); 2048^2 64 -> 18 (blocks 20.5); 4096^2 218 -> 57;
+//   FP16-NEQ: 4096^2 194 -> 71 (two columns per lane: even widths).
+// (below this the 16-bit storages keep the single-step row kernel)
+constexpr long long kNeqMarchNodes = 800000;
+
+MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
+    MultiPlan pl;
+    if (m->launch_block || m->launch_rows || m->launch_vec || m->launch_nt >= 0) {
+        // a shape set by the caller names a single-step kernel, unless it is
+        // the automatic one (what lbm_autotune returns when this path wins)
+        lbm_model_s def;
+        def.coll = m->coll;
+        int b, r, v, nt, b0, r0, v0, nt0;
+        auto_launch(m, f, b, r, v, nt);
+        auto_launch(&def, f, b0, r0, v0, nt0);
+        if (b != b0 || r != r0 || v != v0 || nt != nt0) return pl;
+    }
+    if (m->qid != 4 && m->qid != 5 && m->qid != 9) return pl;
+    if (m->coll != LBM_SRT && m->coll != LBM_TRT &&
+        !(m->coll == LBM_MRT && f->storage == LBM_STORE_F64))
+        return pl;
+    const long long nodes = (long long)f->nx * f->ny;
+    auto any_up_to = [&](int kernel, int t) {
+        pl.kernel = kernel;
+        pl.max_steps = t;
+        // a pass costs about 2 + k units up to its largest size
+        for (int k = 1; k <= t; ++k) pl.cost[k] = 2.0 + k;
+    };
+    // waves and blocks are 64 columns wide and recompute a halo of rows: a
+    // lattice much narrower or lower than that spends its time on nodes that
+    // are not written, and the single-step kernel is faster (FP64 at 32
+    // columns: blocks 7 us against 10 for 270,000 nodes; at 24 they lose)
+    const bool wide = f->nx >= 32 && f->ny >= 12;
+    if (rows_mode(f->storage)) {
+        if (f->nx % 2 || f->nx < 64 || !wide || nodes < kNeqMarchNodes) return pl;
+        pl.kernel = lbm::kMultiMarch;
+        pl.max_steps = 4;
+        const double c[5] = {0, 194, 226, 254, 285};
+        for (int k = 1; k <= 4; ++k) pl.cost[k] = c[k];
+        return pl;
+    }
+    const bool f64 = f->storage == LBM_STORE_F64;
+    if (!f64 && f->storage != LBM_STORE_F32) return pl;
+    // (420 tiles: 164 x 164, FP64 160^2 2.0 us against 1.9 with the 64 x 16 blocks)
+    const long long tiles = (long long)((f->nx + 7) / 8) * ((f->ny + 7) / 8);
+    if (tiles <= 420) any_up_to(lbm::kMultiTile, 8);
+    else if (!wide) return pl;
+    else if (nodes <= 90000) any_up_to(lbm::kMultiBlock16, 6);
+    else if (nodes <= 400000) any_up_to(lbm::kMultiBlock32, 6);
+    else if (nodes <= 2000000) any_up_to(lbm::kMultiBlockWide, f64 ? 5 : 6);
+    else {
+        pl.kernel = lbm::kMultiMarch;
+        pl.max_steps = f64 ? 5 : 6;
+        const double c64[6] = {0, 413, 500, 530, 590, 650};
+        const double c32[7] = {0, 218, 260, 280, 295, 0, 341};
+        for (int k = 1; k <= pl.max_steps; ++k) pl.cost[k] = f64 ? c64[k] : c32[k];
+    }
+    return pl;
+}
+
+// the next pass of a run with `left` collisions to go: the first of the
+// cheapest split (exact for the last 32; before them the largest pass)
+int multi_next(const MultiPlan &pl, int64_t left) {
+    constexpr int N = 32;
+    if (left > N) return pl.max_steps;
+    double best[N + 1] = {};
+    int pass[N + 1] = {};
+    for (int n = 1; n <= (int)left; ++n) {
+        best[n] = 1e300;
+        for (int k = 1; k <= pl.max_steps && k <= n; ++k)
+            if (pl.cost[k] > 0 && best[n - k] + pl.cost[k] <= best[n]) {
+                best[n] = best[n - k] + pl.cost[k];
+                pass[n] = k;
+            }
+    }
+    return pass[left];
+}
+
+int run_multi(const MultiPlan &pl, lbm_model m, lbm_field src, lbm_field dst, int steps, bool first) {
+    lbm::MultiLaunch L{};
+    L.kernel = pl.kernel;
+    L.qid = m->qid;
+    L.coll = m->coll;
+    L.steps = steps;
+    L.first = first ? 1 : 0;
+    for (size_t b = 0; b < m->bcs.size(); ++b) {
+        L.walls |= 1 << m->bcs[b].direction;
+        if (m->bcs[b].kind == LBM_MOVING_WALL) L.moving = (int)b;
+    }
+    L.src = src->d;
+    L.dst = dst->d;
+    const int rc = lbm::dispatch_multi(src->storage, L, make_params(m, src, true), g_stream);
+    if (rc) return fail(-4, "kernel launch failed (code %d): %s", rc,
+                        hipGetErrorString(hipGetLastError()));
+    return 0;
+}
+
 void free_dev(void *&p) {
     if (p) {
         (void)hipFree(p);
@@ -1008,23 +1123,30 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
         if (nlaunch) *nlaunch = 2 * nsteps;
         return 0;
     }
-    // step 1 starts from the canonical state S.  One-speed stencils on
-    // lattices of whole 64 x 8 tiles (every storage) take
-    // C_1 = collide(BC(stream(collide(S_0)))) in one pass (k_fused_first*:
-    // one pass over HBM instead of collide! plus the first fused step);
-    // otherwise C_0 = collide(S_0) first.  Runs that
+    // Runs that time every launch keep one fused step per launch; the others
+    // advance several collisions per pass where a kernel for it exists.
+    const MultiPlan plan = per_launch ? MultiPlan{} : multi_plan(m, S);
+    const bool multi = plan.kernel != lbm::kMultiNone && nsteps >= 2;
+    // step 1 starts from the canonical state S: the first pass collides S_0 in
+    // place.  Without a several-step kernel, one-speed stencils on lattices of
+    // whole 64 x 8 tiles take C_1 = collide(BC(stream(collide(S_0)))) in one
+    // pass (k_fused_first*); otherwise C_0 = collide(S_0) first.  Runs that
     // time every launch keep the two-pass start, so that their launches are
     // all of one kernel.
     const bool first_fused =
-        nsteps >= 2 && !per_launch && (m->qid == 4 || m->qid == 5 || m->qid == 9) &&
+        nsteps >= 2 && !per_launch && !multi && (m->qid == 4 || m->qid == 5 || m->qid == 9) &&
         S->nx % 64 == 0 && S->ny % 8 == 0 &&
         (m->coll <= LBM_TRT || (S->storage == LBM_STORE_F64 && m->coll == LBM_MRT));
-    if (first_fused) {
+    int64_t k_first = 1;  // collisions done by the first pass
+    if (multi && multi_next(plan, nsteps) > 1) {
+        k_first = multi_next(plan, nsteps);
+        if (int rc = run_multi(plan, m, S, C, (int)k_first, true)) return rc;
+    } else if (first_fused) {
         if (int rc = run(lbm::Op::FusedFirst, m, S, C, true)) return rc;
+        k_first = 2;
     } else {
         if (int rc = run(lbm::Op::Collide, m, S, C, false)) return rc;
     }
-    const int64_t k_first = first_fused ? 2 : 1;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ms) {
         HIP_TRY(hipEventCreate(&e0));
@@ -1037,11 +1159,16 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
         ev.assign((size_t)(nsteps > 1 ? nsteps : 1), nullptr);
         for (auto &e : ev) HIP_TRY(hipEventCreate(&e));
     }
-    // the remaining steps: C_k = collide(BC(stream(C_{k-1}))) in one pull pass each
+    // the remaining steps: C_k = collide(BC(stream(C_{k-1}))), one or several
+    // per pass
     lbm_field cur = C, other = S;
-    for (int64_t k = k_first; k < nsteps; ++k) {
+    for (int64_t k = k_first; k < nsteps;) {
         if (per_launch) HIP_TRY(hipEventRecord(ev[(size_t)k - 1], g_stream));
-        if (int rc = run(lbm::Op::Fused, m, cur, other, true)) return rc;
+        const int t = multi ? multi_next(plan, nsteps - k) : 1;
+        if (int rc = t > 1 ? run_multi(plan, m, cur, other, t, false)
+                           : run(lbm::Op::Fused, m, cur, other, true))
+            return rc;
+        k += t;
         std::swap(cur, other);
     }
     if (per_launch) {
@@ -1161,6 +1288,31 @@ int lbm_autotune(lbm_model m, lbm_field f_stream, int trial_steps, int *block_x,
                     bv = vec;
                     bn = nt;
                 }
+            }
+        }
+    }
+    // the several-step kernels (automatic shape): kept by returning that shape
+    if (!rc) {
+        m->launch_block = m->launch_rows = m->launch_vec = 0;
+        m->launch_nt = -1;
+        const MultiPlan plan = multi_plan(m, A);
+        if (plan.kernel != lbm::kMultiNone) {
+            rc = run_multi(plan, m, A, B, plan.max_steps, false);  // warm-up
+            (void)hipEventRecord(e0, g_stream);
+            lbm_field cur = B, other = A;
+            int done = 0;
+            for (; done < trial_steps && !rc; done += plan.max_steps) {
+                rc = run_multi(plan, m, cur, other, plan.max_steps, false);
+                std::swap(cur, other);
+            }
+            (void)hipEventRecord(e1, g_stream);
+            if (hipEventSynchronize(e1) != hipSuccess) rc = fail(-3, "autotune sync failed");
+            float ms = 0.0f;
+            (void)hipEventElapsedTime(&ms, e0, e1);
+            const double us = 1e3 * (double)ms / done;
+            if (!rc && us < best) {
+                best = us;
+                auto_launch(m, A, bb, br, bv, bn);
             }
         }
     }

@@ -33,4 +33,23 @@ int dispatch_lp(const Launch &L, const StepParams<double> &pd, hipStream_t s) {
     }
 }
 
+#define LBM_SWITCH_MULTI(TAG, L, p, s)                      \
+    switch ((L).qid) {                                      \
+    case 4: return run_multi_##TAG##_q4(L, p, s);           \
+    case 5: return run_multi_##TAG##_q5(L, p, s);           \
+    case 9: return run_multi_##TAG##_q9(L, p, s);           \
+    default: return -1;                                     \
+    }
+
+int dispatch_multi(int storage, const MultiLaunch &L, const StepParams<double> &pd, hipStream_t s) {
+    if (storage == 0) LBM_SWITCH_MULTI(f64, L, pd, s)
+    const StepParams<float> p = to_float_params(pd);
+    switch (storage) {
+    case 1: LBM_SWITCH_MULTI(f32, L, p, s)
+    case 4: LBM_SWITCH_MULTI(f16neq, L, p, s)
+    case 5: LBM_SWITCH_MULTI(bf16neq, L, p, s)
+    default: return -1;
+    }
+}
+
 }  // namespace lbm

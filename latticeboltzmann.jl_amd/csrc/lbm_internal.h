@@ -126,6 +126,28 @@ struct Launch {
     int nt = 0;   // fused step: non-temporal stores
 };
 
+// Several fused steps in one pass (lbm_multi.h): one-speed stencils, storages
+// F64, F32 and the non-equilibrium ones.
+enum MultiKernel : int {
+    kMultiTile = 0,   // LDS tile of 8 x 8 nodes, up to 8 steps
+    kMultiBlock16,    // register block of 64 x 16 nodes
+    kMultiBlock32,    // 64 x 32, 16 waves
+    kMultiBlockWide,  // 64 x 24 (FP64) or 64 x 32 (FP32), 8 waves
+    kMultiMarch,      // marching waves: 2-5 steps (FP64), 2-4 or 6 (FP32), 2-4 (16-bit)
+    kMultiNone
+};
+constexpr int kMarchRows = 16;  // fewest rows of a marching wave
+struct MultiLaunch {
+    int kernel;
+    int qid, coll;  // as in Launch
+    int steps;      // collisions of the pass
+    int first;      // the first of them collides the canonical state in place
+    int walls;      // directions in the boundary list (bit = direction)
+    int moving;     // index of its last moving wall
+    const void *src;
+    void *dst;
+};
+
 // Reverse-mode kernels of the periodic SRT/TRT step (lbm_adjoint.h).
 struct AdjLaunch {
     int what;            // 0 S0 = feq(rho0, u0), 1 seed lambda_T + loss, 2 reverse step, 3 dL/du0
@@ -164,6 +186,16 @@ int run_batch_f64_q9(int op, const BatchLattice *lats, const BatchTile *tiles, i
 int run_batch_f32_q9(int op, const BatchLattice *lats, const BatchTile *tiles, int ntiles,
                      void *pool, int parity, int block, int grid, int vec,
                      const StepParams<float> &p, hipStream_t s);
+
+#define LBM_DECLARE_MULTI(TAG, T)                                                                   \
+    int run_multi_##TAG##_q4(const MultiLaunch &L, const StepParams<T> &p, hipStream_t s);           \
+    int run_multi_##TAG##_q5(const MultiLaunch &L, const StepParams<T> &p, hipStream_t s);           \
+    int run_multi_##TAG##_q9(const MultiLaunch &L, const StepParams<T> &p, hipStream_t s);
+LBM_DECLARE_MULTI(f64, double)
+LBM_DECLARE_MULTI(f32, float)
+LBM_DECLARE_MULTI(f16neq, float)
+LBM_DECLARE_MULTI(bf16neq, float)
+int dispatch_multi(int storage, const MultiLaunch &L, const StepParams<double> &p, hipStream_t s);
 
 LBM_DECLARE_ALL_Q(f64, double)
 LBM_DECLARE_ALL_Q(f32, float)

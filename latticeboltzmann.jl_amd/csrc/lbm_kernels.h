@@ -774,12 +774,11 @@ __device__ __forceinline__ void mrt_each(F &&fn, std::integer_sequence<int, Is..
     (fn(std::integral_constant<int, Is>{}), ...);
 }
 
+// the collision of a node whose moments are known
 template <int QID, class T>
-__device__ __forceinline__ void collide_mrt_node(T (&f)[QT<QID>::Q], const StepParams<T> &p,
-                                                 int x, int y) {
+__device__ __forceinline__ void collide_mrt_moments(T (&f)[QT<QID>::Q], const StepParams<T> &p,
+                                                    int x, int y, T rho, T ux, T uy) {
     constexpr int N = QT<QID>::ORDER / 2;
-    T rho, ux, uy;
-    node_moments<QID, T>(f, rho, ux, uy);
     if (p.force_kind != 0) {
         T Fx, Fy;
         node_force(p, x, y, Fx, Fy);
@@ -825,6 +824,13 @@ __device__ __forceinline__ void collide_mrt_node(T (&f)[QT<QID>::Q], const StepP
     mrt_each(out, std::make_integer_sequence<int, QT<QID>::Q>{});
 }
 
+template <int QID, class T>
+__device__ __forceinline__ void collide_mrt_node(T (&f)[QT<QID>::Q], const StepParams<T> &p,
+                                                 int x, int y) {
+    T rho, ux, uy;
+    node_moments<QID, T>(f, rho, ux, uy);
+    collide_mrt_moments<QID, T>(f, p, x, y, rho, ux, uy);
+}
 
 // ---------------------------------------------------------------------------
 // boundary conditions of the ordered list for node (x, y), applied to the

@@ -1,0 +1,986 @@
+// lbm_multi.h -- several fused time steps per launch (temporal blocking).
+//
+// One fused step moves every population through HBM once; a run of n steps is
+// bound by 2 Q sizeof(population) n bytes per node.  The kernels here advance
+// a region by T steps per pass instead, recomputing a halo that shrinks by
+// the stencil's reach per step, so T steps cost one pass:
+//   * k_march: a wave marches up a strip of columns with the rows of the T
+//     levels in registers and in its own LDS;
+//   * k_tile: a block keeps a tile of the lattice in LDS.
+// Every node is updated by the operations of the single-step kernels in their
+// order, wrapped to its lattice position, boundary list included: FP64 results
+// are bit-identical to running the steps one by one.
+#pragma once
+
+#include "lbm_kernels.h"
+
+namespace lbm {
+
+// Constants of the pair-form collision: halves of s^2, -s and of the TRT rates
+// (scaling by a power of two is exact, so folding the 1/2 of the reference's
+// expressions into them changes no rounding), and -2 w per population for the
+// FP32 form.
+template <class T>
+struct MultiConsts {
+    T hs2, hns, homs, homa;
+    T w2[37];
+};
+
+template <class T>
+inline MultiConsts<T> multi_consts(const StepParams<T> &p) {
+    MultiConsts<T> m;
+    m.hs2 = T(0.5) * p.s2;
+    m.hns = T(0.5) * p.neg_s;
+    m.homs = T(0.5) * p.oms;
+    m.homa = T(0.5) * p.oma;
+    for (int i = 0; i < 37; ++i) m.w2[i] = T(-2) * p.w[i];
+    return m;
+}
+
+// first population with the same weight (the same |c| components)
+template <int QID>
+LBM_HD constexpr int weight_rep(int i) {
+    const auto ab = [](int v) { return v < 0 ? -v : v; };
+    const int a = ab(QT<QID>::cx(i)), b = ab(QT<QID>::cy(i));
+    for (int j = 0; j < i; ++j) {
+        const int c = ab(QT<QID>::cx(j)), d = ab(QT<QID>::cy(j));
+        if ((a == c && b == d) || (a == d && b == c)) return j;
+    }
+    return i;
+}
+
+// mx / r and my / r, correctly rounded: one refined reciprocal for both
+// quotients, each finished with the exact remainder of its product (the
+// division expansion's own steps, with the reciprocal shared).  Outside
+// 2^-510 < r < 2^510 the plain divisions run.  A numerator small enough for
+// its remainder to underflow (|m| < 2^-960) gives a velocity whose products
+// vanish against 1 in the equilibrium, so its last bit never reaches a
+// population.
+__device__ __forceinline__ void div2(double mx, double my, double r, double &ux, double &uy) {
+    double y = __builtin_amdgcn_rcp(r);
+    y = __builtin_fma(y, __builtin_fma(-r, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-r, y, 1.0), y);
+    const double qx = mx * y, qy = my * y;
+    ux = __builtin_fma(__builtin_fma(-r, qx, mx), y, qx);
+    uy = __builtin_fma(__builtin_fma(-r, qy, my), y, qy);
+    const unsigned hi = static_cast<unsigned>(__double2hiint(r));
+    if (__builtin_expect(hi - 0x20100000u >= 0x3fc00000u, 0)) {
+        ux = mx / r;
+        uy = my / r;
+    }
+}
+
+// node_moments with the shared reciprocal
+template <int QID, int... Is>
+__device__ __forceinline__ void moments_div2(const double (&f)[QT<QID>::Q], double &rho, double &ux,
+                                             double &uy, std::integer_sequence<int, Is...>) {
+    double mx = 0.0, my = 0.0;
+    rho = f[0] + f[1];
+    ((rho = (Is >= 2 ? rho + f[Is] : rho)), ...);
+    ((mx = (QT<QID>::cx(Is) != 0 ? mx + cmul<QT<QID>::cx(Is)>(f[Is]) : mx)), ...);
+    ((my = (QT<QID>::cy(Is) != 0 ? my + cmul<QT<QID>::cy(Is)>(f[Is]) : my)), ...);
+    div2(mx, my, rho, ux, uy);
+}
+
+// collide! of one node for the first- and second-order equilibria, one
+// opposite pair (i, j) at a time: c_j = -c_i, so u.c, its square, the
+// second-order term and (TRT) the symmetric and antisymmetric parts of the
+// pair are formed once.  Rounding for rounding the values are those of
+// collide_seq (negation and scaling by 1/2 are exact); D2Q9 TRT FP64 takes
+// 137 arithmetic instructions instead of 224.
+template <int QID, int COLL, int... Is>
+__device__ __forceinline__ void collide_pairs(double (&f)[QT<QID>::Q], const StepParams<double> &p,
+                                              const MultiConsts<double> &mc, int x, int y,
+                                              std::integer_sequence<int, Is...>) {
+    constexpr int FEQ = QT<QID>::FEQ;
+    static_assert(FEQ <= 2 && COLL <= 1, "pair form: orders one and two, SRT and TRT");
+    double rho, ux, uy;
+    moments_div2<QID>(f, rho, ux, uy, LBM_SEQ);
+    if (p.force_kind != 0) {
+        double Fx, Fy;
+        node_force(p, x, y, Fx, Fy);
+        ux = ux + p.tau_force * Fx;  // srt.jl:54 / trt.jl:79
+        uy = uy + p.tau_force * Fy;
+    }
+    const double usq = ux * ux + uy * uy;
+    const double hq = mc.hns * usq;
+    double rw[QT<QID>::Q];
+    auto one = [&](auto Ic) {
+        constexpr int i = decltype(Ic)::value;
+        constexpr int j = QT<QID>::opp(i), wr = weight_rep<QID>(i);
+        if constexpr (wr == i) rw[i] = rho * p.w[i];
+        if constexpr (i <= j) {
+            const double ud = udot<QID, i>(ux, uy);
+            double qi, qj;
+            if constexpr (i == j) {
+                qi = FEQ == 2 ? rw[wr] * (1.0 + hq) : rw[wr];
+                qj = qi;
+            } else {
+                const double a1 = p.s * ud;
+                double ai = 1.0 + a1, aj = 1.0 - a1;
+                if constexpr (FEQ == 2) {
+                    const double h2 = mc.hs2 * (ud * ud) + hq;
+                    ai = ai + h2;
+                    aj = aj + h2;
+                }
+                qi = rw[wr] * ai;
+                qj = rw[wr] * aj;
+            }
+            if constexpr (COLL == 0) {
+                f[i] = p.omo * f[i] + p.om * qi;  // srt.jl:57-59
+                if constexpr (j != i) f[j] = p.omo * f[j] + p.om * qj;
+            } else if constexpr (i == j) {
+                f[i] = f[i] + (-p.oms) * (f[i] - qi);
+            } else {  // trt.jl:82-94
+                const double gi = f[i], gj = f[j];
+                const double A = (-mc.homs) * ((gi + gj) - (qi + qj));
+                const double B = mc.homa * ((gi - gj) - (qi - qj));
+                f[i] = gi + (A - B);
+                f[j] = gj + (A + B);
+            }
+        }
+    };
+    (one(std::integral_constant<int, Is>{}), ...);
+}
+
+// The same for the FP32 storages, on shifted populations g = f - w rho0.  The
+// moments are summed from the pairs' sums and differences, which the TRT
+// relaxation uses again; with the even and odd parts of the pair's
+// equilibrium (ev, od as in collide_neq_pairs), ns = (g_i + g_j) - 2 w ev and
+// na = (g_i - g_j) - 2 w od are the relaxed parts: g_i - ns / (2 tau_s) -
+// na / (2 tau_a).  D2Q9 TRT: 66 instructions per node instead of 92.
+template <int QID, int COLL, int... Is>
+__device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const StepParams<float> &p,
+                                              const MultiConsts<float> &mc, int x, int y,
+                                              std::integer_sequence<int, Is...>) {
+    constexpr int FEQ = QT<QID>::FEQ, Q = QT<QID>::Q;
+    static_assert(FEQ <= 2 && COLL <= 1, "pair form: orders one and two, SRT and TRT");
+    float s[Q], d[Q];  // pair sums and differences, at the smaller index
+    auto sums = [&](auto Ic) {
+        constexpr int i = decltype(Ic)::value, j = QT<QID>::opp(i);
+        if constexpr (i < j) {
+            s[i] = f[i] + f[j];
+            d[i] = f[i] - f[j];
+        } else if constexpr (i == j) {
+            s[i] = f[i];
+        }
+    };
+    (sums(std::integral_constant<int, Is>{}), ...);
+    float drho = 0.0f, mx = 0.0f, my = 0.0f;
+    auto mom = [&](auto Ic) {
+        constexpr int i = decltype(Ic)::value, j = QT<QID>::opp(i);
+        constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i);
+        if constexpr (i <= j) drho = drho + s[i];
+        if constexpr (i < j && cx != 0) mx = mx + cmul<cx>(d[i]);
+        if constexpr (i < j && cy != 0) my = my + cmul<cy>(d[i]);
+    };
+    (mom(std::integral_constant<int, Is>{}), ...);
+    const float rho = p.rho0 + drho, ir = rcp_fast(rho);
+    float ux = mx * ir, uy = my * ir;
+    if (p.force_kind != 0) {
+        float Fx, Fy;
+        node_force(p, x, y, Fx, Fy);
+        ux = ux + p.tau_force * Fx;
+        uy = uy + p.tau_force * Fy;
+    }
+    // the record form of the equilibrium (make_rec)
+    const float sr = p.s * rho, ax = sr * ux, ay = sr * uy;
+    const float a0 = FEQ == 2 ? drho - 0.5f * (ax * ux + ay * uy) : drho;
+    const float a3 = 0.5f * ir;
+    auto one = [&](auto Ic) {
+        constexpr int i = decltype(Ic)::value;
+        constexpr int j = QT<QID>::opp(i), wr = weight_rep<QID>(i);
+        if constexpr (i == j) {
+            const float n = f[i] - p.w[wr] * a0;
+            f[i] = f[i] - (COLL == 0 ? p.om : p.oms) * n;
+        } else if constexpr (i < j) {
+            const float od = udot<QID, i>(ax, ay);
+            const float ev = FEQ == 2 ? a0 + a3 * (od * od) : a0;
+            if constexpr (COLL == 0) {
+                const float w = p.w[wr];
+                f[i] = f[i] - p.om * (f[i] - w * (ev + od));
+                f[j] = f[j] - p.om * (f[j] - w * (ev - od));
+            } else {
+                const float ns = s[i] + mc.w2[wr] * ev, na = d[i] + mc.w2[wr] * od;
+                f[i] = (f[i] - mc.homs * ns) - mc.homa * na;
+                f[j] = (f[j] - mc.homs * ns) + mc.homa * na;
+            }
+        }
+    };
+    (one(std::integral_constant<int, Is>{}), ...);
+}
+
+template <int QID, int COLL, class T>
+__device__ __forceinline__ void collide_multi(T (&f)[QT<QID>::Q], const StepParams<T> &p,
+                                              const MultiConsts<T> &mc, int x, int y) {
+    static_assert(COLL <= 2 && QT<QID>::FEQ <= 2, "one-speed stencils, SRT, TRT and MRT");
+    if constexpr (COLL <= 1) {
+        collide_pairs<QID, COLL>(f, p, mc, x, y, LBM_SEQ);
+    } else {
+        double rho, ux, uy;
+        moments_div2<QID>(f, rho, ux, uy, LBM_SEQ);
+        collide_mrt_moments<QID, T>(f, p, x, y, rho, ux, uy);
+    }
+}
+
+// The boundary list of a node (apply_bc_seq's semantics) as a mask, formed once
+// per node and pass: bit i is set when population i is replaced by the node's
+// own post-collision opp(i), bit 16 + i when the last condition that replaces
+// it is a moving wall (its term is added).  One-speed stencils: a wall
+// replaces the populations whose component points away from it, at the row or
+// column next to it.  Walking the list costs tens of dependent scalar loads
+// and branches, applying the mask about 30 vector instructions: with the list
+// walked at every level a 257^2 cavity ran 4.3 us per step instead of 3.3.
+template <int QID>
+LBM_HD constexpr unsigned wall_mask(int dir) {
+    unsigned m = 0;
+    for (int i = 0; i < QT<QID>::Q; ++i) {
+        const int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i);
+        if (dir == 0 ? cy < 0 : (dir == 2 ? cy > 0 : (dir == 1 ? cx < 0 : cx > 0))) m |= 1u << i;
+    }
+    return m;
+}
+
+// the walls of the list (bit = direction) and its last moving wall
+struct WallArgs {
+    int walls, moving;
+};
+
+// whether node (x, y) lies at a wall of the list
+template <class T>
+__device__ __forceinline__ bool at_wall(const StepParams<T> &p, int walls, int x, int y) {
+    return ((walls & 1) && y == p.ny - 1) || ((walls & 2) && x == p.nx - 1) ||
+           ((walls & 4) && y == 0) || ((walls & 8) && x == 0);
+}
+
+template <int QID, class T>
+__device__ __forceinline__ unsigned bc_mask(const StepParams<T> &p, int walls, int x, int y) {
+    static_assert(QT<QID>::MAXC == 1 && QT<QID>::Q <= 16, "one-speed stencils");
+    unsigned m = 0;
+    if (at_wall(p, walls, x, y)) {
+        for (int b = 0; b < p.nbc; ++b) {
+            const BCDev bc = p.bcs[b];
+            const bool at = bc.dir == 0   ? y == p.ny - 1
+                            : bc.dir == 1 ? x == p.nx - 1
+                            : bc.dir == 2 ? y == 0
+                                          : x == 0;
+            const unsigned w = bc.dir == 0   ? wall_mask<QID>(0)
+                               : bc.dir == 1 ? wall_mask<QID>(1)
+                               : bc.dir == 2 ? wall_mask<QID>(2)
+                                             : wall_mask<QID>(3);
+            const bool inr = bc.kind == 1 || (x >= bc.x0 && x <= bc.x1 && y >= bc.y0 && y <= bc.y1);
+            if (at && inr) m = (m & ~(w << 16)) | w | (bc.kind == 1 ? w << 16 : 0u);
+        }
+    }
+    return m;
+}
+
+template <int QID, class T, class F>
+__device__ __forceinline__ void bc_apply(const StepParams<T> &p, int moving, unsigned m,
+                                         T (&f)[QT<QID>::Q], F &&own) {
+    if (m == 0) return;
+    auto one = [&](auto Ic) {
+        constexpr int i = decltype(Ic)::value;
+        constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i), j = QT<QID>::opp(i);
+        if constexpr (cx != 0 || cy != 0) {
+            T v = own(std::integral_constant<int, j>{});
+            if constexpr (cy < 0) {
+                if (m & (1u << (16 + i))) v = v + static_cast<T>(p.mw[moving * QT<QID>::Q + i]);
+            }
+            f[i] = (m & (1u << i)) ? v : f[i];
+        }
+    };
+    adj_each_node<QID>(one);
+}
+
+// ---------------------------------------------------------------------------
+// k_tile
+// ---------------------------------------------------------------------------
+// A block advances a TX x TY tile by `levels` <= TMAX steps.  Level l pulls
+// from level l - 1 and collides on the tile and a halo of M (levels - l)
+// nodes (M = the stencil's reach); level 0 is the lattice in HBM, the levels
+// between share one LDS buffer of the first level's region, where every node
+// keeps its place: a thread pulls its nodes into registers, the block meets,
+// and the results overwrite the buffer.  `first`: the run's first step, level
+// 1 collides the canonical state S_0 of its own node instead of pulling.
+struct TileArgs {
+    int levels;
+    int tiles_x;
+    int first;
+    WallArgs wall;
+};
+
+template <int QID, class ST, int TX, int TY, int TMAX, int NT>
+struct TileShape {
+    static constexpr int H = QT<QID>::MAXC * (TMAX - 1);
+    static constexpr int W = TX + 2 * H, N = W * (TY + 2 * H);
+    static constexpr int K = (N + NT - 1) / NT;  // nodes per thread
+};
+
+template <int QID, int COLL, class ST, int TX, int TY, int TMAX, int NT, bool BC>
+__global__ void __launch_bounds__(NT)
+k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
+       const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc, const TileArgs a) {
+    using T = typename ST::T;
+    using S = typename ST::store_t;
+    using SH = TileShape<QID, ST, TX, TY, TMAX, NT>;
+    constexpr int Q = QT<QID>::Q, M = QT<QID>::MAXC, W = SH::W, N = SH::N, K = SH::K;
+    static_assert(M == 1 && !ST::kNeq, "one-speed stencils, one value per population");
+    __shared__ T buf[Q * N];
+    const int ty = blockIdx.x / a.tiles_x, tx = blockIdx.x - ty * a.tiles_x;
+    int at[K], xs[K], ys[K], ring[K];
+    unsigned bcm[K];
+    bool mine[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int n = (int)threadIdx.x + k * NT;
+        const int hy = n / W, hx = n - hy * W;
+        at[k] = n;
+        const int ux = tx * TX - SH::H + hx, uy = ty * TY - SH::H + hy;
+        xs[k] = wrap(ux, p.nx);
+        ys[k] = wrap(uy, p.ny);
+        bcm[k] = BC ? bc_mask<QID>(p, a.wall.walls, xs[k], ys[k]) : 0u;
+        // distance outside the tile (0 inside): level l needs ring <= levels - l
+        const int dx = max(SH::H - hx, hx - (SH::H + TX - 1)), dy = max(SH::H - hy, hy - (SH::H + TY - 1));
+        ring[k] = n < N ? max(0, max(dx, dy)) : TMAX;
+        mine[k] = ring[k] == 0 && ux < p.nx && uy < p.ny;
+    }
+    const int L = a.levels;
+    T f[K][Q];
+    // level 1 from HBM
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (ring[k] > L - 1) continue;
+        const int x = xs[k], y = ys[k];
+        int xm = x, xp = x, ym = y, yp = y;
+        if (!a.first) {
+            xm = x == 0 ? p.nx - 1 : x - 1;
+            xp = x == p.nx - 1 ? 0 : x + 1;
+            ym = y == 0 ? p.ny - 1 : y - 1;
+            yp = y == p.ny - 1 ? 0 : y + 1;
+        }
+        auto ld = [&](auto Ic) {
+            constexpr int i = decltype(Ic)::value;
+            constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i);
+            const int sx = cx == 0 ? x : (cx > 0 ? xm : xp), sy = cy == 0 ? y : (cy > 0 ? ym : yp);
+            f[k][i] = ST::decode(C[p.plane * i + ((long long)sx + (long long)p.nx * sy)], i, p);
+        };
+        adj_each_node<QID>(ld);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (ring[k] > L - 1) continue;
+        if constexpr (BC) {
+            if (!a.first)
+                bc_apply<QID, T>(p, a.wall.moving, bcm[k], f[k], [&](auto Jc) {
+                    return ld_pop<QID, decltype(Jc)::value, ST>(
+                        C, p, (long long)xs[k] + (long long)p.nx * ys[k]);
+                });
+        }
+        collide_multi<QID, COLL, T>(f[k], p, mc, xs[k], ys[k]);
+    }
+    for (int l = 2; l <= L; ++l) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (ring[k] > L - l + 1) continue;
+            auto put = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                buf[N * i + at[k]] = f[k][i];
+            };
+            adj_each_node<QID>(put);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (ring[k] > L - l) continue;
+            auto pull = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                f[k][i] = buf[N * i + at[k] - QT<QID>::cx(i) - W * QT<QID>::cy(i)];
+            };
+            adj_each_node<QID>(pull);
+            if constexpr (BC) {
+                bc_apply<QID, T>(p, a.wall.moving, bcm[k], f[k],
+                                 [&](auto Jc) { return buf[N * decltype(Jc)::value + at[k]]; });
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (ring[k] > L - l) continue;
+            collide_multi<QID, COLL, T>(f[k], p, mc, xs[k], ys[k]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (!mine[k]) continue;
+        auto st = [&](auto Ic) {
+            constexpr int i = decltype(Ic)::value;
+            Cn[p.plane * i + ((long long)xs[k] + (long long)p.nx * ys[k])] = ST::encode(f[k][i], i, p);
+        };
+        adj_each_node<QID>(st);
+    }
+}
+
+// x-shift inside a wave: the value of the lane below (D = +1) or above (-1)
+template <int D>
+__device__ __forceinline__ int lane_shift(int v) {
+    // DPP wave_shr:1 / wave_shl:1
+    return __builtin_amdgcn_update_dpp(0, v, D > 0 ? 0x138 : 0x130, 0xf, 0xf, true);
+}
+template <int D>
+__device__ __forceinline__ float lane_shift(float v) {
+    return __int_as_float(lane_shift<D>(__float_as_int(v)));
+}
+template <int D>
+__device__ __forceinline__ double lane_shift(double v) {
+    return __hiloint2double(lane_shift<D>(__double2hiint(v)), lane_shift<D>(__double2loint(v)));
+}
+
+// ---------------------------------------------------------------------------
+// k_block
+// ---------------------------------------------------------------------------
+// A block of NW waves advances a region of 64 columns and NW R rows held in
+// registers: wave w keeps R consecutive rows, one column per lane.  A pull
+// along x comes from the neighbour lane, along y from the wave's own rows, and
+// at a wave's first and last row from the neighbouring wave through LDS (two
+// buffers, one barrier per level).  Every level computes the whole region; its
+// outermost ring of valid nodes is lost each time, so T levels write the inner
+// 64 - 2 (T - 1) columns and NW R - 2 (T - 1) rows.
+struct BlockArgs {
+    int levels;
+    int tiles_x, outx, outy;  // nodes written per block
+    int first;
+    WallArgs wall;
+};
+
+template <int QID, int COLL, class ST, int NW, int R, bool BC>
+__global__ void __launch_bounds__(64 * NW)
+k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
+        const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc,
+        const BlockArgs a) {
+    using V = typename ST::T;
+    using S = typename ST::store_t;
+    constexpr int Q = QT<QID>::Q;
+    static_assert(QT<QID>::MAXC == 1 && !ST::kNeq, "one-speed stencils, one value per population");
+    // the c_y != 0 populations of a wave's boundary rows: [buffer][wave][population][column]
+    constexpr auto edge_slot = [](int i) {
+        int n = 0;
+        for (int j = 0; j < i; ++j) n += QT<QID>::cy(j) != 0 ? 1 : 0;
+        return n;
+    };
+    constexpr int ES = edge_slot(Q);
+    __shared__ V xch[2][NW][ES][66];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int ty = blockIdx.x / a.tiles_x, tx = blockIdx.x - ty * a.tiles_x;
+    const int L = a.levels, h = L - 1;
+    const int cx0 = tx * a.outx, cy0 = ty * a.outy;  // first node written
+    const int ux = cx0 - h + lane;
+    const int x = wrap(ux, p.nx);
+    const int xm = a.first ? x : (x == 0 ? p.nx - 1 : x - 1);
+    const int xp = a.first ? x : (x == p.nx - 1 ? 0 : x + 1);
+    const unsigned off = (unsigned)x * (unsigned)sizeof(S);
+    const unsigned offm = (unsigned)xm * (unsigned)sizeof(S), offp = (unsigned)xp * (unsigned)sizeof(S);
+    const int row0 = w * R;  // the wave's first row in the region
+    int ys[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+        ys[j] = __builtin_amdgcn_readfirstlane(wrap(cy0 - h + row0 + j, p.ny));
+    unsigned bcm[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) bcm[j] = BC ? bc_mask<QID>(p, a.wall.walls, x, ys[j]) : 0u;
+    V g[R][Q];
+    // level 1
+    S pre[R][Q];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int y = ys[j];
+        const int ym = a.first ? y : (y == 0 ? p.ny - 1 : y - 1);
+        const int yp = a.first ? y : (y + 1 == p.ny ? 0 : y + 1);
+        auto one = [&](auto Ic) {
+            constexpr int i = decltype(Ic)::value;
+            constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i);
+            const S *base = C + p.plane * i + (long long)p.nx * (cy == 0 ? y : (cy > 0 ? ym : yp));
+            pre[j][i] = ld_g(at_b(base, cx == 0 ? off : (cx > 0 ? offm : offp)));
+        };
+        adj_each_node<QID>(one);
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int y = ys[j];
+        auto dec = [&](auto Ic) {
+            constexpr int i = decltype(Ic)::value;
+            g[j][i] = ST::decode(pre[j][i], i, p);
+        };
+        adj_each_node<QID>(dec);
+        if constexpr (BC) {
+            if (!a.first)
+                bc_apply<QID, V>(p, a.wall.moving, bcm[j], g[j], [&](auto Jc) {
+                    return ld_pop<QID, decltype(Jc)::value, ST>(C, p, (long long)x + (long long)p.nx * y);
+                });
+        }
+        collide_multi<QID, COLL, V>(g[j], p, mc, x, y);
+    }
+    for (int l = 2; l <= L; ++l) {
+        V(*X)[ES][66] = xch[l & 1];
+        auto put = [&](auto Ic) {
+            constexpr int i = decltype(Ic)::value, cy = QT<QID>::cy(i);
+            if constexpr (cy > 0) X[w][edge_slot(i)][lane + 1] = g[R - 1][i];
+            if constexpr (cy < 0) X[w][edge_slot(i)][lane + 1] = g[0][i];
+        };
+        adj_each_node<QID>(put);
+        __syncthreads();
+        V carry[Q];  // c_y > 0 populations of the row below, already shifted along x
+        auto below = [&](auto Ic) {
+            constexpr int i = decltype(Ic)::value, cy = QT<QID>::cy(i);
+            if constexpr (cy > 0) carry[i] = X[w > 0 ? w - 1 : 0][edge_slot(i)][lane + 1 - QT<QID>::cx(i)];
+        };
+        adj_each_node<QID>(below);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const int y = ys[j];
+            V f[Q];
+            auto pull = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i);
+                auto sh = [&](V v) -> V {
+                    if constexpr (cx > 0) return lane_shift<1>(v);
+                    else if constexpr (cx < 0) return lane_shift<-1>(v);
+                    else return v;
+                };
+                if constexpr (cy > 0) {
+                    f[i] = carry[i];
+                    carry[i] = sh(g[j][i]);
+                } else if constexpr (cy == 0) {
+                    f[i] = sh(g[j][i]);
+                } else {
+                    if (j + 1 < R) f[i] = sh(g[j + 1 < R ? j + 1 : j][i]);
+                    else f[i] = X[w + 1 < NW ? w + 1 : w][edge_slot(i)][lane + 1 - cx];
+                }
+            };
+            adj_each_node<QID>(pull);
+            if constexpr (BC) {
+                bc_apply<QID, V>(p, a.wall.moving, bcm[j], f,
+                                 [&](auto Jc) { return g[j][decltype(Jc)::value]; });
+            }
+            collide_multi<QID, COLL, V>(f, p, mc, x, y);
+            auto cp = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                g[j][i] = f[i];
+            };
+            adj_each_node<QID>(cp);
+        }
+    }
+    if (ux >= cx0 && ux < min(cx0 + a.outx, p.nx)) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const int uy = cy0 - h + row0 + j;
+            if (uy >= cy0 && uy < min(cy0 + a.outy, p.ny)) {
+                S *base = Cn + (long long)p.nx * uy;
+                auto st = [&](auto Ic) {
+                    constexpr int i = decltype(Ic)::value;
+                    *at_b(base + p.plane * i, off) = ST::encode(g[j][i], i, p);
+                };
+                adj_each_node<QID>(st);
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// k_march
+// ---------------------------------------------------------------------------
+struct MarchArgs {
+    int strips, chunks, rows;  // strips of columns, chunks of `rows` rows
+    int first;                 // the first level collides S_0 in place
+    WallArgs wall;
+};
+
+// Geometry of the marching kernel.  A wave holds 64 NC columns, NC adjacent
+// ones per lane.  SHIFTED: level 1 pulls straight from HBM (its neighbours
+// come from other addresses), so the halo is T - 1 columns; otherwise level 0
+// is loaded unshifted, decoded, and is itself a kept level.
+template <int QID, class ST, int T, int NC, bool BC>
+struct MarchShape {
+    static constexpr bool SHIFTED = NC == 1 && !ST::kNeq;
+    static constexpr int LINES = SHIFTED ? T - 1 : T;  // levels whose rows are kept
+    static constexpr int COLS = 64 * NC;
+    static constexpr int HX = (LINES + NC - 1) / NC * NC;  // halo columns, whole lanes
+    // columns written, in groups of 64 bytes: where the rows are whole lines a
+    // strip's stores then end on memory-transaction boundaries
+    static constexpr int GROUP = 64 / (int)sizeof(typename ST::store_t);
+    static constexpr int OUT = (COLS - 2 * HX) / GROUP * GROUP;
+    static_assert(OUT > 0, "halo wider than the wave");
+    // LDS rows of population i per kept level
+    LBM_HD static constexpr int slots(int i) {
+        if (QT<QID>::cx(i) == 0) return 0;
+        return QT<QID>::cy(i) > 0 ? 2 : (QT<QID>::cy(i) == 0 ? 1 : (BC ? 1 : 0));
+    }
+    LBM_HD static constexpr int slot0(int i) {
+        int n = 0;
+        for (int j = 0; j < i; ++j) n += slots(j);
+        return n;
+    }
+    static constexpr int LINE = slot0(QT<QID>::Q);  // slots per kept level
+};
+
+// The kept rows of a level, y - 1 (and y - 2 for the populations that moved
+// up), while row y arrives: populations with c_x = 0 in registers (they are
+// read by the same lane), the others in the wave's own LDS, where the reader
+// takes its neighbour's value.  No barrier: a wave's LDS operations execute in
+// order.
+template <int QID, int COLL, class ST, int T, int NC, bool BC>
+__global__ void __launch_bounds__(256)
+k_march(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
+        const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc,
+        const MarchArgs a) {
+    using V = typename ST::T;
+    using S = typename ST::store_t;
+    using SH = MarchShape<QID, ST, T, NC, BC>;
+    constexpr int Q = QT<QID>::Q, COLS = SH::COLS + 2 * NC, LINES = SH::LINES;
+    static_assert(QT<QID>::MAXC == 1, "one-speed stencils");
+    __shared__ V rows[4][LINES][SH::LINE][COLS];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wave = (int)blockIdx.x * 4 + wv;
+    if (wave >= a.strips * a.chunks) return;
+    const int chunk = wave / a.strips, strip = wave - chunk * a.strips;
+    const int y0 = chunk * a.rows, y1 = min(y0 + a.rows, p.ny);
+    const int xo = strip * SH::OUT;           // first column written
+    const int col = xo - SH::HX + lane * NC;  // the lane's first column, unwrapped
+    const bool out = col >= xo && col < min(xo + SH::OUT, p.nx);
+    int xs[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) xs[c] = wrap(col + c, p.nx);
+    const bool pulls = SH::SHIFTED && !a.first;
+    const int xm = pulls ? (xs[0] == 0 ? p.nx - 1 : xs[0] - 1) : xs[0];
+    const int xp = pulls ? (xs[0] == p.nx - 1 ? 0 : xs[0] + 1) : xs[0];
+    const unsigned off = (unsigned)xs[0] * (unsigned)sizeof(S);
+    const unsigned offm = (unsigned)xm * (unsigned)sizeof(S), offp = (unsigned)xp * (unsigned)sizeof(S);
+    // LDS element of the lane's first column and of its neighbours' (rows are
+    // padded by NC at both ends: what the end lanes read there is halo)
+    const int e0 = lane * NC + NC, em = e0 - 1, ep = e0 + 1;
+    // boundary masks of the row each level holds: they move down with the rows
+    unsigned bcm[LINES + 1][NC];
+#pragma unroll
+    for (int l = 0; l <= LINES; ++l)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) bcm[l][c] = 0u;
+    V mid[LINES][NC][Q], up[LINES][NC][Q];  // c_x = 0 only
+#pragma unroll
+    for (int l = 0; l < LINES; ++l)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int i = 0; i < Q; ++i) mid[l][c][i] = up[l][c][i] = V(0);
+    int r = __builtin_amdgcn_readfirstlane(wrap(y0 - LINES, p.ny));  // row of the first level
+    Pack<S, NC> pre[Q];
+    Pack<Rec16, NC> rec;
+    auto fetch = [&](int row) {
+        const int rm = !pulls ? row : (row == 0 ? p.ny - 1 : row - 1);
+        const int rp = !pulls ? row : (row + 1 == p.ny ? 0 : row + 1);
+        if constexpr (ST::kNeq)
+            rec = ld_g(at_b(reinterpret_cast<const Pack<Rec16, NC> *>(ST::recs(C) + (long long)p.nx * row),
+                            off * (unsigned)(sizeof(Rec16) / sizeof(S))));
+        auto one = [&](auto Ic) {
+            constexpr int i = decltype(Ic)::value;
+            constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i);
+            const int rs = cy == 0 ? row : (cy > 0 ? rm : rp);
+            const S *plane0 = C;
+            if constexpr (ST::kNeq) plane0 = ST::pops(C, p.plane);
+            const S *base = plane0 + p.plane * i + (long long)p.nx * rs;
+            const unsigned o = cx == 0 ? off : (cx > 0 ? offm : offp);
+            pre[i] = ld_g(at_b(reinterpret_cast<const Pack<S, NC> *>(base), o));
+        };
+        adj_each_node<QID>(one);
+    };
+    fetch(r);
+    const int iters = (y1 - y0) + 2 * LINES;
+#pragma unroll 1
+    for (int k = 0; k < iters; ++k) {
+        V n[NC][Q];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if constexpr (ST::kNeq) {
+                const Mom4 m = ST::unpack(rec.v[c]);
+                auto dec = [&](auto Ic) {
+                    constexpr int i = decltype(Ic)::value;
+                    n[c][i] = geq_rec<QID, i>(m, p) + ST::to_f(pre[i].v[c], p);
+                };
+                adj_each_node<QID>(dec);
+            } else {
+                auto dec = [&](auto Ic) {
+                    constexpr int i = decltype(Ic)::value;
+                    n[c][i] = ST::decode(pre[i].v[c], i, p);
+                };
+                adj_each_node<QID>(dec);
+            }
+        }
+        int rl = r;  // the row of the level in hand
+        r = __builtin_amdgcn_readfirstlane(r + 1 == p.ny ? 0 : r + 1);
+        if (k + 1 < iters) fetch(r);
+        if constexpr (BC) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+#pragma unroll
+                for (int l = LINES; l > 0; --l) bcm[l][c] = bcm[l - 1][c];
+                bcm[0][c] = bc_mask<QID>(p, a.wall.walls, xs[c], rl);
+            }
+        }
+        if (SH::SHIFTED || a.first) {
+            if constexpr (BC && SH::SHIFTED) {
+                if (!a.first)
+                    bc_apply<QID, V>(p, a.wall.moving, bcm[0][0], n[0], [&](auto Jc) {
+                        return ld_pop<QID, decltype(Jc)::value, ST>(
+                            C, p, (long long)xs[0] + (long long)p.nx * rl);
+                    });
+            }
+#pragma unroll
+            for (int c = 0; c < NC; ++c) collide_multi<QID, COLL, V>(n[c], p, mc, xs[c], rl);
+        }
+        const int par = k & 1;
+        Rec16 orec[NC];
+        float nq[NC][Q];
+        // the next level at row y - 1 from level l's rows y - 2, y - 1, y
+        auto level = [&](auto Lc) {
+            constexpr int l = decltype(Lc)::value;
+            rl = __builtin_amdgcn_readfirstlane(rl == 0 ? p.ny - 1 : rl - 1);
+            V(*L)[COLS] = rows[wv][l];
+            V f[NC][Q];
+            auto pull = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i), s0 = SH::slot0(i);
+                if constexpr (cx == 0) {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        f[c][i] = cy > 0 ? up[l][c][i] : (cy == 0 ? mid[l][c][i] : n[c][i]);
+                } else if constexpr (cy < 0) {
+                    if constexpr (cx > 0) {
+#pragma unroll
+                        for (int c = NC - 1; c > 0; --c) f[c][i] = n[c - 1][i];
+                        f[0][i] = lane_shift<1>(n[NC - 1][i]);
+                    } else {
+#pragma unroll
+                        for (int c = 0; c + 1 < NC; ++c) f[c][i] = n[c + 1][i];
+                        f[NC - 1][i] = lane_shift<-1>(n[0][i]);
+                    }
+                } else {
+                    const V *src = cy > 0 ? L[s0 + par] : L[s0];
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) f[c][i] = src[(cx > 0 ? em : ep) + c];
+                }
+            };
+            adj_each_node<QID>(pull);
+            if constexpr (BC) {
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+                    bc_apply<QID, V>(p, a.wall.moving, bcm[l + 1][c], f[c], [&](auto Jc) {
+                        constexpr int j = decltype(Jc)::value;
+                        constexpr int s0 = SH::slot0(j);
+                        if constexpr (QT<QID>::cx(j) == 0) return mid[l][c][j];
+                        else if constexpr (QT<QID>::cy(j) > 0) return L[s0 + (par ^ 1)][e0 + c];
+                        else return L[s0][e0 + c];
+                    });
+            }
+            // the rows move down; the compiler must not reorder the lane's own
+            // LDS accesses (neighbour lanes read what this lane wrote)
+            asm volatile("" ::: "memory");
+            auto keep = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i), s0 = SH::slot0(i);
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    if constexpr (cx == 0) {
+                        if constexpr (cy > 0) up[l][c][i] = mid[l][c][i];
+                        mid[l][c][i] = n[c][i];
+                    } else if constexpr (cy > 0) {
+                        L[s0 + par][e0 + c] = n[c][i];
+                    } else if constexpr (cy == 0 || BC) {
+                        L[s0][e0 + c] = n[c][i];
+                    }
+                }
+            };
+            adj_each_node<QID>(keep);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                if constexpr (ST::kNeq) {
+                    if constexpr (l == LINES - 1) {
+                        collide_neq<QID, COLL, ST>(f[c], p, xs[c], rl, orec[c], nq[c], LBM_SEQ);
+                        continue;
+                    }
+                }
+                collide_multi<QID, COLL, V>(f[c], p, mc, xs[c], rl);
+                auto cp = [&](auto Ic) {
+                    constexpr int i = decltype(Ic)::value;
+                    n[c][i] = f[c][i];
+                };
+                adj_each_node<QID>(cp);
+            }
+        };
+        mrt_each(level, std::make_integer_sequence<int, LINES>{});
+        if (k >= 2 * LINES && out) {
+            if constexpr (ST::kNeq) {
+                Pack<Rec16, NC> pr;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) pr.v[c] = orec[c];
+                Pack<Pack<Rec16, NC>, 1> pm;
+                pm.v[0] = pr;
+                put_pack<true>(at_b(reinterpret_cast<Pack<Rec16, NC> *>(ST::recs(Cn) + (long long)p.nx * rl),
+                                    off * (unsigned)(sizeof(Rec16) / sizeof(S))), pm);
+            }
+            auto st = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                S *plane0 = Cn;
+                if constexpr (ST::kNeq) plane0 = ST::pops(Cn, p.plane);
+                Pack<S, NC> pk;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    if constexpr (ST::kNeq) pk.v[c] = ST::raw(nq[c][i]);
+                    else pk.v[c] = ST::encode(n[c][i], i, p);
+                }
+                Pack<Pack<S, NC>, 1> pm;
+                pm.v[0] = pk;
+                put_pack<true>(at_b(reinterpret_cast<Pack<S, NC> *>(plane0 + p.plane * i + (long long)p.nx * rl), off), pm);
+            };
+            adj_each_node<QID>(st);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// launches
+// ---------------------------------------------------------------------------
+constexpr int kTileX = 8, kTileY = 8, kTileT = 8, kTileThreads = 512;
+
+template <int QID, int COLL, class ST, bool BC>
+int launch_tile(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
+    using S = typename ST::store_t;
+    if (L.steps < 1 || L.steps > kTileT) return -5;
+    TileArgs a;
+    a.levels = L.steps;
+    a.first = L.first;
+    a.wall = WallArgs{L.walls, L.moving};
+    a.tiles_x = (p.nx + kTileX - 1) / kTileX;
+    const int tiles_y = (p.ny + kTileY - 1) / kTileY;
+    k_tile<QID, COLL, ST, kTileX, kTileY, kTileT, kTileThreads, BC>
+        <<<(unsigned)a.tiles_x * (unsigned)tiles_y, kTileThreads, 0, s>>>(
+            static_cast<const S *>(L.src), static_cast<S *>(L.dst), p, multi_consts(p), a);
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+template <int QID, int COLL, class ST, int NW, int R, bool BC>
+int launch_block(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
+    using S = typename ST::store_t;
+    const int halo = 2 * (L.steps - 1);
+    if (L.steps < 1 || halo >= 64 || halo >= NW * R) return -5;
+    BlockArgs a;
+    a.levels = L.steps;
+    a.first = L.first;
+    a.wall = WallArgs{L.walls, L.moving};
+    // the lattice in equal shares, the width in whole 64-byte groups where
+    // that does not add a column of tiles
+    const int ox = 64 - halo, oy = NW * R - halo, group = 64 / (int)sizeof(S);
+    const int nbx = (p.nx + ox - 1) / ox, nby = (p.ny + oy - 1) / oy;
+    a.outx = (p.nx + nbx - 1) / nbx;
+    const int rounded = (a.outx + group - 1) / group * group;
+    if (rounded <= ox) a.outx = rounded;
+    a.outy = (p.ny + nby - 1) / nby;
+    a.tiles_x = (p.nx + a.outx - 1) / a.outx;
+    const int tiles_y = (p.ny + a.outy - 1) / a.outy;
+    k_block<QID, COLL, ST, NW, R, BC><<<(unsigned)a.tiles_x * (unsigned)tiles_y, 64 * NW, 0, s>>>(
+        static_cast<const S *>(L.src), static_cast<S *>(L.dst), p, multi_consts(p), a);
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+template <int QID, int COLL, class ST, int T, int NC, bool BC>
+int launch_march(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
+    using S = typename ST::store_t;
+    using SH = MarchShape<QID, ST, T, NC, BC>;
+    if (p.nx % NC != 0 || p.nx >= (1 << 27)) return -5;
+    static const int slots = [] {
+        int per_cu = 0, dev = 0, cus = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, k_march<QID, COLL, ST, T, NC, BC>, 256, 0) != hipSuccess ||
+            hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            return 0;
+        return per_cu * cus * 4;
+    }();
+    if (slots < 1) return -4;
+    MarchArgs a;
+    a.first = L.first;
+    a.wall = WallArgs{L.walls, L.moving};
+    a.strips = (p.nx + SH::OUT - 1) / SH::OUT;
+    // rows per wave: one resident round of waves, at least kMarchRows (the
+    // 2 LINES warm-up rows of a chunk are recomputed)
+    const long long per_round = ((long long)p.ny * a.strips + slots - 1) / slots;
+    a.rows = (int)(per_round > kMarchRows ? per_round : kMarchRows);
+    if (a.rows > p.ny) a.rows = p.ny;
+    a.chunks = (p.ny + a.rows - 1) / a.rows;
+    const long long waves = (long long)a.strips * a.chunks;
+    k_march<QID, COLL, ST, T, NC, BC><<<(unsigned)((waves + 3) / 4), 256, 0, s>>>(
+        static_cast<const S *>(L.src), static_cast<S *>(L.dst), p, multi_consts(p), a);
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+template <int QID, int COLL, class ST, bool BC>
+int launch_multi_c(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
+    if constexpr (ST::kNeq) {
+        if (L.kernel != kMultiMarch) return -5;
+        // level 0 is decoded in place: a first pass collides it too
+        switch (L.steps - L.first) {
+        case 1: return launch_march<QID, COLL, ST, 1, 2, BC>(L, p, s);
+        case 2: return launch_march<QID, COLL, ST, 2, 2, BC>(L, p, s);
+        case 3: return launch_march<QID, COLL, ST, 3, 2, BC>(L, p, s);
+        case 4: return launch_march<QID, COLL, ST, 4, 2, BC>(L, p, s);
+        default: return -5;
+        }
+    } else {
+        constexpr bool f64 = sizeof(typename ST::store_t) == 8;
+        switch (L.kernel) {
+        case kMultiTile: return launch_tile<QID, COLL, ST, BC>(L, p, s);
+        case kMultiBlock16: return launch_block<QID, COLL, ST, 16, 1, BC>(L, p, s);
+        case kMultiBlock32: return launch_block<QID, COLL, ST, 16, 2, BC>(L, p, s);
+        case kMultiBlockWide:
+            if constexpr (f64) return launch_block<QID, COLL, ST, 8, 3, BC>(L, p, s);
+            else return launch_block<QID, COLL, ST, 8, 4, BC>(L, p, s);
+        case kMultiMarch: break;
+        default: return -5;
+        }
+        switch (L.steps) {
+        case 2: return launch_march<QID, COLL, ST, 2, 1, BC>(L, p, s);
+        case 3: return launch_march<QID, COLL, ST, 3, 1, BC>(L, p, s);
+        case 4: return launch_march<QID, COLL, ST, 4, 1, BC>(L, p, s);
+        case 5: if constexpr (f64) return launch_march<QID, COLL, ST, 5, 1, BC>(L, p, s); break;
+        case 6: if constexpr (!f64) return launch_march<QID, COLL, ST, 6, 1, BC>(L, p, s); break;
+        default: break;
+        }
+        return -5;
+    }
+}
+
+template <int QID, class ST>
+int launch_multi(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
+    const bool bc = p.nbc > 0;
+    switch (L.coll) {
+    case 0: return bc ? launch_multi_c<QID, 0, ST, true>(L, p, s) : launch_multi_c<QID, 0, ST, false>(L, p, s);
+    case 1: return bc ? launch_multi_c<QID, 1, ST, true>(L, p, s) : launch_multi_c<QID, 1, ST, false>(L, p, s);
+    case 2:
+        if constexpr (ST::id == 0)
+            return bc ? launch_multi_c<QID, 2, ST, true>(L, p, s)
+                      : launch_multi_c<QID, 2, ST, false>(L, p, s);
+        break;
+    default: break;
+    }
+    return -2;
+}
+
+// one translation unit per (storage, quadrature)
+#define LBM_DEFINE_MULTI(TAG, ST, QID)                                                      \
+    int run_multi_##TAG##_q##QID(const MultiLaunch &L, const StepParams<typename ST::T> &p, \
+                                 hipStream_t s) {                                           \
+        return launch_multi<QID, ST>(L, p, s);                                              \
+    }
+
+}  // namespace lbm

@@ -14,8 +14,9 @@ reference's step loop (lattice_boltzmann_model.jl:60-77)::
     next!(model, last(time) + 1)
 
 Without a processing method, and with a force that does not depend on time,
-the whole loop is one ``lbm_simulate`` call: one fused pull collide-stream
-kernel per step, after which both buffers hold what the reference's hold.
+the whole loop is one ``lbm_simulate`` call: fused pull collide-stream kernels
+of one or several steps, after which both buffers hold what the reference's
+hold.
 """
 from __future__ import annotations
 
@@ -146,8 +147,8 @@ def simulate(model: LatticeBoltzmannModel, time) -> LatticeBoltzmannModel:
 
 def simulate_timed(model: LatticeBoltzmannModel, nsteps: int):
     """As ``simulate(model, range(nsteps))`` without processing; returns
-    (milliseconds spent in the fused kernels, number of fused launches),
-    measured with HIP events on the library's stream."""
+    (milliseconds spent in the fused kernels after the first pass, number of
+    steps they advance), measured with HIP events on the library's stream."""
     import ctypes
 
     m = native_model(model.quadrature).configure(model.collision_model, model.f_stream,

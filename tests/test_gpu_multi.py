@@ -1,0 +1,148 @@
+"""Runs that advance several steps per pass (lbm_multi.h) against the oracle.
+
+A run without a launch shape picks its kernel by the number of nodes: 8 x 8
+tiles, register blocks of 64 x 16, 64 x 32 and 64 x 24 (FP32 64 x 32) nodes,
+marching waves.  The shapes below sit at every kernel's edges: lattices
+narrower or lower than one tile (the halo wraps several times), the narrowest
+and lowest ones that the wide kernels take (32 columns, 12 rows) and those
+just below, widths and heights that leave remainders, step counts that need
+every pass size."""
+import numpy as np
+import pytest
+
+from lbm_cases import bc_dicts, force_for, random_populations, to_lbmhip
+
+pytestmark = pytest.mark.gpu
+
+# (nx, ny): by kernel, smallest to largest
+TILE = [(1, 1), (2, 3), (3, 40), (9, 8), (64, 64), (200, 199)]
+BLOCK16 = [(257, 160), (32, 2500), (9001, 12), (31, 2501), (9001, 11)]
+BLOCK32 = [(513, 300), (55, 2500)]
+WIDE = [(1021, 517), (57, 8001)]
+MARCH = [(2049, 1000), (33, 61001), (170001, 12), (700001, 3)]
+SHAPES = TILE + BLOCK16 + BLOCK32 + WIDE + MARCH
+
+
+def _L():
+    import lbmhip
+    return lbmhip
+
+
+def _populations(qid, nx, ny, seed, noise=2e-3):
+    """A random field of at most 61 x 53 nodes, repeated over the lattice."""
+    f = random_populations(qid, min(nx, 61), min(ny, 53), seed=seed, noise=noise)
+    reps = (-(-nx // f.shape[0]), -(-ny // f.shape[1]), 1)
+    return np.asfortranarray(np.tile(f, reps)[:nx, :ny])
+
+
+def _model(qid, coll, F):
+    L = _L()
+    q = L.Quadratures[f"D2Q{qid}"]()
+    if coll == 0:
+        return q, L.SRT(0.8, F), [0.8]
+    if coll == 1:
+        return q, L.TRT.fields(0.7, 1.3, F), [0.7, 1.3]
+    return q, L.MRT(q, [0.9, 0.75], force=F), [0.9, 0.75]
+
+
+def _oracle(oracle_lib, qid, f0, coll, taus, steps, F, bcs):
+    S, C = f0.copy(order="F"), f0.copy(order="F")
+    oracle_lib.set_threads(16)
+    try:
+        oracle_lib.simulate(qid, S, C, coll, taus, steps, force=F, bcs=bcs)
+    finally:
+        oracle_lib.set_threads(1)
+    return S, C
+
+
+def _check_f64(oracle_lib, qid, coll, nx, ny, bcname, force, steps):
+    f0 = _populations(qid, nx, ny, seed=qid + 3 * coll)
+    F = force_for(force, nx, ny)
+    q, cm, taus = _model(qid, coll, F)
+    bcs = bc_dicts(bcname, nx, ny)
+    model = _L().LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs))
+    print(f"multi D2Q{qid} coll {coll} {nx}x{ny} {bcname} {force} {steps} steps", flush=True)
+    _L().simulate(model, range(steps))
+    S, C = _oracle(oracle_lib, qid, f0, coll, taus, steps, F, bcs)
+    assert np.array_equal(model.f_stream.to_numpy(), S), (nx, ny, steps)
+    assert np.array_equal(model.f_collision.to_numpy(), C), (nx, ny, steps)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("coll,bcname,force,steps", [
+    (0, "periodic", "none", 11), (1, "cavity", "field", 13), (2, "partial", "const", 9)])
+def test_f64_bit_exact(oracle_lib, shape, coll, bcname, force, steps):
+    _check_f64(oracle_lib, 9, coll, *shape, bcname, force, steps)
+
+
+@pytest.mark.parametrize("shape", [(70, 33), (257, 160), (1021, 517)])
+@pytest.mark.parametrize("steps", range(2, 9))
+def test_f64_every_pass_size(oracle_lib, shape, steps):
+    _check_f64(oracle_lib, 9, 1, *shape, "couette", "const", steps)
+
+
+@pytest.mark.parametrize("steps", [2, 3, 4, 6, 7])
+def test_f64_march_pass_sizes(oracle_lib, steps):
+    _check_f64(oracle_lib, 9, 1, 2049, 1000, "couette", "const", steps)
+
+
+@pytest.mark.parametrize("qid", [4, 5])
+@pytest.mark.parametrize("coll", [0, 1, 2])
+@pytest.mark.parametrize("shape", [(19, 40), (257, 160), (513, 300), (700, 650), (2049, 1000)])
+def test_f64_other_one_speed_sets(oracle_lib, qid, coll, shape):
+    _check_f64(oracle_lib, qid, coll, *shape, "cavity", "const", 9)
+
+
+@pytest.mark.parametrize("coll", [0, 1])
+@pytest.mark.parametrize("shape", [(3, 40), (64, 64), (257, 160), (513, 300), (1021, 517),
+                                   (2050, 1000), (33, 61001)])
+@pytest.mark.parametrize("bcname,force", [("periodic", "none"), ("cavity", "field")])
+def test_f32_tracks_oracle(oracle_lib, coll, shape, bcname, force):
+    """FP32 on shifted populations |g| = |f - w| <= G: a step's rounding errors
+    are below 16 half-ulps of G per population (the pair sums, the
+    equilibrium's five operations, the relaxation), and the collision with
+    tau > 1/2 carries a deviation on with a factor of at most 1 in the summed
+    norm, so after n steps |error| <= 16 n 2^-24 G with room for the initial
+    rounding."""
+    nx, ny = shape
+    steps = 13
+    f0 = _populations(9, nx, ny, seed=5, noise=1e-4)
+    F = force_for(force, nx, ny)
+    q, cm, taus = _model(9, coll, F)
+    bcs = bc_dicts(bcname, nx, ny)
+    m = _L().LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs), storage="f32")
+    _L().simulate(m, range(steps))
+    S, C = _oracle(oracle_lib, 9, f0, coll, taus, steps, F, bcs)
+    w = np.asarray(q.weights)
+    G = max(np.abs(S - w).max(), np.abs(C - w).max(), np.abs(f0 - w).max())
+    tol = 16 * (steps + 1) * 2.0 ** -24 * G
+    assert np.abs(m.f_stream.to_numpy() - S).max() <= tol
+    assert np.abs(m.f_collision.to_numpy() - C).max() <= tol
+
+
+@pytest.mark.parametrize("storage", ["f16neq", "bf16neq"])
+@pytest.mark.parametrize("qid", [4, 5, 9])
+@pytest.mark.parametrize("coll", [0, 1])
+@pytest.mark.parametrize("shape", [(1022, 800), (112, 7200), (64, 12600), (66700, 12)])
+@pytest.mark.parametrize("bcname,force,steps", [("periodic", "none", 2), ("cavity", "field", 9),
+                                                ("couette", "const", 11)])
+def test_neq_error_no_larger_than_single_steps(oracle_lib, storage, qid, coll, shape, bcname,
+                                               force, steps):
+    """The 16-bit storages round once per pass instead of once per step: the
+    populations' error against the oracle's FP64 run is at most that of the
+    single-step kernels (which the per-launch timing entry point keeps), with
+    a tenth for the scatter of roundings."""
+    L = _L()
+    nx, ny = shape
+    f0 = _populations(qid, nx, ny, seed=7, noise=1e-4)
+    F = force_for(force, nx, ny)
+    q, cm, taus = _model(qid, coll, F)
+    bcs = bc_dicts(bcname, nx, ny)
+    many = L.LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs), storage=storage)
+    L.simulate(many, range(steps))
+    one = L.LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs), storage=storage)
+    L.simulate_launch_times(one, steps)
+    S, C = _oracle(oracle_lib, qid, f0, coll, taus, steps, F, bcs)
+    for a, b, ref in ((many.f_stream, one.f_stream, S), (many.f_collision, one.f_collision, C)):
+        ea, eb = (np.linalg.norm(x.to_numpy() - ref) for x in (a, b))
+        assert ea <= 1.1 * eb, (ea, eb)
