@@ -249,8 +249,13 @@ int lbm_batch_info(lbm_batch b, int *n, int64_t *nodes, int64_t *bytes);
  * f_stream, 1 = f_collision */
 int lbm_batch_upload(lbm_batch b, int k, const double *f);
 int lbm_batch_download(lbm_batch b, int k, int role, double *f);
-/* threads per tile-block (64, 128, 256; 0 = 128) and grid size (0 = one block
- * per tile; smaller grids make the blocks stride over the tile table) */
+/* launch shape of the single-step kernel: threads per tile-block (64, 128,
+ * 256; 0 = 128) and grid size (0 = one block per tile; smaller grids make the
+ * blocks stride over the tile table).  The default, and again after (0, 0)
+ * with one node per thread, is automatic: several steps per pass over blocks
+ * of 64 x 24 (FP64) or 64 x 32 (FP32) nodes, unless the lattices are much
+ * smaller than such a block.  Results are the same bits in FP64; in FP32 the
+ * passes round like lbm_simulate's. */
 int lbm_batch_set_launch(lbm_batch b, int block, int grid);
 /* nodes per thread of the batch kernel (1, 2 or 4; default 1): a tile holds
  * block x nodes consecutive nodes of one lattice, a lane nodes of them that
@@ -262,8 +267,9 @@ int lbm_batch_get_launch(lbm_batch b, int *block, int *grid, int *nodes_per_thre
 /* times launch shapes on the batch (state saved and restored), keeps the fastest */
 int lbm_batch_autotune(lbm_batch b, int trial_steps, int *block, int *grid, double *us_per_step);
 /* nsteps of every lattice; graph_chunk > 0 replays runs of graph_chunk fused
- * steps from one captured hipGraph (0: direct launches).  *ms_fused (may be
- * NULL) receives the time of the fused steps (HIP events). */
+ * steps from one captured hipGraph (0: direct launches; several steps per
+ * pass are launched directly).  *ms_fused (may be NULL) receives the time of
+ * the fused steps (HIP events; with several steps per pass, of every pass). */
 int lbm_batch_simulate(lbm_batch b, int64_t nsteps, int graph_chunk, double *ms_fused);
 
 /* ---- snapshots ----------------------------------------------------------- */

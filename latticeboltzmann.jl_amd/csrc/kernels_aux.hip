@@ -66,6 +66,29 @@ k_convert(const double *__restrict__ hostlike, void *dev, int Q, int to_device,
     }
 }
 
+// Rows row0 .. row0 + rows of one lattice of a batch: dense Float64 rows of nx
+// <-> the pool's rows of `pitch` elements (to the device: both ping-pong
+// buffers).  The host copy is then one contiguous transfer: downloading 48
+// lattices of 32^2 .. 512^2 nodes took 0.6 s with hipMemcpy2D of the rows, it
+// takes 12 ms with this pass.
+template <int SID>
+__global__ void __launch_bounds__(256)
+k_batch_xfer(double *__restrict__ dense, void *pooled, void *pooled2, int nx, int pitch, int ny,
+             int row0, int rows, int to_device, const StepParams<double> p) {
+    const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= (long long)nx * rows) return;
+    const int r = (int)(n / nx), row = row0 + r, i = row / ny;
+    const long long slot = (long long)row * pitch + (n - (long long)r * nx);
+    // load_d / store_d with a plane of 0: the flat slot, population i's weight
+    if (to_device) {
+        const double v = dense[n];
+        store_d<SID>(pooled, 0, slot, i, v, p);
+        store_d<SID>(pooled2, 0, slot, i, v, p);
+    } else {
+        dense[n] = load_d<SID>(pooled, 0, slot, i, p);
+    }
+}
+
 // density / velocity! / deviatoric_tensor per node, in the CPU restatement's order
 // (moments.jl:1-19, 81-96; hermite_polynomials.jl:47-51; hermite.jl:45-48)
 template <int QID, int SID>
@@ -542,6 +565,21 @@ int dispatch_upload(int qid, int storage, const double *src, void *dst,
     case 3: k_convert<3><<<blocks, 256, 0, s>>>(src, dst, Q, to_device, out, p); break;
     default: return -1;
     }
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+int dispatch_batch_xfer(int storage, double *dense, void *pooled, void *pooled2,
+                        const BatchLattice &L, int row0, int rows, const StepParams<double> &p,
+                        int to_device, hipStream_t s) {
+    const unsigned blocks = (unsigned)(((long long)rows * L.nx + 255) / 256);
+    if (storage == 0)
+        k_batch_xfer<0><<<blocks, 256, 0, s>>>(dense, pooled, pooled2, L.nx, L.pitch, L.ny, row0,
+                                               rows, to_device, p);
+    else if (storage == 1)
+        k_batch_xfer<1><<<blocks, 256, 0, s>>>(dense, pooled, pooled2, L.nx, L.pitch, L.ny, row0,
+                                               rows, to_device, p);
+    else
+        return -1;
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

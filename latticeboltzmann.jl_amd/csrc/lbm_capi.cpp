@@ -1711,6 +1711,14 @@ struct lbm_batch_s {
     int64_t nodes = 0;
     int parity_stream = 0;  // buffer holding f_stream
     int block = 128, grid = 0, vec = 1;  // threads per block, grid, nodes per thread
+    // several steps per pass: the regions of its blocks, used while the launch
+    // shape is automatic (region_mode: -1 undecided, 0 not worth it, 1 in use)
+    bool explicit_shape = false;
+    int region_mode = -1;
+    lbm::BatchRegion *dRegions = nullptr;
+    int nregions = 0;
+    double *dStage = nullptr;  // host transfers: dense FP64 rows
+    size_t stage_doubles = 0;
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph = nullptr;
     int g_chunk = 0, g_parity = -1, g_block = 0, g_grid = 0, g_vec = 0;
@@ -1776,6 +1784,56 @@ int batch_launch(lbm_batch b, int op, int parity) {
     else
         rc = lbm::run_batch_f32_q9(op, b->dLats, b->dTiles, b->ntiles, b->pool, parity, b->block,
                                    grid, b->vec, lbm::to_float_params(p), g_stream);
+    if (rc) return fail(-4, "batch kernel launch failed (%d)", rc);
+    return 0;
+}
+
+// The region table of the several-step kernel (64 x 24 or 64 x 32 nodes a
+// block, cut for its largest pass).  Blocks are 64 columns wide, so a batch of
+// small lattices computes mostly nodes that are not written, while the
+// single-step kernel packs a lattice's nodes densely.  us a step, several
+// steps / single steps: 512 lattices of 200 x 200 (2 computed nodes a written
+// one) 194 / 510 in FP64 and 90 / 303 in FP32, of 64 x 64 (3) 33 / 52 and
+// 14 / 29; the two would meet near 5, and the line is drawn at 4.  Up to one
+// block a CU the number of nodes computed does not matter (48 lattices of
+// 40 x 40: 3.2 / 5.8 and 2.1 / 5.0).
+// Returns < 0 on error; otherwise b->region_mode says which.
+int batch_regions(lbm_batch b) {
+    if (b->region_mode >= 0) return 0;
+    const bool f64 = b->storage == LBM_STORE_F64;
+    const int halo = 2 * ((f64 ? lbm::kBatchStepsF64 : lbm::kBatchStepsF32) - 1);
+    const int rows = f64 ? lbm::kBatchRowsF64 : lbm::kBatchRowsF32;
+    const int ox = 64 - halo, oy = rows - halo;
+    std::vector<lbm::BatchRegion> reg;
+    for (int k = 0; k < b->n; ++k) {
+        const int nx = b->nx[k], ny = b->ny[k];
+        const int bx = (nx + ox - 1) / ox, by = (ny + oy - 1) / oy;
+        const int outx = (nx + bx - 1) / bx, outy = (ny + by - 1) / by;
+        for (int y = 0; y < ny; y += outy)
+            for (int x = 0; x < nx; x += outx) reg.push_back(lbm::BatchRegion{k, x, y, outx, outy});
+    }
+    if (reg.size() > 256 && (double)reg.size() * 64.0 * rows > 4.0 * (double)b->nodes) {
+        b->region_mode = 0;
+        return 0;
+    }
+    HIP_TRY(hipMalloc(&b->dRegions, reg.size() * sizeof(lbm::BatchRegion)));
+    HIP_TRY(hipMemcpyAsync(b->dRegions, reg.data(), reg.size() * sizeof(lbm::BatchRegion),
+                           hipMemcpyHostToDevice, g_stream));
+    HIP_TRY(hipStreamSynchronize(g_stream));
+    b->nregions = (int)reg.size();
+    b->region_mode = 1;
+    return 0;
+}
+
+int batch_pass(lbm_batch b, int parity, int steps, bool first) {
+    const lbm::StepParams<double> p = batch_params(b);
+    const int coll = b->lats[0].coll;
+    const int rc = b->storage == LBM_STORE_F64
+                       ? lbm::run_batch_block_f64_q9(coll, b->dLats, b->dRegions, b->nregions,
+                                                     b->pool, parity, steps, first, p, g_stream)
+                       : lbm::run_batch_block_f32_q9(coll, b->dLats, b->dRegions, b->nregions,
+                                                     b->pool, parity, steps, first,
+                                                     lbm::to_float_params(p), g_stream);
     if (rc) return fail(-4, "batch kernel launch failed (%d)", rc);
     return 0;
 }
@@ -1894,6 +1952,8 @@ int lbm_batch_destroy(lbm_batch b) {
     free_dev(b->pool);
     free_dev(reinterpret_cast<void *&>(b->dLats));
     free_dev(reinterpret_cast<void *&>(b->dTiles));
+    free_dev(reinterpret_cast<void *&>(b->dRegions));
+    free_dev(reinterpret_cast<void *&>(b->dStage));
     delete b;
     return 0;
 }
@@ -1906,53 +1966,41 @@ int lbm_batch_info(lbm_batch b, int *n, int64_t *nodes, int64_t *bytes) {
     return 0;
 }
 
+// the host array is dense (nx, ny, Q), the pool's rows are `pitch` long: rows
+// go through a dense FP64 buffer of at most 64 MiB, kept in the handle
 static int batch_xfer(lbm_batch b, int k, int buf, double *host, bool up) {
     if (!b) return fail(-1, "null batch");
     if (k < 0 || k >= b->n) return fail(-1, "lattice index %d outside 0..%d", k, b->n - 1);
     if (!host) return fail(-1, "null host array");
     const lbm::BatchLattice &L = b->lats[k];
-    // the host array is dense (nx, ny, Q); the pool's rows are `pitch` long:
-    // ny * Q rows of nx values either way
-    const size_t nb64 = (size_t)L.plane * b->q.Q * sizeof(double);
-    const size_t hrow = (size_t)L.nx * sizeof(double), drow = (size_t)L.pitch * sizeof(double);
-    const size_t rows = (size_t)L.ny * b->q.Q;
-    const int eb = batch_elem(b);
-    char *dst = static_cast<char *>(b->pool) + (size_t)L.off[buf] * eb;
-    if (b->storage == LBM_STORE_F64) {
-        if (up)
-            HIP_TRY(hipMemcpy2DAsync(dst, drow, host, hrow, hrow, rows, hipMemcpyHostToDevice,
-                                     g_stream));
-        else
-            HIP_TRY(hipMemcpy2DAsync(host, hrow, dst, drow, hrow, rows, hipMemcpyDeviceToHost,
-                                     g_stream));
-        HIP_TRY(hipStreamSynchronize(g_stream));
-        return 0;
+    constexpr size_t kStageMax = (size_t)8 << 20;  // doubles
+    const size_t rows = (size_t)L.ny * b->q.Q, nx = (size_t)L.nx;
+    const size_t fit = kStageMax / nx > 0 ? kStageMax / nx : 1;
+    const size_t step = rows < fit ? rows : fit;
+    if (step * nx > b->stage_doubles) {
+        free_dev(reinterpret_cast<void *&>(b->dStage));
+        b->stage_doubles = 0;
+        HIP_TRY(hipMalloc(&b->dStage, step * nx * sizeof(double)));
+        b->stage_doubles = step * nx;
     }
-    // FP32: through an FP64 buffer of the pool's shape (its padding slots are
-    // converted along and never read back)
-    double *tmp = nullptr;
-    HIP_TRY(hipMalloc(&tmp, nb64));
-    lbm::StepParams<double> p = batch_params(b);
-    p.nx = L.pitch;
-    p.ny = L.ny;
-    p.plane = L.plane;
-    hipError_t e = hipSuccess;
-    if (up) e = hipMemcpy2DAsync(tmp, drow, host, hrow, hrow, rows, hipMemcpyHostToDevice, g_stream);
-    int rc = 0;
-    if (e == hipSuccess) rc = lbm::dispatch_upload(b->qid, b->storage, tmp, dst, p, up ? 1 : 0, g_stream);
-    if (e == hipSuccess && !rc && !up)
-        e = hipMemcpy2DAsync(host, hrow, tmp, drow, hrow, rows, hipMemcpyDeviceToHost, g_stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
-    (void)hipFree(tmp);
-    if (e != hipSuccess) return fail(-3, "batch transfer failed: %s", hipGetErrorString(e));
-    if (rc) return fail(-4, "conversion kernel failed (%d)", rc);
+    const int eb = batch_elem(b);
+    char *pool = static_cast<char *>(b->pool);
+    const lbm::StepParams<double> p = batch_params(b);
+    for (size_t r = 0; r < rows; r += step) {
+        const size_t n = rows - r < step ? rows - r : step, bytes = n * nx * sizeof(double);
+        if (up) HIP_TRY(hipMemcpyAsync(b->dStage, host + r * nx, bytes, hipMemcpyHostToDevice, g_stream));
+        if (lbm::dispatch_batch_xfer(b->storage, b->dStage, pool + (size_t)L.off[up ? 0 : buf] * eb,
+                                     pool + (size_t)L.off[1] * eb, L, (int)r, (int)n, p, up ? 1 : 0,
+                                     g_stream))
+            return fail(-4, "batch transfer kernel failed");
+        if (!up) HIP_TRY(hipMemcpyAsync(host + r * nx, b->dStage, bytes, hipMemcpyDeviceToHost, g_stream));
+    }
+    HIP_TRY(hipStreamSynchronize(g_stream));
     return 0;
 }
 
 int lbm_batch_upload(lbm_batch b, int k, const double *f) {
-    if (int rc = batch_xfer(b, k, 0, const_cast<double *>(f), true)) return rc;
-    if (int rc = batch_xfer(b, k, 1, const_cast<double *>(f), true)) return rc;
-    return 0;
+    return batch_xfer(b, k, 0, const_cast<double *>(f), true);
 }
 
 int lbm_batch_download(lbm_batch b, int k, int role, double *f) {
@@ -1969,6 +2017,7 @@ int lbm_batch_set_launch(lbm_batch b, int block, int grid) {
     if (grid < 0) return fail(-1, "grid must be >= 0");
     b->block = block ? block : 128;
     b->grid = grid;
+    b->explicit_shape = block != 0 || grid != 0;
     return 0;
 }
 
@@ -1993,17 +2042,42 @@ int lbm_batch_simulate(lbm_batch b, int64_t nsteps, int graph_chunk, double *ms_
     if (nsteps < 0 || graph_chunk < 0) return fail(-1, "negative step count");
     if (ms_fused) *ms_fused = 0.0;
     if (nsteps == 0) return 0;
+    const bool automatic = !b->explicit_shape && b->vec == 1;
+    if (automatic)
+        if (int rc = batch_regions(b)) return rc;
+    const bool multi = automatic && b->region_mode == 1 && nsteps >= 2;
+    const int tmax = b->storage == LBM_STORE_F64 ? lbm::kBatchStepsF64 : lbm::kBatchStepsF32;
+    // equal passes: the last ones are not left with a single step
+    auto pass = [&](int64_t left) {
+        const int64_t n = (left + tmax - 1) / tmax;
+        return (int)((left + n - 1) / n);
+    };
     const int chunk = graph_chunk & ~1;  // even: the parity returns after a replay
-    if (int rc = batch_launch(b, 0, b->parity_stream)) return rc;  // C_0 = collide(S_0)
-    int cur = b->parity_stream ^ 1;
+    int64_t left = nsteps;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (ms_fused) {
         HIP_TRY(hipEventCreate(&e0));
         HIP_TRY(hipEventCreate(&e1));
-        HIP_TRY(hipEventRecord(e0, g_stream));
+        if (multi) HIP_TRY(hipEventRecord(e0, g_stream));  // its first pass is t - 1 of the steps
     }
-    int64_t left = nsteps - 1;
-    if (chunk > 0 && left >= chunk) {
+    if (multi) {
+        const int t = pass(left);  // C_{t-1} from S_0
+        if (int rc = batch_pass(b, b->parity_stream, t, true)) return rc;
+        left -= t;
+    } else {
+        if (int rc = batch_launch(b, 0, b->parity_stream)) return rc;  // C_0 = collide(S_0)
+        left -= 1;
+    }
+    int cur = b->parity_stream ^ 1;
+    if (ms_fused && !multi) HIP_TRY(hipEventRecord(e0, g_stream));
+    if (multi) {
+        while (left > 0) {
+            const int t = pass(left);
+            if (int rc = batch_pass(b, cur, t, false)) return rc;
+            cur ^= 1;
+            left -= t;
+        }
+    } else if (chunk > 0 && left >= chunk) {
         if (int rc = batch_graph(b, chunk, cur)) return rc;
         while (left >= chunk) {
             HIP_TRY(hipGraphLaunch(b->gexec, g_stream));
@@ -2037,6 +2111,8 @@ int lbm_batch_autotune(lbm_batch b, int trial_steps, int *block, int *grid, doub
     HIP_TRY(hipMalloc(&save, b->pool_bytes));
     int rc = lbm_field_copy_raw(save, b->pool, b->pool_bytes);
     const int saved_parity = b->parity_stream, sb = b->block, sg = b->grid, sv = b->vec;
+    const bool se = b->explicit_shape;
+    b->explicit_shape = true;
     double best = 1e300;
     int bb = 256, bg = 0, bv = 1;
     int dev = 0, cus = 256;
@@ -2069,10 +2145,30 @@ int lbm_batch_autotune(lbm_batch b, int trial_steps, int *block, int *grid, doub
                 }
             }
         }
+    // the several-step passes (the automatic shape), timed over whole passes
+    bool multi = false;
+    if (!rc && !(rc = batch_regions(b)) && b->region_mode == 1) {
+        const int tmax = b->storage == LBM_STORE_F64 ? lbm::kBatchStepsF64 : lbm::kBatchStepsF32;
+        const int steps = ((trial_steps + tmax - 1) / tmax + 1) * tmax;
+        double ms = 0.0;
+        b->explicit_shape = false;
+        b->vec = 1;
+        rc = lbm_batch_simulate(b, steps, 0, &ms);
+        const double us = 1e3 * ms / steps;
+        if (!rc && us < best) {
+            best = us;
+            multi = true;
+            bb = 128;
+            bv = 1;
+            rc = batch_tiles(b, bb * bv);
+            bg = b->ntiles;
+        }
+    }
     if (!rc) rc = lbm_field_copy_raw(b->pool, save, b->pool_bytes);
     (void)hipStreamSynchronize(g_stream);
     (void)hipFree(save);
     b->parity_stream = saved_parity;
+    b->explicit_shape = rc ? se : !multi;
     batch_drop_graph(b);
     if (rc) {
         b->block = sb;

@@ -107,6 +107,15 @@ struct BatchTile {
     int n0;
 };
 
+// One block's nodes of a batched lattice in a pass of several steps.
+struct BatchRegion {
+    int lat;
+    int x0, y0;
+    int outx, outy;
+};
+// rows of a block's region and largest pass (lbm_multi.h's wide blocks)
+constexpr int kBatchRowsF64 = 24, kBatchStepsF64 = 5, kBatchRowsF32 = 32, kBatchStepsF32 = 6;
+
 // FusedFirst: the first step of a run from the canonical state, collide +
 // stream + BCs + collide in one pass (FP64, one-speed stencils; the host
 // checks the tile shape)
@@ -196,6 +205,19 @@ LBM_DECLARE_MULTI(f32, float)
 LBM_DECLARE_MULTI(f16neq, float)
 LBM_DECLARE_MULTI(bf16neq, float)
 int dispatch_multi(int storage, const MultiLaunch &L, const StepParams<double> &p, hipStream_t s);
+
+// several steps of every batched lattice in one pass
+int run_batch_block_f64_q9(int coll, const BatchLattice *lats, const BatchRegion *regions,
+                           int nregions, void *pool, int parity, int levels, int first,
+                           const StepParams<double> &p, hipStream_t s);
+int run_batch_block_f32_q9(int coll, const BatchLattice *lats, const BatchRegion *regions,
+                           int nregions, void *pool, int parity, int levels, int first,
+                           const StepParams<float> &p, hipStream_t s);
+// rows row0 .. row0 + rows (of ny Q) of one batched lattice between a dense
+// FP64 array and the pool's padded rows; to the device both buffers are filled
+int dispatch_batch_xfer(int storage, double *dense, void *pooled, void *pooled2,
+                        const BatchLattice &L, int row0, int rows, const StepParams<double> &p,
+                        int to_device, hipStream_t s);
 
 LBM_DECLARE_ALL_Q(f64, double)
 LBM_DECLARE_ALL_Q(f32, float)

@@ -453,32 +453,37 @@ struct BlockArgs {
     WallArgs wall;
 };
 
+// the c_y != 0 populations of a wave's boundary rows, in LDS
+template <int QID>
+LBM_HD constexpr int edge_slot(int i) {
+    int n = 0;
+    for (int j = 0; j < i; ++j) n += QT<QID>::cy(j) != 0 ? 1 : 0;
+    return n;
+}
+// [buffer][wave][population][column]
+template <int QID, class V, int NW>
+using BlockEdges = V[2][NW][edge_slot<QID>(QT<QID>::Q)][66];
+
+// One block's region: writes the outx x outy nodes from (cx0, cy0) of a lattice
+// of p.nx x p.ny nodes with rows `pitch` apart.
 template <int QID, int COLL, class ST, int NW, int R, bool BC>
-__global__ void __launch_bounds__(64 * NW)
-k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
-        const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc,
-        const BlockArgs a) {
+__device__ __forceinline__ void
+block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
+             const StepParams<typename ST::T> &p, const MultiConsts<typename ST::T> &mc, int pitch,
+             int cx0, int cy0, int outx, int outy, int L, int first, WallArgs wall,
+             BlockEdges<QID, typename ST::T, NW> &xch) {
     using V = typename ST::T;
     using S = typename ST::store_t;
     constexpr int Q = QT<QID>::Q;
     static_assert(QT<QID>::MAXC == 1 && !ST::kNeq, "one-speed stencils, one value per population");
-    // the c_y != 0 populations of a wave's boundary rows: [buffer][wave][population][column]
-    constexpr auto edge_slot = [](int i) {
-        int n = 0;
-        for (int j = 0; j < i; ++j) n += QT<QID>::cy(j) != 0 ? 1 : 0;
-        return n;
-    };
-    constexpr int ES = edge_slot(Q);
-    __shared__ V xch[2][NW][ES][66];
+    constexpr int ES = edge_slot<QID>(Q);
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int ty = blockIdx.x / a.tiles_x, tx = blockIdx.x - ty * a.tiles_x;
-    const int L = a.levels, h = L - 1;
-    const int cx0 = tx * a.outx, cy0 = ty * a.outy;  // first node written
+    const int h = L - 1;
     const int ux = cx0 - h + lane;
     const int x = wrap(ux, p.nx);
-    const int xm = a.first ? x : (x == 0 ? p.nx - 1 : x - 1);
-    const int xp = a.first ? x : (x == p.nx - 1 ? 0 : x + 1);
+    const int xm = first ? x : (x == 0 ? p.nx - 1 : x - 1);
+    const int xp = first ? x : (x == p.nx - 1 ? 0 : x + 1);
     const unsigned off = (unsigned)x * (unsigned)sizeof(S);
     const unsigned offm = (unsigned)xm * (unsigned)sizeof(S), offp = (unsigned)xp * (unsigned)sizeof(S);
     const int row0 = w * R;  // the wave's first row in the region
@@ -488,19 +493,19 @@ k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
         ys[j] = __builtin_amdgcn_readfirstlane(wrap(cy0 - h + row0 + j, p.ny));
     unsigned bcm[R];
 #pragma unroll
-    for (int j = 0; j < R; ++j) bcm[j] = BC ? bc_mask<QID>(p, a.wall.walls, x, ys[j]) : 0u;
+    for (int j = 0; j < R; ++j) bcm[j] = BC ? bc_mask<QID>(p, wall.walls, x, ys[j]) : 0u;
     V g[R][Q];
     // level 1
     S pre[R][Q];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         const int y = ys[j];
-        const int ym = a.first ? y : (y == 0 ? p.ny - 1 : y - 1);
-        const int yp = a.first ? y : (y + 1 == p.ny ? 0 : y + 1);
+        const int ym = first ? y : (y == 0 ? p.ny - 1 : y - 1);
+        const int yp = first ? y : (y + 1 == p.ny ? 0 : y + 1);
         auto one = [&](auto Ic) {
             constexpr int i = decltype(Ic)::value;
             constexpr int cx = QT<QID>::cx(i), cy = QT<QID>::cy(i);
-            const S *base = C + p.plane * i + (long long)p.nx * (cy == 0 ? y : (cy > 0 ? ym : yp));
+            const S *base = C + p.plane * i + (long long)pitch * (cy == 0 ? y : (cy > 0 ? ym : yp));
             pre[j][i] = ld_g(at_b(base, cx == 0 ? off : (cx > 0 ? offm : offp)));
         };
         adj_each_node<QID>(one);
@@ -514,8 +519,8 @@ k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
         };
         adj_each_node<QID>(dec);
         if constexpr (BC) {
-            if (!a.first)
-                bc_apply<QID, V>(p, a.wall.moving, bcm[j], g[j], [&](auto Jc) {
+            if (!first)
+                bc_apply<QID, V>(p, wall.moving, bcm[j], g[j], [&](auto Jc) {
                     return ld_pop<QID, decltype(Jc)::value, ST>(C, p, (long long)x + (long long)p.nx * y);
                 });
         }
@@ -525,15 +530,15 @@ k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
         V(*X)[ES][66] = xch[l & 1];
         auto put = [&](auto Ic) {
             constexpr int i = decltype(Ic)::value, cy = QT<QID>::cy(i);
-            if constexpr (cy > 0) X[w][edge_slot(i)][lane + 1] = g[R - 1][i];
-            if constexpr (cy < 0) X[w][edge_slot(i)][lane + 1] = g[0][i];
+            if constexpr (cy > 0) X[w][edge_slot<QID>(i)][lane + 1] = g[R - 1][i];
+            if constexpr (cy < 0) X[w][edge_slot<QID>(i)][lane + 1] = g[0][i];
         };
         adj_each_node<QID>(put);
         __syncthreads();
         V carry[Q];  // c_y > 0 populations of the row below, already shifted along x
         auto below = [&](auto Ic) {
             constexpr int i = decltype(Ic)::value, cy = QT<QID>::cy(i);
-            if constexpr (cy > 0) carry[i] = X[w > 0 ? w - 1 : 0][edge_slot(i)][lane + 1 - QT<QID>::cx(i)];
+            if constexpr (cy > 0) carry[i] = X[w > 0 ? w - 1 : 0][edge_slot<QID>(i)][lane + 1 - QT<QID>::cx(i)];
         };
         adj_each_node<QID>(below);
 #pragma unroll
@@ -555,12 +560,12 @@ k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
                     f[i] = sh(g[j][i]);
                 } else {
                     if (j + 1 < R) f[i] = sh(g[j + 1 < R ? j + 1 : j][i]);
-                    else f[i] = X[w + 1 < NW ? w + 1 : w][edge_slot(i)][lane + 1 - cx];
+                    else f[i] = X[w + 1 < NW ? w + 1 : w][edge_slot<QID>(i)][lane + 1 - cx];
                 }
             };
             adj_each_node<QID>(pull);
             if constexpr (BC) {
-                bc_apply<QID, V>(p, a.wall.moving, bcm[j], f,
+                bc_apply<QID, V>(p, wall.moving, bcm[j], f,
                                  [&](auto Jc) { return g[j][decltype(Jc)::value]; });
             }
             collide_multi<QID, COLL, V>(f, p, mc, x, y);
@@ -571,12 +576,12 @@ k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
             adj_each_node<QID>(cp);
         }
     }
-    if (ux >= cx0 && ux < min(cx0 + a.outx, p.nx)) {
+    if (ux >= cx0 && ux < min(cx0 + outx, p.nx)) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             const int uy = cy0 - h + row0 + j;
-            if (uy >= cy0 && uy < min(cy0 + a.outy, p.ny)) {
-                S *base = Cn + (long long)p.nx * uy;
+            if (uy >= cy0 && uy < min(cy0 + outy, p.ny)) {
+                S *base = Cn + (long long)pitch * uy;
                 auto st = [&](auto Ic) {
                     constexpr int i = decltype(Ic)::value;
                     *at_b(base + p.plane * i, off) = ST::encode(g[j][i], i, p);
@@ -585,6 +590,47 @@ k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
             }
         }
     }
+}
+
+template <int QID, int COLL, class ST, int NW, int R, bool BC>
+__global__ void __launch_bounds__(64 * NW)
+k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
+        const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc,
+        const BlockArgs a) {
+    __shared__ BlockEdges<QID, typename ST::T, NW> xch;
+    const int ty = blockIdx.x / a.tiles_x, tx = blockIdx.x - ty * a.tiles_x;
+    block_region<QID, COLL, ST, NW, R, BC>(C, Cn, p, mc, p.nx, tx * a.outx, ty * a.outy, a.outx,
+                                           a.outy, a.levels, a.first, a.wall, xch);
+}
+
+// Batched lattices: one region per block from a table; the lattice record is
+// read in place with a wave-uniform index (scalar loads).  Bound by FP
+// arithmetic like k_block; 512 lattices of 200 x 200, us a step against the
+// single-step kernel's: 194 / 510 in FP64, 90 / 303 in FP32 (single steps are
+// bound by the passes over the pool, 2.9 and 2.4 TB/s there).
+template <int QID, int COLL, class ST, int NW, int R>
+__global__ void __launch_bounds__(64 * NW)
+k_batch_block(const BatchLattice *__restrict__ lats, const BatchRegion *__restrict__ regions,
+              typename ST::store_t *__restrict__ pool, int parity, int levels, int first,
+              const StepParams<typename ST::T> base, const MultiConsts<typename ST::T> base_mc) {
+    using T = typename ST::T;
+    __shared__ BlockEdges<QID, T, NW> xch;
+    const BatchRegion g = regions[blockIdx.x];
+    const BatchLattice &lat = lats[__builtin_amdgcn_readfirstlane(g.lat)];
+    StepParams<T> p = base;
+    p.nx = lat.nx;
+    p.ny = lat.ny;
+    p.plane = lat.plane;
+    p.omo = static_cast<T>(lat.omo);
+    p.om = static_cast<T>(lat.om);
+    p.oms = static_cast<T>(lat.oms);
+    p.oma = static_cast<T>(lat.oma);
+    MultiConsts<T> mc = base_mc;
+    mc.homs = T(0.5) * p.oms;
+    mc.homa = T(0.5) * p.oma;
+    block_region<QID, COLL, ST, NW, R, false>(pool + lat.off[parity], pool + lat.off[parity ^ 1], p,
+                                              mc, lat.pitch, g.x0, g.y0, g.outx, g.outy, levels,
+                                              first, WallArgs{0, 0}, xch);
 }
 
 // ---------------------------------------------------------------------------
@@ -975,6 +1021,35 @@ int launch_multi(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipS
     }
     return -2;
 }
+
+// Batched lattices: the wide blocks (the region table is cut for the largest
+// pass; smaller passes use the same regions)
+template <int QID, class ST>
+int launch_batch_block(int coll, const BatchLattice *lats, const BatchRegion *regions, int nregions,
+                       void *pool, int parity, int levels, int first,
+                       const StepParams<typename ST::T> &p, hipStream_t s) {
+    using S = typename ST::store_t;
+    constexpr int NW = 8, R = sizeof(S) == 8 ? kBatchRowsF64 / NW : kBatchRowsF32 / NW;
+    constexpr int tmax = sizeof(S) == 8 ? kBatchStepsF64 : kBatchStepsF32;
+    if (levels < 1 || levels > tmax || nregions < 1) return -5;
+    S *pl = static_cast<S *>(pool);
+    if (coll == 0)
+        k_batch_block<QID, 0, ST, NW, R><<<(unsigned)nregions, 64 * NW, 0, s>>>(
+            lats, regions, pl, parity, levels, first, p, multi_consts(p));
+    else
+        k_batch_block<QID, 1, ST, NW, R><<<(unsigned)nregions, 64 * NW, 0, s>>>(
+            lats, regions, pl, parity, levels, first, p, multi_consts(p));
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+#define LBM_DEFINE_BATCH_BLOCK(TAG, ST, QID)                                                     \
+    int run_batch_block_##TAG##_q##QID(int coll, const BatchLattice *lats,                       \
+                                       const BatchRegion *regions, int nregions, void *pool,     \
+                                       int parity, int levels, int first,                        \
+                                       const StepParams<typename ST::T> &p, hipStream_t s) {     \
+        return launch_batch_block<QID, ST>(coll, lats, regions, nregions, pool, parity, levels,  \
+                                           first, p, s);                                         \
+    }
 
 // one translation unit per (storage, quadrature)
 #define LBM_DEFINE_MULTI(TAG, ST, QID)                                                      \

@@ -146,3 +146,56 @@ def test_neq_error_no_larger_than_single_steps(oracle_lib, storage, qid, coll, s
     for a, b, ref in ((many.f_stream, one.f_stream, S), (many.f_collision, one.f_collision, C)):
         ea, eb = (np.linalg.norm(x.to_numpy() - ref) for x in (a, b))
         assert ea <= 1.1 * eb, (ea, eb)
+
+
+# a batch: widths and heights at one and two blocks' outputs (56 x 16 FP64,
+# 54 x 22 FP32) and beside them, narrower and lower than a block's halo, long
+# rows; big enough on average for the several-step passes
+BATCH = [(56, 16), (57, 17), (54, 22), (300, 129), (113, 45), (129, 200), (7, 90), (200, 5),
+         (256, 256), (1, 64), (64, 1), (333, 77)]
+
+
+def _batch(storage, trt, noise):
+    rng = np.random.default_rng(3)
+    ts = rng.uniform(0.55, 1.4, len(BATCH))
+    ta = 0.5 + 0.25 / (ts - 0.5) if trt else None
+    L = _L()
+    b = L.LatticeBatch(L.D2Q9(), BATCH, ts, ta, storage=storage)
+    f0 = [_populations(9, nx, ny, seed=k, noise=noise) for k, (nx, ny) in enumerate(BATCH)]
+    for k, f in enumerate(f0):
+        b.upload(k, f)
+        if storage == "f64":
+            assert np.array_equal(b.download(k, "f_collision"), f)
+    return b, f0, [[ts[k], ta[k]] if trt else [ts[k]] for k in range(len(BATCH))]
+
+
+@pytest.mark.parametrize("trt", [False, True])
+@pytest.mark.parametrize("calls", [(1, 2), (3, 1), (4,), (5,), (6, 7), (23,)])
+def test_batch_f64_bit_exact(oracle_lib, trt, calls):
+    b, f0, taus = _batch("f64", trt, 2e-3)
+    print(f"batch f64 trt {trt} {calls}", flush=True)
+    for n in calls:
+        b.simulate(n)
+    b.set_launch(64, 0)  # the single-step kernel goes on from the same state
+    b.simulate(2)
+    b.set_launch(0, 0)
+    b.simulate(2)
+    for k, f in enumerate(f0):
+        S, C = _oracle(oracle_lib, 9, f, int(trt), taus[k], sum(calls) + 4, None, [])
+        assert np.array_equal(b.download(k, "f_stream"), S), BATCH[k]
+        assert np.array_equal(b.download(k, "f_collision"), C), BATCH[k]
+
+
+@pytest.mark.parametrize("trt", [False, True])
+@pytest.mark.parametrize("steps", [2, 6, 13])
+def test_batch_f32_tracks_oracle(oracle_lib, trt, steps):
+    """the bound of test_f32_tracks_oracle, lattice by lattice"""
+    b, f0, taus = _batch("f32", trt, 1e-4)
+    b.simulate(steps)
+    w = np.asarray(_L().D2Q9().weights)
+    for k, f in enumerate(f0):
+        S, C = _oracle(oracle_lib, 9, f, int(trt), taus[k], steps, None, [])
+        G = max(np.abs(S - w).max(), np.abs(C - w).max(), np.abs(f - w).max())
+        tol = 16 * (steps + 1) * 2.0 ** -24 * G
+        assert np.abs(b.download(k, "f_stream") - S).max() <= tol, BATCH[k]
+        assert np.abs(b.download(k, "f_collision") - C).max() <= tol, BATCH[k]
