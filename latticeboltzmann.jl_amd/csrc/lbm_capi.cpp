@@ -529,6 +529,12 @@ struct MultiPlan {
 // (below this the 16-bit storages keep the single-step row kernel)
 constexpr long long kNeqMarchNodes = 800000;
 
+// lattices for the 8 x 8 tiles (420 of them: 164 x 164, FP64 160^2 2.0 us a
+// step against 1.9 with the 64 x 16 blocks)
+bool small_tiles(const lbm_field_s *f) {
+    return (long long)((f->nx + 7) / 8) * ((f->ny + 7) / 8) <= 420;
+}
+
 MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     MultiPlan pl;
     if (m->launch_block || m->launch_rows || m->launch_vec || m->launch_nt >= 0) {
@@ -567,9 +573,7 @@ MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     }
     const bool f64 = f->storage == LBM_STORE_F64;
     if (!f64 && f->storage != LBM_STORE_F32) return pl;
-    // (420 tiles: 164 x 164, FP64 160^2 2.0 us against 1.9 with the 64 x 16 blocks)
-    const long long tiles = (long long)((f->nx + 7) / 8) * ((f->ny + 7) / 8);
-    if (tiles <= 420) any_up_to(lbm::kMultiTile, 8);
+    if (small_tiles(f)) any_up_to(lbm::kMultiTile, 8);
     else if (!wide) return pl;
     else if (nodes <= 90000) any_up_to(lbm::kMultiBlock16, 6);
     else if (nodes <= 400000) any_up_to(lbm::kMultiBlock32, 6);
@@ -602,6 +606,13 @@ int multi_next(const MultiPlan &pl, int64_t left) {
     return pass[left];
 }
 
+void boundary_walls(const lbm_model_s *m, lbm::MultiLaunch &L) {
+    for (size_t b = 0; b < m->bcs.size(); ++b) {
+        L.walls |= 1 << m->bcs[b].direction;
+        if (m->bcs[b].kind == LBM_MOVING_WALL) L.moving = (int)b;
+    }
+}
+
 int run_multi(const MultiPlan &pl, lbm_model m, lbm_field src, lbm_field dst, int steps, bool first) {
     lbm::MultiLaunch L{};
     L.kernel = pl.kernel;
@@ -609,10 +620,7 @@ int run_multi(const MultiPlan &pl, lbm_model m, lbm_field src, lbm_field dst, in
     L.coll = m->coll;
     L.steps = steps;
     L.first = first ? 1 : 0;
-    for (size_t b = 0; b < m->bcs.size(); ++b) {
-        L.walls |= 1 << m->bcs[b].direction;
-        if (m->bcs[b].kind == LBM_MOVING_WALL) L.moving = (int)b;
-    }
+    boundary_walls(m, L);
     L.src = src->d;
     L.dst = dst->d;
     const int rc = lbm::dispatch_multi(src->storage, L, make_params(m, src, true), g_stream);
@@ -1487,6 +1495,25 @@ int lbm_field_node(lbm_field f, int x, int y, double *out) {
     return 0;
 }
 
+namespace {
+// several steps per launch: lattices that the 8 x 8 tiles suit (multi_plan's line)
+bool mei_tiles(const lbm_model_s *m, const lbm_field_s *f) {
+    return (m->qid == 4 || m->qid == 5 || m->qid == 9) && small_tiles(f);
+}
+
+int run_mei_tiles(lbm_model m, const lbm::StepParams<double> &p, lbm_field src, lbm_field dst,
+                  int n, const lbm::MeiStop &stop) {
+    lbm::MultiLaunch L{};
+    L.qid = m->qid;
+    L.steps = n;
+    boundary_walls(m, L);
+    L.src = src->d;
+    L.dst = dst->d;
+    L.mei = stop;
+    return lbm::run_mei_tile(L, p, g_stream);
+}
+}  // namespace
+
 int lbm_mei_initialize(lbm_model m, lbm_field f_stream, lbm_field f_collision, double eps,
                        int64_t max_steps, int64_t *steps) {
     if (int rc = check_pair(m, f_stream, f_collision, "lbm_mei_initialize", true, true)) return rc;
@@ -1494,42 +1521,65 @@ int lbm_mei_initialize(lbm_model m, lbm_field f_stream, lbm_field f_collision, d
         return fail(-1, "lbm_mei_initialize: the model has no initialization velocity "
                         "(lbm_model_set_mei)");
     if (max_steps < 1) return fail(-1, "lbm_mei_initialize: max_steps must be positive");
-    const lbm::StepParams<double> p = field_params(f_stream);
-    // f = w everywhere (mei_et_al.jl:21-25), in both roles
-    int rc = lbm::dispatch_fill_weights(static_cast<double *>(f_stream->d), p, f_stream->Q, g_stream);
-    if (!rc) rc = lbm::dispatch_fill_weights(static_cast<double *>(f_collision->d), p,
-                                             f_stream->Q, g_stream);
+    // f = w everywhere (mei_et_al.jl:21-25); C_0 = collide(f)
+    const lbm::StepParams<double> p = make_params(m, f_stream, true);
+    int rc = lbm::dispatch_fill_weights(static_cast<double *>(f_stream->d), field_params(f_stream),
+                                        f_stream->Q, g_stream);
     if (rc) return fail(-4, "lbm_mei_initialize: fill kernel failed (%d)", rc);
-    double *dnode = nullptr;
-    HIP_TRY(hipMalloc(&dnode, 64 * sizeof(double)));
-    const long long corner = (long long)(f_stream->nx - 1) + (long long)f_stream->nx * (f_stream->ny - 1);
-    double rho = 0.0, rho_old = 0.0, node[64];
-    int64_t t = 1;
-    hipError_t e = hipSuccess;
-    for (; t <= max_steps; ++t) {
-        if ((rc = run(lbm::Op::Collide, m, f_stream, f_collision, false))) break;
-        if ((rc = run(lbm::Op::StreamBC, m, f_collision, f_stream, true))) break;
-        // next!(ProcessIterativeInitialization): DensityConvergence at node (nx, ny)
-        if ((rc = lbm::dispatch_gather_node(LBM_STORE_F64, f_stream->d, p, corner, f_stream->Q,
-                                            dnode, g_stream))) {
-            rc = fail(-4, "lbm_mei_initialize: gather kernel failed (%d)", rc);
-            break;
+    if ((rc = run(lbm::Op::Collide, m, f_stream, f_collision, false))) return rc;
+    lbm::MeiWatch *watch = nullptr, host{};
+    HIP_TRY(hipMalloc(&watch, sizeof(lbm::MeiWatch)));
+    hipError_t e = hipMemcpyAsync(watch, &host, sizeof(host), hipMemcpyHostToDevice, g_stream);
+    // Steps 1 .. max_steps - 1 run as C_(t-1) -> C_t, each checking its S_t
+    // (ProcessIterativeInitialization, DensityConvergence at node (nx, ny));
+    // S_max_steps, which ends the loop whether it converged or not, is only
+    // streamed.  Launches after the one that converged do nothing, so the host
+    // looks at the record once per batch of them.
+    const bool tiles = mei_tiles(m, f_stream);
+    const int tmax = tiles ? 8 : 1;
+    auto pass = [&](lbm_field src, lbm_field dst, int64_t t, int n, bool watched) {
+        const lbm::MeiStop stop{watched ? watch : nullptr, eps, t};
+        const int r = tiles ? run_mei_tiles(m, p, src, dst, n, stop)
+                            : lbm::run_mei_step(m->qid, static_cast<const double *>(src->d),
+                                                static_cast<double *>(dst->d), p, stop, g_stream);
+        return r ? fail(-4, "lbm_mei_initialize: step kernel failed (%d)", r) : 0;
+    };
+    lbm_field cur = f_collision, other = f_stream;
+    int64_t t = 1, stopped = 0;  // cur holds C_(t-1)
+    for (int batch = 4; !rc && e == hipSuccess && t < max_steps && !stopped;
+         batch = batch < 32 ? 2 * batch : 32) {
+        const lbm_field cur0 = cur, other0 = other;
+        const int64_t t0 = t;
+        for (int k = 0; !rc && k < batch && t < max_steps; ++k) {
+            const int n = (int)std::min<int64_t>(tmax, max_steps - t);
+            rc = pass(cur, other, t, n, true);
+            t += n;
+            std::swap(cur, other);
         }
-        e = hipMemcpyAsync(node, dnode, (size_t)f_stream->Q * sizeof(double),
-                           hipMemcpyDeviceToHost, g_stream);
+        if (rc) break;
+        e = hipMemcpyAsync(&host, watch, sizeof(host), hipMemcpyDeviceToHost, g_stream);
         if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
-        if (e != hipSuccess) break;
-        double r = node[0] + node[1];
-        for (int i = 2; i < f_stream->Q; ++i) r = r + node[i];
-        rho_old = rho;
-        rho = r;
-        const double d = std::fabs(rho - rho_old);
-        if (d < eps || d > 100.0) break;
+        if (e != hipSuccess || !host.stop) continue;
+        // the pass that holds step `stop`: its source C_(t-1) was not written
+        // again; run it as far as C_(stop-1)
+        stopped = host.stop;
+        cur = cur0;
+        other = other0;
+        for (t = t0; t + tmax <= stopped; t += tmax) std::swap(cur, other);
+        if (stopped > t) {
+            rc = pass(cur, other, t, (int)(stopped - t), false);
+            std::swap(cur, other);
+        }
     }
-    free_dev(reinterpret_cast<void *&>(dnode));
+    (void)hipStreamSynchronize(g_stream);
+    free_dev(reinterpret_cast<void *&>(watch));
     if (e != hipSuccess) return fail(-3, "lbm_mei_initialize: %s", hipGetErrorString(e));
     if (rc) return rc;
-    if (steps) *steps = t > max_steps ? max_steps : t;
+    if (cur != f_collision)
+        HIP_TRY(hipMemcpyAsync(f_collision->d, cur->d, f_collision->bytes, hipMemcpyDeviceToDevice,
+                               g_stream));
+    if ((rc = run(lbm::Op::StreamBC, m, f_collision, f_stream, true))) return rc;
+    if (steps) *steps = stopped ? stopped : max_steps;
     return 0;
 }
 

@@ -146,6 +146,17 @@ enum MultiKernel : int {
     kMultiNone
 };
 constexpr int kMarchRows = 16;  // fewest rows of a marching wave
+// Stop of the iterative initialization, kept on the device: the density of
+// node (nx, ny) after the last step and the first step that converged (0: none)
+struct MeiWatch {
+    double rho;
+    long long stop;
+};
+struct MeiStop {
+    MeiWatch *watch;  // null: the steps run unconditionally
+    double eps;
+    long long step;  // the state that the launch's first level collides is S_step
+};
 struct MultiLaunch {
     int kernel;
     int qid, coll;  // as in Launch
@@ -155,6 +166,7 @@ struct MultiLaunch {
     int moving;     // index of its last moving wall
     const void *src;
     void *dst;
+    MeiStop mei;    // iterative initialization only
 };
 
 // Reverse-mode kernels of the periodic SRT/TRT step (lbm_adjoint.h).
@@ -204,6 +216,11 @@ LBM_DECLARE_MULTI(f64, double)
 LBM_DECLARE_MULTI(f32, float)
 LBM_DECLARE_MULTI(f16neq, float)
 LBM_DECLARE_MULTI(bf16neq, float)
+// steps of the iterative initialization, C_(t-1) -> C_t: one (every stencil),
+// or several on tiles (one-speed stencils)
+int run_mei_step(int qid, const double *src, double *dst, const StepParams<double> &p,
+                 const MeiStop &stop, hipStream_t s);
+int run_mei_tile(const MultiLaunch &L, const StepParams<double> &p, hipStream_t s);
 int dispatch_multi(int storage, const MultiLaunch &L, const StepParams<double> &p, hipStream_t s);
 
 // several steps of every batched lattice in one pass

@@ -223,6 +223,31 @@ __device__ __forceinline__ void collide_multi(T (&f)[QT<QID>::Q], const StepPara
     }
 }
 
+// The stop of the iterative initialization (DensityConvergence at node
+// (nx, ny)), taken on the device: the thread that holds the corner compares the
+// density of each new state with the previous one's and records the first step
+// that converged; launches after that return at once, so the state before it
+// is still in its buffer.  Blocks of the recording launch may or may not see
+// the record: its output is not used once the record is set.
+template <int QID, int... Is>
+__device__ __forceinline__ double mei_density(const double (&f)[QT<QID>::Q],
+                                              std::integer_sequence<int, Is...>) {
+    double r = f[0] + f[1];
+    ((Is > 1 ? (void)(r = r + f[Is]) : (void)0), ...);
+    return r;
+}
+__device__ __forceinline__ long long mei_stopped(const MeiWatch *w) {
+    return __hip_atomic_load(&w->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int QID>
+__device__ __forceinline__ void mei_check(const MeiStop &m, const double (&f)[QT<QID>::Q], long long step) {
+    const double rho = mei_density<QID>(f, LBM_SEQ), d = fabs(rho - m.watch->rho);
+    if (mei_stopped(m.watch) != 0) return;
+    m.watch->rho = rho;
+    if (d < m.eps || d > 100.0)
+        __hip_atomic_store(&m.watch->stop, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The boundary list of a node (apply_bc_seq's semantics) as a mask, formed once
 // per node and pass: bit i is set when population i is replaced by the node's
 // own post-collision opp(i), bit 16 + i when the last condition that replaces
@@ -308,6 +333,7 @@ struct TileArgs {
     int tiles_x;
     int first;
     WallArgs wall;
+    MeiStop mei;  // COLL == 3: the iterative initialization's stop
 };
 
 template <int QID, class ST, int TX, int TY, int TMAX, int NT>
@@ -327,6 +353,8 @@ k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restr
     constexpr int Q = QT<QID>::Q, M = QT<QID>::MAXC, W = SH::W, N = SH::N, K = SH::K;
     static_assert(M == 1 && !ST::kNeq, "one-speed stencils, one value per population");
     __shared__ T buf[Q * N];
+    if constexpr (COLL == 3)
+        if (a.mei.watch && mei_stopped(a.mei.watch) != 0) return;
     const int ty = blockIdx.x / a.tiles_x, tx = blockIdx.x - ty * a.tiles_x;
     int at[K], xs[K], ys[K], ring[K];
     unsigned bcm[K];
@@ -347,6 +375,35 @@ k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restr
     }
     const int L = a.levels;
     T f[K][Q];
+    // the prescribed velocity's part of the equilibrium, read once for all levels
+    T pre[COLL == 3 ? K : 1][COLL == 3 ? Q : 1];
+    if constexpr (COLL == 3) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (ring[k] > L - 1) continue;
+            auto ld = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                pre[k][i] = p.mei[p.plane * i + (long long)xs[k] + (long long)p.nx * ys[k]];
+            };
+            adj_each_node<QID>(ld);
+        }
+    }
+    // level l's collision of node k, whose state is S_(step + l - 1)
+    auto collide = [&](int k, int l) {
+        if constexpr (COLL == 3) {
+            if (a.mei.watch && mine[k] && xs[k] == p.nx - 1 && ys[k] == p.ny - 1)
+                mei_check<QID>(a.mei, f[k], a.mei.step + l - 1);
+            const T rho = mei_density<QID>(f[k], LBM_SEQ);
+            auto one = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                const T feq = p.w[i] * rho + pre[k][i];
+                f[k][i] = p.omo * f[k][i] + p.om * feq;
+            };
+            adj_each_node<QID>(one);
+        } else {
+            collide_multi<QID, COLL, T>(f[k], p, mc, xs[k], ys[k]);
+        }
+    };
     // level 1 from HBM
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -377,7 +434,7 @@ k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restr
                         C, p, (long long)xs[k] + (long long)p.nx * ys[k]);
                 });
         }
-        collide_multi<QID, COLL, T>(f[k], p, mc, xs[k], ys[k]);
+        collide(k, 1);
     }
     for (int l = 2; l <= L; ++l) {
 #pragma unroll
@@ -407,7 +464,7 @@ k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restr
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             if (ring[k] > L - l) continue;
-            collide_multi<QID, COLL, T>(f[k], p, mc, xs[k], ys[k]);
+            collide(k, l);
         }
     }
 #pragma unroll
@@ -907,6 +964,7 @@ int launch_tile(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipSt
     a.levels = L.steps;
     a.first = L.first;
     a.wall = WallArgs{L.walls, L.moving};
+    a.mei = L.mei;
     a.tiles_x = (p.nx + kTileX - 1) / kTileX;
     const int tiles_y = (p.ny + kTileY - 1) / kTileY;
     k_tile<QID, COLL, ST, kTileX, kTileY, kTileT, kTileThreads, BC>

@@ -199,3 +199,44 @@ def test_batch_f32_tracks_oracle(oracle_lib, trt, steps):
         tol = 16 * (steps + 1) * 2.0 ** -24 * G
         assert np.abs(b.download(k, "f_stream") - S).max() <= tol, BATCH[k]
         assert np.abs(b.download(k, "f_collision") - C).max() <= tol, BATCH[k]
+
+
+# the iterative initialization: up to 420 tiles (168 x 160) several steps a
+# launch, beyond them and on the other stencils one
+MEI = [(9, 5, 7), (9, 33, 20), (9, 168, 160), (9, 169, 160), (4, 24, 31), (5, 24, 31),
+       (13, 40, 17), (17, 70, 9), (37, 20, 33)]
+
+
+def _mei_run(qid, u, bcs, eps, max_steps):
+    import ctypes
+    L = _L()
+    from lbmhip import _lib
+    from lbmhip.operators import native_model
+    q = L.Quadratures[f"D2Q{qid}"]()
+    nx, ny = u.shape[:2]
+    fs, fc = L.HipLattice(q, nx, ny), L.HipLattice(q, nx, ny)
+    m = native_model(q).configure(L.IterativeInitializationCollisionModel(0.8, u), fs, bcs)
+    steps = ctypes.c_int64()
+    _lib.check(_lib.lib().lbm_mei_initialize(m.handle, fs.handle, fc.handle, eps, max_steps,
+                                             ctypes.byref(steps)), "lbm_mei_initialize")
+    return fs.to_numpy(), fc.to_numpy(), steps.value
+
+
+@pytest.mark.parametrize("qid,nx,ny", MEI)
+@pytest.mark.parametrize("bcname", ["periodic", "couette"])
+@pytest.mark.parametrize("eps,max_steps", [
+    (0.0, 1), (0.0, 2), (0.0, 9), (0.0, 10), (0.0, 41), (2.0, 30),
+    (5e-3, 200), (3e-3, 200), (1e-3, 200), (5e-4, 200), (1e-4, 200), (1e-6, 200)])
+def test_mei_initialize_bit_exact(oracle_lib, qid, nx, ny, bcname, eps, max_steps):
+    """steps run, f_stream and f_collision, with stops inside and at the ends
+    of passes"""
+    x, y = np.meshgrid(np.arange(nx) * 2 * np.pi / nx, np.arange(ny) * 2 * np.pi / ny,
+                       indexing="ij")
+    u = np.asfortranarray(np.stack([0.03 * np.cos(x) * np.sin(y), 0.02 * np.sin(x + y)], axis=-1))
+    bcd = bc_dicts(bcname, nx, ny)
+    print(f"mei D2Q{qid} {nx}x{ny} {bcname} eps {eps} {max_steps}", flush=True)
+    S, C, n = oracle_lib.mei_initialize(qid, u, 0.8, eps, max_steps, bcd)
+    s, c, steps = _mei_run(qid, u, to_lbmhip(bcd), eps, max_steps)
+    assert steps == n
+    assert np.array_equal(s, S)
+    assert np.array_equal(c, C)
