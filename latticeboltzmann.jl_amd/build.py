@@ -64,7 +64,7 @@ def _deps(src):
     if src.startswith("k_multi"):
         return kern + [os.path.join(CSRC, "lbm_multi.h")]
     if src.startswith("k_adjoint"):
-        return kern + [os.path.join(CSRC, "lbm_adjoint.h")]
+        return kern + [os.path.join(CSRC, "lbm_multi.h"), os.path.join(CSRC, "lbm_adjoint.h")]
     return kern
 
 

@@ -529,8 +529,8 @@ struct MultiPlan {
 // (below this the 16-bit storages keep the single-step row kernel)
 constexpr long long kNeqMarchNodes = 800000;
 
-// lattices for the 8 x 8 tiles (420 of them: 164 x 164, FP64 160^2 2.0 us a
-// step against 1.9 with the 64 x 16 blocks)
+// lattices for the 8 x 8 tiles (420 of them: 164 x 164; us a step on 160^2
+// against the 64 x 16 blocks: 1.66 / 1.79 in FP64, 0.95 / 1.09 in FP32)
 bool small_tiles(const lbm_field_s *f) {
     return (long long)((f->nx + 7) / 8) * ((f->ny + 7) / 8) <= 420;
 }
@@ -2327,10 +2327,71 @@ int adj_forward_op(lbm_adjoint a, lbm::Op op, const void *src, void *dst) {
     return 0;
 }
 
-// post-collision buffer of forward step t: checkpoints at t = aK - 1
-void *adj_cbuf(lbm_adjoint a, int64_t t) {
-    if ((t + 1) % a->K == 0 && t + 1 < a->nsteps) return a->ck[(size_t)((t + 1) / a->K)];
-    return a->pp[t & 1];
+// n collisions from src, several per pass where the lattice suits it; `first`:
+// the first one collides the canonical state in place, the others follow a
+// stream.  Intermediate fields alternate between pp[0] and pp[1]; the last one
+// goes to dst or, when that is null, to the next of the two.  *result: where.
+int adj_advance(lbm_adjoint a, const MultiPlan &plan, const void *src, int64_t n, bool first,
+                void *dst, const void **result) {
+    const void *cur = src;
+    while (n > 0) {
+        const int k = plan.kernel != lbm::kMultiNone ? multi_next(plan, n) : 1;
+        n -= k;
+        void *to = n == 0 && dst ? dst : (cur == a->pp[0] ? a->pp[1] : a->pp[0]);
+        int rc;
+        if (k > 1) {
+            lbm_field_s fs = a->geo, fd = a->geo;
+            fs.d = const_cast<void *>(cur);
+            fd.d = to;
+            rc = run_multi(plan, a->m, &fs, &fd, k, first);
+        } else {
+            rc = adj_forward_op(a, first ? lbm::Op::Collide : lbm::Op::Fused, cur, to);
+        }
+        if (rc) return rc;
+        cur = to;
+        first = false;
+    }
+    if (result) *result = cur;
+    return 0;
+}
+
+// The fields C_j .. of n collisions from src, each kept: out[0 .. n-1]
+int adj_advance_all(lbm_adjoint a, const MultiPlan &plan, const void *src, int64_t n, bool first,
+                    void *const *out) {
+    MultiPlan pl = plan;
+    if (pl.kernel == lbm::kMultiMarch) {  // waves keep their levels' rows: blocks instead
+        pl.kernel = lbm::kMultiBlockWide;
+        for (int k = 1; k <= pl.max_steps; ++k) pl.cost[k] = 2.0 + k;
+    }
+    const lbm::StepParams<double> p = make_params(a->m, &a->geo, false);
+    while (n > 0) {
+        const int k = pl.kernel != lbm::kMultiNone ? multi_next(pl, n) : 1;
+        int rc;
+        if (k > 1) {
+            lbm::MultiLaunch L{};
+            L.kernel = pl.kernel;
+            L.qid = a->geo.qid;
+            L.coll = a->m->coll;
+            L.steps = k;
+            L.first = first ? 1 : 0;
+            L.src = src;
+            lbm::LevelOut o{};
+            for (int l = 0; l < k; ++l) o.out[l] = out[l];
+            rc = a->geo.storage == LBM_STORE_F64
+                     ? lbm::run_multi_all_f64(L, o, p, g_stream)
+                     : lbm::run_multi_all_f32(L, o, lbm::to_float_params(p), g_stream);
+            if (rc) return fail(-4, "kernel launch failed (code %d): %s", rc,
+                                hipGetErrorString(hipGetLastError()));
+        } else {
+            rc = adj_forward_op(a, first ? lbm::Op::Collide : lbm::Op::Fused, src, out[0]);
+            if (rc) return rc;
+        }
+        src = out[k - 1];
+        out += k;
+        n -= k;
+        first = false;
+    }
+    return 0;
 }
 
 // S_0 from u0, the forward pass with checkpoints, lambda_T and the loss
@@ -2344,17 +2405,20 @@ int adjoint_forward(lbm_adjoint a, const double *u0, const double *ut, bool want
     L.pops = a->S0;
     L.u = a->du0;
     if (int rc = adj_launch(a, p, L)) return rc;
+    // segment by segment to the checkpoints C_{K-1}, C_{2K-1}, .. and to C_{T-1}
     const int64_t T = a->nsteps;
-    if (T > 0) {
-        if (int rc = adj_forward_op(a, lbm::Op::Collide, a->S0, adj_cbuf(a, 0))) return rc;
-        for (int64_t t = 1; t < T; ++t)
-            if (int rc = adj_forward_op(a, lbm::Op::Fused, adj_cbuf(a, t - 1), adj_cbuf(a, t)))
-                return rc;
+    const MultiPlan plan = multi_plan(a->m, &a->geo);
+    const void *last = a->S0;
+    for (int s = 0; s < a->nseg; ++s) {
+        const int64_t n = std::min<int64_t>(a->K, T - (int64_t)s * a->K);
+        if (int rc = adj_advance(a, plan, last, n, s == 0, s + 1 < a->nseg ? a->ck[s + 1] : nullptr,
+                                 &last))
+            return rc;
     }
     L = lbm::AdjLaunch{};
     L.what = 1;
     L.direct = T == 0 ? 1 : 0;
-    L.state = T == 0 ? a->S0 : adj_cbuf(a, T - 1);
+    L.state = last;
     L.u = a->dut;
     L.lam_out = a->lam[0];
     L.out = a->dlossn;
@@ -2487,33 +2551,34 @@ int lbm_adjoint_gradient(lbm_adjoint a, const double *u0, const double *u_target
     const lbm::StepParams<double> p = make_params(a->m, &a->geo, false);
     const long long plane = (long long)a->geo.nx * a->geo.ny;
     HIP_TRY(hipMemsetAsync(a->dgtau, 0, (size_t)plane * 2 * sizeof(double), g_stream));
+    const MultiPlan plan = multi_plan(a->m, &a->geo);
+    const bool tiled = a->geo.qid == 4 || a->geo.qid == 5 || a->geo.qid == 9;
     int cur = 0;  // lam[cur] holds lambda_{t+1}
     for (int s = a->nseg - 1; s >= 0; --s) {
         const int64_t t0 = (int64_t)s * a->K;
         const int64_t t1 = t0 + a->K < a->nsteps ? t0 + a->K : a->nsteps;
         // recompute C_{t0} .. C_{t1-2}
-        for (int64_t j = 0; t0 + j <= t1 - 2; ++j) {
-            int rc;
-            if (j > 0) rc = adj_forward_op(a, lbm::Op::Fused, a->seg[j - 1], a->seg[j]);
-            else if (s == 0) rc = adj_forward_op(a, lbm::Op::Collide, a->S0, a->seg[0]);
-            else rc = adj_forward_op(a, lbm::Op::Fused, a->ck[s], a->seg[0]);
-            if (rc) return rc;
-        }
-        for (int64_t t = t1 - 1; t >= t0; --t) {
+        if (int rc = adj_advance_all(a, plan, s == 0 ? a->S0 : a->ck[s], t1 - 1 - t0, s == 0,
+                                     a->seg.data()))
+            return rc;
+        for (int64_t t = t1 - 1; t >= t0;) {
+            // steps t, t - 1, .. t - n + 1 of one launch, in equal shares
+            const int64_t left = t - t0 + 1;
+            const int shares = tiled ? (int)((left + lbm::kAdjLevels - 1) / lbm::kAdjLevels) : 1;
+            const int n = tiled ? (int)((left + shares - 1) / shares) : 1;
             lbm::AdjLaunch L{};
-            L.what = 2;
-            if (t == t0) {
-                L.direct = s == 0 ? 1 : 0;
-                L.state = s == 0 ? a->S0 : a->ck[s];
-            } else {
-                L.direct = 0;
-                L.state = a->seg[t - 1 - t0];
-            }
+            for (int l = 0; l < n; ++l)
+                L.states[l] = t - l > t0 ? a->seg[t - l - 1 - t0] : (s == 0 ? a->S0 : a->ck[s]);
+            L.what = n > 1 ? 4 : 2;
+            L.levels = n;
+            L.state = L.states[0];
+            L.direct = s == 0 && t - n + 1 == 0 ? 1 : 0;
             L.lam_in = a->lam[cur];
             L.lam_out = a->lam[cur ^ 1];
             L.out = a->dgtau;
             if (int rc = adj_launch(a, p, L)) return rc;
             cur ^= 1;
+            t -= n;
         }
     }
     lbm::AdjLaunch L{};

@@ -145,6 +145,24 @@ enum MultiKernel : int {
     kMultiMarch,      // marching waves: 2-5 steps (FP64), 2-4 or 6 (FP32), 2-4 (16-bit)
     kMultiNone
 };
+// A register block is 64 columns x `rows` rows and computes a halo of steps - 1
+// nodes on each side: the nodes it writes, as equal shares of the lattice (the
+// width in whole 64-byte groups where that does not add a column of blocks).
+struct BlockShape {
+    int outx, outy, across, down;
+};
+inline BlockShape block_shape(int nx, int ny, int steps, int rows, int elem_bytes) {
+    const int ox = 64 - 2 * (steps - 1), oy = rows - 2 * (steps - 1), group = 64 / elem_bytes;
+    const int nbx = (nx + ox - 1) / ox, nby = (ny + oy - 1) / oy;
+    BlockShape b;
+    b.outx = (nx + nbx - 1) / nbx;
+    const int rounded = (b.outx + group - 1) / group * group;
+    if (rounded <= ox) b.outx = rounded;
+    b.outy = (ny + nby - 1) / nby;
+    b.across = (nx + b.outx - 1) / b.outx;
+    b.down = (ny + b.outy - 1) / b.outy;
+    return b;
+}
 constexpr int kMarchRows = 16;  // fewest rows of a marching wave
 // Stop of the iterative initialization, kept on the device: the density of
 // node (nx, ny) after the last step and the first step that converged (0: none)
@@ -170,8 +188,10 @@ struct MultiLaunch {
 };
 
 // Reverse-mode kernels of the periodic SRT/TRT step (lbm_adjoint.h).
+constexpr int kAdjLevels = 4;  // most reverse steps of one launch
 struct AdjLaunch {
-    int what;            // 0 S0 = feq(rho0, u0), 1 seed lambda_T + loss, 2 reverse step, 3 dL/du0
+    int what;            // 0 S0 = feq(rho0, u0), 1 seed lambda_T + loss, 2 reverse step, 3 dL/du0,
+                         // 4 several reverse steps (one-speed stencils)
     int qid, coll;       // coll 0 SRT, 1 TRT
     int direct;          // state stored directly (1) or pulled from a post-collision field (0)
     const void *state;   // populations read by the seed / reverse step
@@ -181,6 +201,8 @@ struct AdjLaunch {
     const double *u;     // u0 (init, dL/du0) or u_target (seed), (nx, ny, 2) column-major
     double *out;         // per-node loss (seed), dL/dtau accumulators (step), dL/du0
     double *aux;         // seed: u(S_T), (nx, ny, 2) column-major, or nullptr
+    int levels;                      // several reverse steps: their number and states,
+    const void *states[kAdjLevels];  // latest step first
 };
 int run_adjoint_f64(const AdjLaunch &L, const StepParams<double> &p, hipStream_t s);
 int run_adjoint_f32(const AdjLaunch &L, const StepParams<float> &p, hipStream_t s);
@@ -216,6 +238,15 @@ LBM_DECLARE_MULTI(f64, double)
 LBM_DECLARE_MULTI(f32, float)
 LBM_DECLARE_MULTI(f16neq, float)
 LBM_DECLARE_MULTI(bf16neq, float)
+// several fused steps of a periodic SRT/TRT model that store every step's field
+// (out[l]: collision l of the pass); tile and block kernels
+struct LevelOut {
+    void *out[8];
+};
+int run_multi_all_f64(const MultiLaunch &L, const LevelOut &o, const StepParams<double> &p,
+                      hipStream_t s);
+int run_multi_all_f32(const MultiLaunch &L, const LevelOut &o, const StepParams<float> &p,
+                      hipStream_t s);
 // steps of the iterative initialization, C_(t-1) -> C_t: one (every stencil),
 // or several on tiles (one-speed stencils)
 int run_mei_step(int qid, const double *src, double *dst, const StepParams<double> &p,

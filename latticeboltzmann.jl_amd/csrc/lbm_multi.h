@@ -319,6 +319,24 @@ __device__ __forceinline__ void bc_apply(const StepParams<T> &p, int moving, uns
 }
 
 // ---------------------------------------------------------------------------
+// Tiles and blocks are dealt to the 8 XCDs (workgroups go to them in turn) in
+// contiguous chunks: neighbours, which read each other's halo, share an L2.
+// D2Q9 TRT, us a step dealt in turn / in chunks, FP64 and FP32: tiles 160^2
+// 1.92 / 1.66, 1.10 / 0.95; 64 x 16 blocks 257^2 2.55 / 1.99, 1.54 / 1.17;
+// 64 x 32 blocks 512^2 4.01 / 3.61, 2.29 / 1.88; the wide ones 1021 x 517
+// 7.50 / 7.11, 3.73 / 3.20.
+template <class A>
+__device__ __forceinline__ int tile_of_block(const A &a) {
+    return (int)(blockIdx.x & 7) * a.chunk + (int)(blockIdx.x >> 3);
+}
+template <class A>
+unsigned deal_tiles(A &a, int tiles_y) {
+    a.tiles = a.tiles_x * tiles_y;
+    a.chunk = (a.tiles + 7) / 8;
+    return 8u * (unsigned)a.chunk;
+}
+
+// ---------------------------------------------------------------------------
 // k_tile
 // ---------------------------------------------------------------------------
 // A block advances a TX x TY tile by `levels` <= TMAX steps.  Level l pulls
@@ -330,7 +348,7 @@ __device__ __forceinline__ void bc_apply(const StepParams<T> &p, int moving, uns
 // 1 collides the canonical state S_0 of its own node instead of pulling.
 struct TileArgs {
     int levels;
-    int tiles_x;
+    int tiles_x, tiles, chunk;
     int first;
     WallArgs wall;
     MeiStop mei;  // COLL == 3: the iterative initialization's stop
@@ -343,10 +361,11 @@ struct TileShape {
     static constexpr int K = (N + NT - 1) / NT;  // nodes per thread
 };
 
-template <int QID, int COLL, class ST, int TX, int TY, int TMAX, int NT, bool BC>
-__global__ void __launch_bounds__(NT)
-k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
-       const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc, const TileArgs a) {
+template <int QID, int COLL, class ST, int TX, int TY, int TMAX, int NT, bool BC, bool ALL>
+__device__ __forceinline__ void
+tile_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
+            const StepParams<typename ST::T> &p, const MultiConsts<typename ST::T> &mc,
+            const TileArgs &a, const LevelOut *all) {
     using T = typename ST::T;
     using S = typename ST::store_t;
     using SH = TileShape<QID, ST, TX, TY, TMAX, NT>;
@@ -355,7 +374,9 @@ k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restr
     __shared__ T buf[Q * N];
     if constexpr (COLL == 3)
         if (a.mei.watch && mei_stopped(a.mei.watch) != 0) return;
-    const int ty = blockIdx.x / a.tiles_x, tx = blockIdx.x - ty * a.tiles_x;
+    const int tile = tile_of_block(a);
+    if (tile >= a.tiles) return;
+    const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;
     int at[K], xs[K], ys[K], ring[K];
     unsigned bcm[K];
     bool mine[K];
@@ -404,6 +425,14 @@ k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restr
             collide_multi<QID, COLL, T>(f[k], p, mc, xs[k], ys[k]);
         }
     };
+    auto store = [&](S *dst, int k) {
+        if (!mine[k]) return;
+        auto st = [&](auto Ic) {
+            constexpr int i = decltype(Ic)::value;
+            dst[p.plane * i + ((long long)xs[k] + (long long)p.nx * ys[k])] = ST::encode(f[k][i], i, p);
+        };
+        adj_each_node<QID>(st);
+    };
     // level 1 from HBM
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -435,6 +464,7 @@ k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restr
                 });
         }
         collide(k, 1);
+        if constexpr (ALL) store(static_cast<S *>(all->out[0]), k);
     }
     for (int l = 2; l <= L; ++l) {
 #pragma unroll
@@ -465,17 +495,29 @@ k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restr
         for (int k = 0; k < K; ++k) {
             if (ring[k] > L - l) continue;
             collide(k, l);
+            if constexpr (ALL) store(static_cast<S *>(all->out[l - 1]), k);
         }
     }
+    if constexpr (!ALL) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        if (!mine[k]) continue;
-        auto st = [&](auto Ic) {
-            constexpr int i = decltype(Ic)::value;
-            Cn[p.plane * i + ((long long)xs[k] + (long long)p.nx * ys[k])] = ST::encode(f[k][i], i, p);
-        };
-        adj_each_node<QID>(st);
+        for (int k = 0; k < K; ++k) store(Cn, k);
     }
+}
+
+template <int QID, int COLL, class ST, int TX, int TY, int TMAX, int NT, bool BC>
+__global__ void __launch_bounds__(NT)
+k_tile(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
+       const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc, const TileArgs a) {
+    tile_region<QID, COLL, ST, TX, TY, TMAX, NT, BC, false>(C, Cn, p, mc, a, nullptr);
+}
+
+// every level's field kept (k_block_all)
+template <int QID, int COLL, class ST, int TX, int TY, int TMAX, int NT>
+__global__ void __launch_bounds__(NT)
+k_tile_all(const typename ST::store_t *__restrict__ C, const LevelOut o,
+           const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc,
+           const TileArgs a) {
+    tile_region<QID, COLL, ST, TX, TY, TMAX, NT, false, true>(C, nullptr, p, mc, a, &o);
 }
 
 // x-shift inside a wave: the value of the lane below (D = +1) or above (-1)
@@ -505,7 +547,8 @@ __device__ __forceinline__ double lane_shift(double v) {
 // 64 - 2 (T - 1) columns and NW R - 2 (T - 1) rows.
 struct BlockArgs {
     int levels;
-    int tiles_x, outx, outy;  // nodes written per block
+    int tiles_x, tiles, chunk;
+    int outx, outy;  // nodes written per block
     int first;
     WallArgs wall;
 };
@@ -523,12 +566,12 @@ using BlockEdges = V[2][NW][edge_slot<QID>(QT<QID>::Q)][66];
 
 // One block's region: writes the outx x outy nodes from (cx0, cy0) of a lattice
 // of p.nx x p.ny nodes with rows `pitch` apart.
-template <int QID, int COLL, class ST, int NW, int R, bool BC>
+template <int QID, int COLL, class ST, int NW, int R, bool BC, bool ALL = false>
 __device__ __forceinline__ void
 block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *__restrict__ Cn,
              const StepParams<typename ST::T> &p, const MultiConsts<typename ST::T> &mc, int pitch,
              int cx0, int cy0, int outx, int outy, int L, int first, WallArgs wall,
-             BlockEdges<QID, typename ST::T, NW> &xch) {
+             BlockEdges<QID, typename ST::T, NW> &xch, const LevelOut *all = nullptr) {
     using V = typename ST::T;
     using S = typename ST::store_t;
     constexpr int Q = QT<QID>::Q;
@@ -552,6 +595,19 @@ block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *_
 #pragma unroll
     for (int j = 0; j < R; ++j) bcm[j] = BC ? bc_mask<QID>(p, wall.walls, x, ys[j]) : 0u;
     V g[R][Q];
+    const bool mine_x = ux >= cx0 && ux < min(cx0 + outx, p.nx);
+    // row j of a level to `dst`, where this block owns it
+    auto store = [&](S *dst, int j, const V(&f)[Q]) {
+        const int uy = cy0 - h + row0 + j;
+        if (mine_x && uy >= cy0 && uy < min(cy0 + outy, p.ny)) {
+            S *base = dst + (long long)pitch * uy;
+            auto st = [&](auto Ic) {
+                constexpr int i = decltype(Ic)::value;
+                *at_b(base + p.plane * i, off) = ST::encode(f[i], i, p);
+            };
+            adj_each_node<QID>(st);
+        }
+    };
     // level 1
     S pre[R][Q];
 #pragma unroll
@@ -582,6 +638,7 @@ block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *_
                 });
         }
         collide_multi<QID, COLL, V>(g[j], p, mc, x, y);
+        if constexpr (ALL) store(static_cast<S *>(all->out[0]), j, g[j]);
     }
     for (int l = 2; l <= L; ++l) {
         V(*X)[ES][66] = xch[l & 1];
@@ -631,21 +688,12 @@ block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *_
                 g[j][i] = f[i];
             };
             adj_each_node<QID>(cp);
+            if constexpr (ALL) store(static_cast<S *>(all->out[l - 1]), j, g[j]);
         }
     }
-    if (ux >= cx0 && ux < min(cx0 + outx, p.nx)) {
+    if constexpr (!ALL) {
 #pragma unroll
-        for (int j = 0; j < R; ++j) {
-            const int uy = cy0 - h + row0 + j;
-            if (uy >= cy0 && uy < min(cy0 + outy, p.ny)) {
-                S *base = Cn + (long long)pitch * uy;
-                auto st = [&](auto Ic) {
-                    constexpr int i = decltype(Ic)::value;
-                    *at_b(base + p.plane * i, off) = ST::encode(g[j][i], i, p);
-                };
-                adj_each_node<QID>(st);
-            }
-        }
+        for (int j = 0; j < R; ++j) store(Cn, j, g[j]);
     }
 }
 
@@ -655,9 +703,28 @@ k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
         const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc,
         const BlockArgs a) {
     __shared__ BlockEdges<QID, typename ST::T, NW> xch;
-    const int ty = blockIdx.x / a.tiles_x, tx = blockIdx.x - ty * a.tiles_x;
+    const int tile = tile_of_block(a);
+    if (tile >= a.tiles) return;
+    const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;
     block_region<QID, COLL, ST, NW, R, BC>(C, Cn, p, mc, p.nx, tx * a.outx, ty * a.outy, a.outx,
                                            a.outy, a.levels, a.first, a.wall, xch);
+}
+
+// Every level's field kept (the reverse pass needs each step's state): a pass
+// reads the lattice once and writes it once per step, where single steps read
+// it at each.
+template <int QID, int COLL, class ST, int NW, int R>
+__global__ void __launch_bounds__(64 * NW)
+k_block_all(const typename ST::store_t *__restrict__ C, const LevelOut o,
+            const StepParams<typename ST::T> p, const MultiConsts<typename ST::T> mc,
+            const BlockArgs a) {
+    __shared__ BlockEdges<QID, typename ST::T, NW> xch;
+    const int tile = tile_of_block(a);
+    if (tile >= a.tiles) return;
+    const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;
+    block_region<QID, COLL, ST, NW, R, false, true>(C, nullptr, p, mc, p.nx, tx * a.outx,
+                                                    ty * a.outy, a.outx, a.outy, a.levels, a.first,
+                                                    a.wall, xch, &o);
 }
 
 // Batched lattices: one region per block from a table; the lattice record is
@@ -668,11 +735,14 @@ k_block(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
 template <int QID, int COLL, class ST, int NW, int R>
 __global__ void __launch_bounds__(64 * NW)
 k_batch_block(const BatchLattice *__restrict__ lats, const BatchRegion *__restrict__ regions,
-              typename ST::store_t *__restrict__ pool, int parity, int levels, int first,
-              const StepParams<typename ST::T> base, const MultiConsts<typename ST::T> base_mc) {
+              int nregions, int chunk, typename ST::store_t *__restrict__ pool, int parity,
+              int levels, int first, const StepParams<typename ST::T> base,
+              const MultiConsts<typename ST::T> base_mc) {
     using T = typename ST::T;
     __shared__ BlockEdges<QID, T, NW> xch;
-    const BatchRegion g = regions[blockIdx.x];
+    const int r = (int)(blockIdx.x & 7) * chunk + (int)(blockIdx.x >> 3);  // as tile_of_block
+    if (r >= nregions) return;
+    const BatchRegion g = regions[r];
     const BatchLattice &lat = lats[__builtin_amdgcn_readfirstlane(g.lat)];
     StepParams<T> p = base;
     p.nx = lat.nx;
@@ -956,46 +1026,94 @@ k_march(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
 // ---------------------------------------------------------------------------
 constexpr int kTileX = 8, kTileY = 8, kTileT = 8, kTileThreads = 512;
 
-template <int QID, int COLL, class ST, bool BC>
-int launch_tile(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
-    using S = typename ST::store_t;
-    if (L.steps < 1 || L.steps > kTileT) return -5;
+template <class T>
+TileArgs tile_args(const MultiLaunch &L, const StepParams<T> &p, unsigned &blocks) {
     TileArgs a;
     a.levels = L.steps;
     a.first = L.first;
     a.wall = WallArgs{L.walls, L.moving};
     a.mei = L.mei;
     a.tiles_x = (p.nx + kTileX - 1) / kTileX;
-    const int tiles_y = (p.ny + kTileY - 1) / kTileY;
-    k_tile<QID, COLL, ST, kTileX, kTileY, kTileT, kTileThreads, BC>
-        <<<(unsigned)a.tiles_x * (unsigned)tiles_y, kTileThreads, 0, s>>>(
-            static_cast<const S *>(L.src), static_cast<S *>(L.dst), p, multi_consts(p), a);
+    blocks = deal_tiles(a, (p.ny + kTileY - 1) / kTileY);
+    return a;
+}
+
+template <int QID, int COLL, class ST, bool BC>
+int launch_tile(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
+    using S = typename ST::store_t;
+    if (L.steps < 1 || L.steps > kTileT) return -5;
+    unsigned blocks;
+    const TileArgs a = tile_args(L, p, blocks);
+    k_tile<QID, COLL, ST, kTileX, kTileY, kTileT, kTileThreads, BC><<<blocks, kTileThreads, 0, s>>>(
+        static_cast<const S *>(L.src), static_cast<S *>(L.dst), p, multi_consts(p), a);
     return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+template <class S, int ROWS, class T>
+BlockArgs block_args(const MultiLaunch &L, const StepParams<T> &p, unsigned &blocks) {
+    BlockArgs a;
+    a.levels = L.steps;
+    a.first = L.first;
+    a.wall = WallArgs{L.walls, L.moving};
+    const BlockShape b = block_shape(p.nx, p.ny, L.steps, ROWS, (int)sizeof(S));
+    a.outx = b.outx;
+    a.outy = b.outy;
+    a.tiles_x = b.across;
+    blocks = deal_tiles(a, b.down);
+    return a;
+}
+// the output of a block is at least two rows and two columns
+constexpr bool block_fits(int steps, int rows) {
+    return steps >= 1 && 2 * (steps - 1) < 64 && 2 * (steps - 1) < rows;
 }
 
 template <int QID, int COLL, class ST, int NW, int R, bool BC>
 int launch_block(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
     using S = typename ST::store_t;
-    const int halo = 2 * (L.steps - 1);
-    if (L.steps < 1 || halo >= 64 || halo >= NW * R) return -5;
-    BlockArgs a;
-    a.levels = L.steps;
-    a.first = L.first;
-    a.wall = WallArgs{L.walls, L.moving};
-    // the lattice in equal shares, the width in whole 64-byte groups where
-    // that does not add a column of tiles
-    const int ox = 64 - halo, oy = NW * R - halo, group = 64 / (int)sizeof(S);
-    const int nbx = (p.nx + ox - 1) / ox, nby = (p.ny + oy - 1) / oy;
-    a.outx = (p.nx + nbx - 1) / nbx;
-    const int rounded = (a.outx + group - 1) / group * group;
-    if (rounded <= ox) a.outx = rounded;
-    a.outy = (p.ny + nby - 1) / nby;
-    a.tiles_x = (p.nx + a.outx - 1) / a.outx;
-    const int tiles_y = (p.ny + a.outy - 1) / a.outy;
-    k_block<QID, COLL, ST, NW, R, BC><<<(unsigned)a.tiles_x * (unsigned)tiles_y, 64 * NW, 0, s>>>(
+    if (!block_fits(L.steps, NW * R)) return -5;
+    unsigned blocks;
+    const BlockArgs a = block_args<S, NW * R>(L, p, blocks);
+    k_block<QID, COLL, ST, NW, R, BC><<<blocks, 64 * NW, 0, s>>>(
         static_cast<const S *>(L.src), static_cast<S *>(L.dst), p, multi_consts(p), a);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
+
+// every step's field kept, periodic SRT/TRT lattices
+template <int QID, int COLL, class ST, int NW, int R>
+int launch_block_all(const MultiLaunch &L, const LevelOut &o, const StepParams<typename ST::T> &p,
+                     hipStream_t s) {
+    using S = typename ST::store_t;
+    if (!block_fits(L.steps, NW * R) || L.steps > 8) return -5;
+    unsigned blocks;
+    const BlockArgs a = block_args<S, NW * R>(L, p, blocks);
+    k_block_all<QID, COLL, ST, NW, R><<<blocks, 64 * NW, 0, s>>>(
+        static_cast<const S *>(L.src), o, p, multi_consts(p), a);
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+template <int QID, int COLL, class ST>
+int launch_all(const MultiLaunch &L, const LevelOut &o, const StepParams<typename ST::T> &p,
+               hipStream_t s) {
+    using S = typename ST::store_t;
+    constexpr bool f64 = sizeof(S) == 8;
+    switch (L.kernel) {
+    case kMultiTile: {
+        if (L.steps < 1 || L.steps > kTileT) return -5;
+        unsigned blocks;
+        const TileArgs a = tile_args(L, p, blocks);
+        k_tile_all<QID, COLL, ST, kTileX, kTileY, kTileT, kTileThreads>
+            <<<blocks, kTileThreads, 0, s>>>(static_cast<const S *>(L.src), o, p, multi_consts(p), a);
+        return hipGetLastError() == hipSuccess ? 0 : -4;
+    }
+    case kMultiBlock16: return launch_block_all<QID, COLL, ST, 16, 1>(L, o, p, s);
+    case kMultiBlock32: return launch_block_all<QID, COLL, ST, 16, 2>(L, o, p, s);
+    case kMultiBlockWide: return launch_block_all<QID, COLL, ST, 8, f64 ? 3 : 4>(L, o, p, s);
+    default: return -5;
+    }
+}
+
+#define LBM_DEFINE_MULTI_ALL(TAG, ST)                                                             int run_multi_all_##TAG(const MultiLaunch &L, const LevelOut &o,                                                      const StepParams<typename ST::T> &p, hipStream_t s) {                     switch (L.qid * 2 + L.coll) {                                                                 case 8: return launch_all<4, 0, ST>(L, o, p, s);                                              case 9: return launch_all<4, 1, ST>(L, o, p, s);                                              case 10: return launch_all<5, 0, ST>(L, o, p, s);                                             case 11: return launch_all<5, 1, ST>(L, o, p, s);                                             case 18: return launch_all<9, 0, ST>(L, o, p, s);                                             case 19: return launch_all<9, 1, ST>(L, o, p, s);                                             default: return -1;                                                                           }                                                                                         }
+
 
 template <int QID, int COLL, class ST, int T, int NC, bool BC>
 int launch_march(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
@@ -1091,12 +1209,14 @@ int launch_batch_block(int coll, const BatchLattice *lats, const BatchRegion *re
     constexpr int tmax = sizeof(S) == 8 ? kBatchStepsF64 : kBatchStepsF32;
     if (levels < 1 || levels > tmax || nregions < 1) return -5;
     S *pl = static_cast<S *>(pool);
+    const int chunk = (nregions + 7) / 8;
+    const unsigned blocks = 8u * (unsigned)chunk;
     if (coll == 0)
-        k_batch_block<QID, 0, ST, NW, R><<<(unsigned)nregions, 64 * NW, 0, s>>>(
-            lats, regions, pl, parity, levels, first, p, multi_consts(p));
+        k_batch_block<QID, 0, ST, NW, R><<<blocks, 64 * NW, 0, s>>>(
+            lats, regions, nregions, chunk, pl, parity, levels, first, p, multi_consts(p));
     else
-        k_batch_block<QID, 1, ST, NW, R><<<(unsigned)nregions, 64 * NW, 0, s>>>(
-            lats, regions, pl, parity, levels, first, p, multi_consts(p));
+        k_batch_block<QID, 1, ST, NW, R><<<blocks, 64 * NW, 0, s>>>(
+            lats, regions, nregions, chunk, pl, parity, levels, first, p, multi_consts(p));
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

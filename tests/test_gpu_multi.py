@@ -240,3 +240,43 @@ def test_mei_initialize_bit_exact(oracle_lib, qid, nx, ny, bcname, eps, max_step
     assert steps == n
     assert np.array_equal(s, S)
     assert np.array_equal(c, C)
+
+
+# the reverse pass: 16 x 16 tiles of up to four steps, forward and recomputed
+# segments by every several-step kernel and, at 31 x 2501, single steps
+ADJOINT = [(1, 1), (2, 3), (16, 16), (17, 33), (130, 47), (257, 160), (340, 340), (513, 300),
+           (700, 650), (31, 2501), (2049, 1500)]
+
+
+def _adjoint(qid, coll, shape, T, K, storage, u0, ut):
+    L = _L()
+    cm = L.SRT(0.8) if coll == 0 else L.TRT.fields(0.75, 1.2)
+    prob = L.AdjointProblem(L.Quadratures[f"D2Q{qid}"](), cm, shape, T, storage=storage,
+                            checkpoint_every=K)
+    r = prob.gradient(u0, ut)
+    prob.close()
+    return r
+
+
+@pytest.mark.parametrize("qid,shape", [(9, s) for s in ADJOINT] +
+                         [(4, (130, 47)), (5, (130, 47)), (5, (257, 160))])
+@pytest.mark.parametrize("coll", [0, 1])
+@pytest.mark.parametrize("T", [2, 11, 13])
+def test_adjoint_passes(qid, shape, coll, T):
+    """FP64: single steps (a checkpoint at each step) and passes give the same
+    bits.  FP32 against FP64: a step rounds each of its terms a few times, 64
+    half-ulps in the summed norm with the forward run's share, so after T
+    steps the relative difference is below 64 (T + 1) 2^-24."""
+    rng = np.random.default_rng(T)
+    u0, ut = (0.03 * rng.standard_normal((*shape, 2)) for _ in (0, 1))
+    print(f"adjoint D2Q{qid} {shape} coll {coll} T {T}", flush=True)
+    ref = _adjoint(qid, coll, shape, T, 1, "f64", u0, ut)
+    for K in (0, 3, T):
+        r = _adjoint(qid, coll, shape, T, K, "f64", u0, ut)
+        assert r["loss"] == ref["loss"], K
+        assert np.array_equal(r["grad_u0"], ref["grad_u0"]), K
+        assert np.array_equal(r["grad_tau"], ref["grad_tau"]), K
+    r = _adjoint(qid, coll, shape, T, T, "f32", u0, ut)
+    tol = 64 * (T + 1) * 2.0 ** -24
+    assert np.linalg.norm(r["grad_u0"] - ref["grad_u0"]) <= tol * np.linalg.norm(ref["grad_u0"])
+    assert abs(r["loss"] - ref["loss"]) <= tol * ref["loss"]
