@@ -4,5 +4,8 @@
 #include "lbm_multi.h"
 
 namespace lbm {
-LBM_DEFINE_MULTI_ALL(f64, StF64)
+int run_multi_all_f64(const MultiLaunch &L, const LevelOut &o, const StepParams<double> &p,
+                      hipStream_t s) {
+    return launch_all_any<StF64>(L, o, p, s);
+}
 }  // namespace lbm

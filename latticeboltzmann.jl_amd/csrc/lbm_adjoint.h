@@ -226,13 +226,14 @@ __device__ __forceinline__ void adj_node_sum(const typename ST::T (&f)[QT<QID>::
     });
 }
 
+// FP32 keeps the plain sums: its dL/dtau moves less with their rounding unchanged
 template <int QID, class ST, int COLL>
 __device__ __forceinline__ void adj_node(const typename ST::T (&f)[QT<QID>::Q],
                                          const typename ST::T (&mu)[QT<QID>::Q],
                                          const StepParams<typename ST::T> &p,
                                          typename ST::T (&lam)[QT<QID>::Q], typename ST::T &gs,
                                          typename ST::T &ga) {
-    if constexpr (QT<QID>::FEQ <= 2) adj_node_pairs<QID, ST, COLL>(f, mu, p, lam, gs, ga);
+    if constexpr (QT<QID>::FEQ <= 2 && !ST::kShift) adj_node_pairs<QID, ST, COLL>(f, mu, p, lam, gs, ga);
     else adj_node_sum<QID, ST, COLL>(f, mu, p, lam, gs, ga);
 }
 
@@ -283,8 +284,8 @@ k_adj_step(const typename ST::T *__restrict__ lam_next, const typename ST::store
 // from its post-collision field (loaded before the block meets, so that it
 // arrives behind the exchange).  A single step reads lambda and the state and
 // writes lambda, 27 populations a node; here lambda moves once per launch.
-// Same operations in the same order per node and step: the bits of single
-// steps.
+// Same operations in the same order per node and step: in FP64 the bits of
+// single steps (FP32: another contraction of products and sums).
 // Bound by the pulls of the state: a tile's 22 columns touch three 128-byte
 // lines a row, so neighbouring tiles share most lines and run on one XCD, with
 // one L2 (consecutive workgroups go to the 8 XCDs in turn; the tiles are dealt
@@ -503,7 +504,8 @@ int launch_adjoint(const AdjLaunch &L, const StepParams<typename ST::T> &p, hipS
             a.chunk = (a.tiles + 7) / 8;
             const unsigned tiles = 8u * (unsigned)a.chunk;
             if (L.coll == 0) k_adj_tile<QID, ST, 0><<<tiles, kAdjThreads, 0, s>>>(li, lo, L.out, p, a);
-            else if (L.coll == 1) k_adj_tile<QID, ST, 1><<<tiles, kAdjThreads, 0, s>>>(li, lo, L.out, p, a);
+            else if constexpr (!ST::kShift)
+                k_adj_tile<QID, ST, 1><<<tiles, kAdjThreads, 0, s>>>(li, lo, L.out, p, a);
             else return -2;
             break;
         } else {

@@ -529,6 +529,46 @@ struct MultiPlan {
 // (below this the 16-bit storages keep the single-step row kernel)
 constexpr long long kNeqMarchNodes = 800000;
 
+// The register-block kernels: a pass takes a + b per further round of 256
+// blocks (one per CU), by its steps; microseconds, D2Q9 TRT, measured on 100^2
+// .. 1400^2 and 2000 x 150.  The first round's slope within it is small, so a
+// lattice wants the kernel and the steps that just fill a whole number of
+// rounds: 300^2 FP64 has 300 blocks of 64 x 16 at 6 steps (3.5 us a step) and
+// 228 at 5 (2.25); 560^2 273 of 64 x 32 at 6 (6.8) and 252 at 5 (4.3).
+struct BlockCost {
+    int kernel, rows, tmax;
+    double a[9], b[9];
+};
+const BlockCost kBlockCost64[3] = {
+    {lbm::kMultiBlock16, 16, 6, {0, 0, 7.8, 8.8, 9.9, 11.2, 12.5}, {0, 0, 6, 7, 7, 8.5, 10}},
+    {lbm::kMultiBlock32, 32, 8, {0, 0, 12, 15, 18, 21.2, 23.5, 25.5, 27},
+     {0, 0, 13, 15, 16.5, 18, 20.5, 22.5, 25.5}},
+    {lbm::kMultiBlockWide, 24, 7, {0, 0, 12, 13.5, 15, 17, 19, 21},
+     {0, 0, 7.5, 8.2, 9, 10.5, 12.2, 13.8}}};
+const BlockCost kBlockCost32[3] = {
+    {lbm::kMultiBlock16, 16, 6, {0, 0, 5.1, 5.6, 6.1, 6.7, 7.1}, {0, 0, 2.4, 2.6, 2.9, 3.1, 3.4}},
+    {lbm::kMultiBlock32, 32, 8, {0, 0, 7.6, 8.5, 9.4, 10.4, 11.3, 12.3, 13},
+     {0, 0, 4.6, 5.3, 6.2, 7.4, 8.2, 9.3, 10.1}},
+    {lbm::kMultiBlockWide, 32, 7, {0, 0, 9, 10, 11, 12.2, 13.2, 14.2},
+     {0, 0, 4.7, 5, 5.4, 6.1, 6.7, 7.4}}};
+
+// the costs of a block kernel's passes on a lattice; max_steps the best per step
+void plan_blocks(MultiPlan &pl, const BlockCost &c, const lbm_field_s *f, bool f64) {
+    pl.kernel = c.kernel;
+    // the single-step kernel, for a remainder of one
+    pl.cost[1] = 4.0 + (f64 ? 2.5e-5 : 1.4e-5) * (double)f->nx * (double)f->ny;
+    // both fields beyond the last-level cache (256 MB): 4 TB/s at best
+    const double bytes = 2.0 * f->Q * (f64 ? 8 : 4) * (double)f->nx * (double)f->ny;
+    const double memory = bytes > 2e8 ? bytes / 4e6 : 0.0;
+    pl.max_steps = 2;
+    for (int t = 2; t <= c.tmax; ++t) {
+        const lbm::BlockShape b = lbm::block_shape(f->nx, f->ny, t, c.rows, f64 ? 8 : 4);
+        const long long rounds = ((long long)b.across * b.down + 255) / 256;
+        pl.cost[t] = std::max(c.a[t] + c.b[t] * (double)(rounds - 1), memory);
+        if (pl.cost[t] / t < pl.cost[pl.max_steps] / pl.max_steps) pl.max_steps = t;
+    }
+}
+
 // lattices for the 8 x 8 tiles (420 of them: 164 x 164; us a step on 160^2
 // against the 64 x 16 blocks: 1.66 / 1.79 in FP64, 0.95 / 1.09 in FP32)
 bool small_tiles(const lbm_field_s *f) {
@@ -575,9 +615,17 @@ MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     if (!f64 && f->storage != LBM_STORE_F32) return pl;
     if (small_tiles(f)) any_up_to(lbm::kMultiTile, 8);
     else if (!wide) return pl;
-    else if (nodes <= 90000) any_up_to(lbm::kMultiBlock16, 6);
-    else if (nodes <= 400000) any_up_to(lbm::kMultiBlock32, 6);
-    else if (nodes <= 2000000) any_up_to(lbm::kMultiBlockWide, f64 ? 5 : 6);
+    else if (nodes <= (f64 ? 3000000 : 10000000)) {
+        // (marching waves / wide blocks, us a step: FP64 32.5 / 32.8 on 1800^2,
+        // 73 / 78 on 3000^2; FP32 37 / 35 on 3000^2, 56 / 60 on 4096^2)
+        const BlockCost *table = f64 ? kBlockCost64 : kBlockCost32;
+        plan_blocks(pl, table[0], f, f64);
+        for (int k = 1; k < 3; ++k) {
+            MultiPlan o;
+            plan_blocks(o, table[k], f, f64);
+            if (o.cost[o.max_steps] / o.max_steps < pl.cost[pl.max_steps] / pl.max_steps) pl = o;
+        }
+    }
     else {
         pl.kernel = lbm::kMultiMarch;
         pl.max_steps = f64 ? 5 : 6;
@@ -2327,65 +2375,76 @@ int adj_forward_op(lbm_adjoint a, lbm::Op op, const void *src, void *dst) {
     return 0;
 }
 
-// n collisions from src, several per pass where the lattice suits it; `first`:
-// the first one collides the canonical state in place, the others follow a
-// stream.  Intermediate fields alternate between pp[0] and pp[1]; the last one
-// goes to dst or, when that is null, to the next of the two.  *result: where.
+// FP32 TRT stays with single steps in both directions: its dL/dtau_a is a sum
+// whose terms cancel by up to six digits, so that another rounding of the last
+// place (4e-8 of a step) moves it by up to a third
+bool adj_single_steps(lbm_adjoint a) {
+    return a->geo.storage == LBM_STORE_F32 && a->m->coll == LBM_TRT;
+}
+
+// the passes of an adjoint: as lbm_simulate's, but blocks where that takes
+// marching waves (the kernels that can keep every step's field)
+MultiPlan adj_plan(lbm_adjoint a) {
+    if (adj_single_steps(a)) return MultiPlan{};
+    MultiPlan pl = multi_plan(a->m, &a->geo);
+    if (pl.kernel == lbm::kMultiMarch) {
+        pl = MultiPlan{};
+        const bool f64 = a->geo.storage == LBM_STORE_F64;
+        plan_blocks(pl, (f64 ? kBlockCost64 : kBlockCost32)[2], &a->geo, f64);
+    }
+    return pl;
+}
+
+// One pass of n collisions from src, the field after collision l + 1 kept in
+// out[l] (null: not kept, never the last); `first`: the first one collides the
+// canonical state in place, the others follow a stream.
+int adj_pass(lbm_adjoint a, const MultiPlan &plan, const void *src, int n, bool first,
+             void *const *out) {
+    if (n == 1)
+        return adj_forward_op(a, first ? lbm::Op::Collide : lbm::Op::Fused, src, out[0]);
+    lbm::MultiLaunch L{};
+    L.kernel = plan.kernel;
+    L.qid = a->geo.qid;
+    L.coll = a->m->coll;
+    L.steps = n;
+    L.first = first ? 1 : 0;
+    L.src = src;
+    lbm::LevelOut o{};
+    for (int l = 0; l < n; ++l) o.out[l] = out[l];
+    const lbm::StepParams<double> p = make_params(a->m, &a->geo, false);
+    const int rc = a->geo.storage == LBM_STORE_F64
+                       ? lbm::run_multi_all_f64(L, o, p, g_stream)
+                       : lbm::run_multi_all_f32(L, o, lbm::to_float_params(p), g_stream);
+    if (rc) return fail(-4, "kernel launch failed (code %d): %s", rc,
+                        hipGetErrorString(hipGetLastError()));
+    return 0;
+}
+
+// n collisions from src; intermediate fields alternate between pp[0] and pp[1],
+// the last one goes to dst or, when that is null, to the next of the two.
+// *result: where.
 int adj_advance(lbm_adjoint a, const MultiPlan &plan, const void *src, int64_t n, bool first,
                 void *dst, const void **result) {
     const void *cur = src;
     while (n > 0) {
         const int k = plan.kernel != lbm::kMultiNone ? multi_next(plan, n) : 1;
         n -= k;
-        void *to = n == 0 && dst ? dst : (cur == a->pp[0] ? a->pp[1] : a->pp[0]);
-        int rc;
-        if (k > 1) {
-            lbm_field_s fs = a->geo, fd = a->geo;
-            fs.d = const_cast<void *>(cur);
-            fd.d = to;
-            rc = run_multi(plan, a->m, &fs, &fd, k, first);
-        } else {
-            rc = adj_forward_op(a, first ? lbm::Op::Collide : lbm::Op::Fused, cur, to);
-        }
-        if (rc) return rc;
-        cur = to;
+        void *out[8] = {};
+        out[k - 1] = n == 0 && dst ? dst : (cur == a->pp[0] ? a->pp[1] : a->pp[0]);
+        if (int rc = adj_pass(a, plan, cur, k, first, out)) return rc;
+        cur = out[k - 1];
         first = false;
     }
-    if (result) *result = cur;
+    *result = cur;
     return 0;
 }
 
-// The fields C_j .. of n collisions from src, each kept: out[0 .. n-1]
+// the fields of n collisions from src, each kept: out[0 .. n-1]
 int adj_advance_all(lbm_adjoint a, const MultiPlan &plan, const void *src, int64_t n, bool first,
                     void *const *out) {
-    MultiPlan pl = plan;
-    if (pl.kernel == lbm::kMultiMarch) {  // waves keep their levels' rows: blocks instead
-        pl.kernel = lbm::kMultiBlockWide;
-        for (int k = 1; k <= pl.max_steps; ++k) pl.cost[k] = 2.0 + k;
-    }
-    const lbm::StepParams<double> p = make_params(a->m, &a->geo, false);
     while (n > 0) {
-        const int k = pl.kernel != lbm::kMultiNone ? multi_next(pl, n) : 1;
-        int rc;
-        if (k > 1) {
-            lbm::MultiLaunch L{};
-            L.kernel = pl.kernel;
-            L.qid = a->geo.qid;
-            L.coll = a->m->coll;
-            L.steps = k;
-            L.first = first ? 1 : 0;
-            L.src = src;
-            lbm::LevelOut o{};
-            for (int l = 0; l < k; ++l) o.out[l] = out[l];
-            rc = a->geo.storage == LBM_STORE_F64
-                     ? lbm::run_multi_all_f64(L, o, p, g_stream)
-                     : lbm::run_multi_all_f32(L, o, lbm::to_float_params(p), g_stream);
-            if (rc) return fail(-4, "kernel launch failed (code %d): %s", rc,
-                                hipGetErrorString(hipGetLastError()));
-        } else {
-            rc = adj_forward_op(a, first ? lbm::Op::Collide : lbm::Op::Fused, src, out[0]);
-            if (rc) return rc;
-        }
+        const int k = plan.kernel != lbm::kMultiNone ? multi_next(plan, n) : 1;
+        if (int rc = adj_pass(a, plan, src, k, first, out)) return rc;
         src = out[k - 1];
         out += k;
         n -= k;
@@ -2407,7 +2466,7 @@ int adjoint_forward(lbm_adjoint a, const double *u0, const double *ut, bool want
     if (int rc = adj_launch(a, p, L)) return rc;
     // segment by segment to the checkpoints C_{K-1}, C_{2K-1}, .. and to C_{T-1}
     const int64_t T = a->nsteps;
-    const MultiPlan plan = multi_plan(a->m, &a->geo);
+    const MultiPlan plan = adj_plan(a);
     const void *last = a->S0;
     for (int s = 0; s < a->nseg; ++s) {
         const int64_t n = std::min<int64_t>(a->K, T - (int64_t)s * a->K);
@@ -2551,8 +2610,9 @@ int lbm_adjoint_gradient(lbm_adjoint a, const double *u0, const double *u_target
     const lbm::StepParams<double> p = make_params(a->m, &a->geo, false);
     const long long plane = (long long)a->geo.nx * a->geo.ny;
     HIP_TRY(hipMemsetAsync(a->dgtau, 0, (size_t)plane * 2 * sizeof(double), g_stream));
-    const MultiPlan plan = multi_plan(a->m, &a->geo);
-    const bool tiled = a->geo.qid == 4 || a->geo.qid == 5 || a->geo.qid == 9;
+    const MultiPlan plan = adj_plan(a);
+    const bool tiled =
+        (a->geo.qid == 4 || a->geo.qid == 5 || a->geo.qid == 9) && !adj_single_steps(a);
     int cur = 0;  // lam[cur] holds lambda_{t+1}
     for (int s = a->nseg - 1; s >= 0; --s) {
         const int64_t t0 = (int64_t)s * a->K;

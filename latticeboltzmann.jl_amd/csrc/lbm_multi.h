@@ -213,8 +213,10 @@ __device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const Step
 template <int QID, int COLL, class T>
 __device__ __forceinline__ void collide_multi(T (&f)[QT<QID>::Q], const StepParams<T> &p,
                                               const MultiConsts<T> &mc, int x, int y) {
-    static_assert(COLL <= 2 && QT<QID>::FEQ <= 2, "one-speed stencils, SRT, TRT and MRT");
-    if constexpr (COLL <= 1) {
+    static_assert(QT<QID>::FEQ <= 2, "one-speed stencils");
+    if constexpr (COLL == 4) {  // SRT in the single-step kernels' own form
+        collide_any<QID, 0>(f, p, x, y);
+    } else if constexpr (COLL <= 1) {
         collide_pairs<QID, COLL>(f, p, mc, x, y, LBM_SEQ);
     } else {
         double rho, ux, uy;
@@ -426,7 +428,7 @@ tile_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *__
         }
     };
     auto store = [&](S *dst, int k) {
-        if (!mine[k]) return;
+        if (!mine[k] || (ALL && !dst)) return;
         auto st = [&](auto Ic) {
             constexpr int i = decltype(Ic)::value;
             dst[p.plane * i + ((long long)xs[k] + (long long)p.nx * ys[k])] = ST::encode(f[k][i], i, p);
@@ -599,7 +601,7 @@ block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *_
     // row j of a level to `dst`, where this block owns it
     auto store = [&](S *dst, int j, const V(&f)[Q]) {
         const int uy = cy0 - h + row0 + j;
-        if (mine_x && uy >= cy0 && uy < min(cy0 + outy, p.ny)) {
+        if (mine_x && uy >= cy0 && uy < min(cy0 + outy, p.ny) && (!ALL || dst)) {
             S *base = dst + (long long)pitch * uy;
             auto st = [&](auto Ic) {
                 constexpr int i = decltype(Ic)::value;
@@ -1112,7 +1114,27 @@ int launch_all(const MultiLaunch &L, const LevelOut &o, const StepParams<typenam
     }
 }
 
-#define LBM_DEFINE_MULTI_ALL(TAG, ST)                                                             int run_multi_all_##TAG(const MultiLaunch &L, const LevelOut &o,                                                      const StepParams<typename ST::T> &p, hipStream_t s) {                     switch (L.qid * 2 + L.coll) {                                                                 case 8: return launch_all<4, 0, ST>(L, o, p, s);                                              case 9: return launch_all<4, 1, ST>(L, o, p, s);                                              case 10: return launch_all<5, 0, ST>(L, o, p, s);                                             case 11: return launch_all<5, 1, ST>(L, o, p, s);                                             case 18: return launch_all<9, 0, ST>(L, o, p, s);                                             case 19: return launch_all<9, 1, ST>(L, o, p, s);                                             default: return -1;                                                                           }                                                                                         }
+// FP64: the pair form (the same bits as the single-step kernels').  FP32: SRT
+// in the single-step kernels' own form, which gives their bits too; TRT has no
+// such kernels (see adj_plan).
+template <class ST>
+int launch_all_any(const MultiLaunch &L, const LevelOut &o, const StepParams<typename ST::T> &p,
+                   hipStream_t s) {
+    constexpr bool f64 = sizeof(typename ST::store_t) == 8;
+    if constexpr (f64)
+        switch (L.coll == 1 ? L.qid : 0) {
+        case 4: return launch_all<4, 1, ST>(L, o, p, s);
+        case 5: return launch_all<5, 1, ST>(L, o, p, s);
+        case 9: return launch_all<9, 1, ST>(L, o, p, s);
+        }
+    constexpr int SRT = f64 ? 0 : 4;
+    switch (L.coll == 0 ? L.qid : 0) {
+    case 4: return launch_all<4, SRT, ST>(L, o, p, s);
+    case 5: return launch_all<5, SRT, ST>(L, o, p, s);
+    case 9: return launch_all<9, SRT, ST>(L, o, p, s);
+    default: return -1;
+    }
+}
 
 
 template <int QID, int COLL, class ST, int T, int NC, bool BC>

@@ -16,10 +16,12 @@ pytestmark = pytest.mark.gpu
 
 # (nx, ny): by kernel, smallest to largest
 TILE = [(1, 1), (2, 3), (3, 40), (9, 8), (64, 64), (200, 199)]
-BLOCK16 = [(257, 160), (32, 2500), (9001, 12), (31, 2501), (9001, 11)]
-BLOCK32 = [(513, 300), (55, 2500)]
-WIDE = [(1021, 517), (57, 8001)]
-MARCH = [(2049, 1000), (33, 61001), (170001, 12), (700001, 3)]
+# (the steps per pass of a block kernel differ by shape)
+BLOCK16 = [(257, 160), (32, 2500), (9001, 12), (31, 2501), (9001, 11), (300, 300), (340, 340),
+           (380, 380)]
+BLOCK32 = [(513, 300), (55, 2500), (460, 460), (560, 560), (600, 600)]
+WIDE = [(1021, 517), (57, 8001), (700, 700), (760, 760), (2049, 1000), (33, 61001), (170001, 12)]
+MARCH = [(2049, 1500), (47, 65001), (250001, 12), (1200001, 3)]
 SHAPES = TILE + BLOCK16 + BLOCK32 + WIDE + MARCH
 
 
@@ -83,19 +85,20 @@ def test_f64_every_pass_size(oracle_lib, shape, steps):
 
 @pytest.mark.parametrize("steps", [2, 3, 4, 6, 7])
 def test_f64_march_pass_sizes(oracle_lib, steps):
-    _check_f64(oracle_lib, 9, 1, 2049, 1000, "couette", "const", steps)
+    _check_f64(oracle_lib, 9, 1, 2049, 1500, "couette", "const", steps)
 
 
 @pytest.mark.parametrize("qid", [4, 5])
 @pytest.mark.parametrize("coll", [0, 1, 2])
-@pytest.mark.parametrize("shape", [(19, 40), (257, 160), (513, 300), (700, 650), (2049, 1000)])
+@pytest.mark.parametrize("shape", [(19, 40), (257, 160), (513, 300), (700, 650), (2049, 1500)])
 def test_f64_other_one_speed_sets(oracle_lib, qid, coll, shape):
     _check_f64(oracle_lib, qid, coll, *shape, "cavity", "const", 9)
 
 
 @pytest.mark.parametrize("coll", [0, 1])
 @pytest.mark.parametrize("shape", [(3, 40), (64, 64), (257, 160), (513, 300), (1021, 517),
-                                   (2050, 1000), (33, 61001)])
+                                   (2050, 1000), (33, 61001), (300, 300), (340, 340), (380, 380),
+                                   (460, 460), (560, 560), (4097, 2500), (161, 65001)])
 @pytest.mark.parametrize("bcname,force", [("periodic", "none"), ("cavity", "field")])
 def test_f32_tracks_oracle(oracle_lib, coll, shape, bcname, force):
     """FP32 on shifted populations |g| = |f - w| <= G: a step's rounding errors
