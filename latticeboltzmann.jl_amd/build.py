@@ -25,6 +25,8 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+import time
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
@@ -63,6 +65,8 @@ def _deps(src):
         return [os.path.join(CSRC, "lbm_internal.h")]
     if src.startswith("k_multi"):
         return kern + [os.path.join(CSRC, "lbm_multi.h")]
+    if src.startswith("k_stage"):
+        return kern + [os.path.join(CSRC, "lbm_multi.h"), os.path.join(CSRC, "lbm_stage.h")]
     if src.startswith("k_adjoint"):
         return kern + [os.path.join(CSRC, "lbm_multi.h"), os.path.join(CSRC, "lbm_adjoint.h")]
     return kern
@@ -87,7 +91,8 @@ def build(force: bool = False, verbose: bool = False) -> str:
         jobs.append((src, [HIPCC, *COMMON, *flags, "-c", s, "-o", o]))
     # heaviest units first, at most one hipcc per CPU
     jobs.sort(key=lambda j: (not j[0].startswith("k_"),
-                             "q37" not in j[0] and "multi_f" not in j[0], j[0]))
+                             "q37" not in j[0] and "multi_f" not in j[0]
+                             and "stage" not in j[0], j[0]))
     width = max(1, min(len(jobs), os.cpu_count() or 1, 16))
     procs = []
     failed = []
@@ -97,11 +102,17 @@ def build(force: bool = False, verbose: bool = False) -> str:
             src, cmd = pending.pop(0)
             if verbose:
                 print(" ".join(cmd), flush=True)
-            procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE,
-                                                stderr=subprocess.STDOUT)))
-        src, p = procs.pop(0)
-        out, _ = p.communicate()
-        text = out.decode(errors="replace")
+            log = tempfile.TemporaryFile()
+            procs.append((src, subprocess.Popen(cmd, stdout=log, stderr=subprocess.STDOUT), log))
+        time.sleep(0.05)
+        done = [q for q in procs if q[1].poll() is not None]
+        if not done:
+            continue
+        procs.remove(done[0])
+        src, p, log = done[0]
+        log.seek(0)
+        text = log.read().decode(errors="replace")
+        log.close()
         # the host pass does not know the packed-fp32 target feature; that warning is harmless
         lines = [ln for ln in text.splitlines() if "packed-fp32-ops" not in ln
                  and "not a recognized feature" not in ln]

@@ -1,0 +1,7 @@
+// k_stage_f64_q13.hip -- several fused steps per pass, storage f64, D2Q13.
+// Plain FP64: compiled with -ffp-contract=off (bit-exact with the CPU restatement).
+#include "lbm_stage.h"
+
+namespace lbm {
+LBM_DEFINE_STAGES(f64, StF64, 13)
+}  // namespace lbm

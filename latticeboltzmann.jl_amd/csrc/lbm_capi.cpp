@@ -575,6 +575,56 @@ bool small_tiles(const lbm_field_s *f) {
     return (long long)((f->nx + 7) / 8) * ((f->ny + 7) / 8) <= 420;
 }
 
+// Pipelines of wave groups for the stencils that reach two or three nodes: us a
+// step of the single-step kernels (a1 + b1 per million nodes) and of the
+// pipeline (a2 + b2 per million nodes of whole strips), measured on 192^2 and
+// 512^2, SRT and TRT.  The lines cross between 0.12 million nodes (D2Q13 FP64)
+// and 0.4 (D2Q17 FP32); the pipeline's run-in costs more than it saves below.
+struct StageCost {
+    int qid;
+    bool f64;
+    double a1, b1, a2, b2;
+};
+const StageCost kStageCost[8] = {
+    {13, true, 4.4, 33, 7.4, 6.3},  {13, false, 4.4, 13.6, 5.7, 6.0},
+    {17, true, 5.1, 42, 11.8, 9.1}, {17, false, 4.9, 19.2, 9.8, 6.4},
+    {21, true, 6.0, 67, 15.3, 14.3}, {21, false, 6.1, 29.9, 10.7, 6.7},
+    {37, true, 9.5, 121, 22.5, 30.8}, {37, false, 8.7, 40, 13.7, 7.7}};
+
+MultiPlan plan_stages(const lbm_model_s *m, const lbm_field_s *f) {
+    MultiPlan pl;
+    const bool f64 = f->storage == LBM_STORE_F64;
+    if ((!f64 && f->storage != LBM_STORE_F32) || (m->coll != LBM_SRT && m->coll != LBM_TRT))
+        return pl;
+    int walls = 0;
+    bool full = true;
+    for (const auto &b : m->bcs) {
+        if (b.direction != LBM_NORTH && b.direction != LBM_SOUTH) return pl;
+        walls |= 1 << b.direction;
+        full = full && (b.kind == LBM_MOVING_WALL ||
+                        (b.x0 <= 1 && b.x1 >= f->nx && b.y0 <= 1 && b.y1 >= f->ny));
+    }
+    if (f->nx < 64 || f->ny < 16) return pl;
+    int steps = lbm::stage_steps(m->qid, f64);
+    // (see k_stages: three steps need walls that span the lattice)
+    if (walls == (1 << LBM_NORTH | 1 << LBM_SOUTH) && !full) steps = 2;
+    const int out = lbm::stage_out(m->qid == 13 ? 2 : 3, steps, f64 ? 8 : 4);
+    const double nodes = 1e-6 * (double)f->nx * (double)f->ny;
+    const double strips = 1e-6 * (double)((f->nx + out - 1) / out * out) * (double)f->ny;
+    for (const StageCost &c : kStageCost)
+        if (c.qid == m->qid && c.f64 == f64 &&
+            c.a2 + c.b2 * strips > 0.95 * (c.a1 + c.b1 * nodes))
+            return pl;
+    pl.kernel = lbm::kMultiStages;
+    pl.max_steps = steps;
+    // passes of one, two and three steps on 2048 x 1024: 47, 62, 87 us (D2Q13
+    // FP32) to 253, 340 us (D2Q37 FP64)
+    pl.cost[1] = 10;
+    pl.cost[2] = 13;
+    if (steps > 2) pl.cost[3] = 16.5;
+    return pl;
+}
+
 MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     MultiPlan pl;
     if (m->launch_block || m->launch_rows || m->launch_vec || m->launch_nt >= 0) {
@@ -587,7 +637,7 @@ MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
         auto_launch(&def, f, b0, r0, v0, nt0);
         if (b != b0 || r != r0 || v != v0 || nt != nt0) return pl;
     }
-    if (m->qid != 4 && m->qid != 5 && m->qid != 9) return pl;
+    if (m->qid != 4 && m->qid != 5 && m->qid != 9) return plan_stages(m, f);
     if (m->coll != LBM_SRT && m->coll != LBM_TRT &&
         !(m->coll == LBM_MRT && f->storage == LBM_STORE_F64))
         return pl;
@@ -2387,6 +2437,7 @@ bool adj_single_steps(lbm_adjoint a) {
 MultiPlan adj_plan(lbm_adjoint a) {
     if (adj_single_steps(a)) return MultiPlan{};
     MultiPlan pl = multi_plan(a->m, &a->geo);
+    if (pl.kernel == lbm::kMultiStages) return MultiPlan{};  // keeps no step's field
     if (pl.kernel == lbm::kMultiMarch) {
         pl = MultiPlan{};
         const bool f64 = a->geo.storage == LBM_STORE_F64;

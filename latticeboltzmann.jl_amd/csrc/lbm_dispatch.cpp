@@ -41,9 +41,25 @@ int dispatch_lp(const Launch &L, const StepParams<double> &pd, hipStream_t s) {
     default: return -1;                                     \
     }
 
+#define LBM_SWITCH_STAGES(TAG, L, p, s)                     \
+    switch ((L).qid) {                                      \
+    case 13: return run_multi_##TAG##_q13(L, p, s);         \
+    case 17: return run_multi_##TAG##_q17(L, p, s);         \
+    case 21: return run_multi_##TAG##_q21(L, p, s);         \
+    case 37: return run_multi_##TAG##_q37(L, p, s);         \
+    default: return -1;                                     \
+    }
+
 int dispatch_multi(int storage, const MultiLaunch &L, const StepParams<double> &pd, hipStream_t s) {
-    if (storage == 0) LBM_SWITCH_MULTI(f64, L, pd, s)
+    if (storage == 0) {
+        if (L.kernel == kMultiStages) LBM_SWITCH_STAGES(f64, L, pd, s)
+        LBM_SWITCH_MULTI(f64, L, pd, s)
+    }
     const StepParams<float> p = to_float_params(pd);
+    if (L.kernel == kMultiStages) {
+        if (storage != 1) return -1;
+        LBM_SWITCH_STAGES(f32, L, p, s)
+    }
     switch (storage) {
     case 1: LBM_SWITCH_MULTI(f32, L, p, s)
     case 4: LBM_SWITCH_MULTI(f16neq, L, p, s)

@@ -135,14 +135,15 @@ struct Launch {
     int nt = 0;   // fused step: non-temporal stores
 };
 
-// Several fused steps in one pass (lbm_multi.h): one-speed stencils, storages
-// F64, F32 and the non-equilibrium ones.
+// Several fused steps in one pass: one-speed stencils, storages F64, F32 and the
+// non-equilibrium ones (lbm_multi.h), the others F64 and F32 (lbm_stage.h).
 enum MultiKernel : int {
     kMultiTile = 0,   // LDS tile of 8 x 8 nodes, up to 8 steps
     kMultiBlock16,    // register block of 64 x 16 nodes
     kMultiBlock32,    // 64 x 32, 16 waves
     kMultiBlockWide,  // 64 x 24 (FP64) or 64 x 32 (FP32), 8 waves
     kMultiMarch,      // marching waves: 2-5 steps (FP64), 2-4 or 6 (FP32), 2-4 (16-bit)
+    kMultiStages,     // pipelines of wave groups on D2Q13/17/21/37: stage_steps()
     kMultiNone
 };
 // A register block is 64 columns x `rows` rows and computes a halo of steps - 1
@@ -164,6 +165,18 @@ inline BlockShape block_shape(int nx, int ny, int steps, int rows, int elem_byte
     return b;
 }
 constexpr int kMarchRows = 16;  // fewest rows of a marching wave
+constexpr int kStageRows = 8;   // fewest rows of a pipeline's chunk
+// Most steps of a pipeline pass.  FP64 D2Q21/37: the rings of one hand-over
+// fill the LDS.  FP32 D2Q17: four blocks of two steps on a CU hide more latency
+// than two blocks of three (2048 x 1024 channel: 43 us a step against 50).
+constexpr int stage_steps(int qid, bool f64) { return f64 ? (qid <= 17 ? 3 : 2) : (qid == 17 ? 2 : 3); }
+// columns that a block of the pipeline computes, and those it writes: whole
+// 64-byte groups
+constexpr int kStageCols = 128;
+constexpr int stage_out(int maxc, int steps, int elem_bytes) {
+    const int group = 64 / elem_bytes;
+    return (kStageCols - 2 * maxc * (steps - 1)) / group * group;
+}
 // Stop of the iterative initialization, kept on the device: the density of
 // node (nx, ny) after the last step and the first step that converged (0: none)
 struct MeiWatch {
@@ -237,6 +250,13 @@ int run_batch_f32_q9(int op, const BatchLattice *lats, const BatchTile *tiles, i
 LBM_DECLARE_MULTI(f64, double)
 LBM_DECLARE_MULTI(f32, float)
 LBM_DECLARE_MULTI(f16neq, float)
+#define LBM_DECLARE_STAGES(TAG, T)                                                        \
+    int run_multi_##TAG##_q13(const MultiLaunch &L, const StepParams<T> &p, hipStream_t s); \
+    int run_multi_##TAG##_q17(const MultiLaunch &L, const StepParams<T> &p, hipStream_t s); \
+    int run_multi_##TAG##_q21(const MultiLaunch &L, const StepParams<T> &p, hipStream_t s); \
+    int run_multi_##TAG##_q37(const MultiLaunch &L, const StepParams<T> &p, hipStream_t s);
+LBM_DECLARE_STAGES(f64, double)
+LBM_DECLARE_STAGES(f32, float)
 LBM_DECLARE_MULTI(bf16neq, float)
 // several fused steps of a periodic SRT/TRT model that store every step's field
 // (out[l]: collision l of the pass); tile and block kernels

@@ -82,46 +82,63 @@ __device__ __forceinline__ void moments_div2(const double (&f)[QT<QID>::Q], doub
     div2(mx, my, rho, ux, uy);
 }
 
-// collide! of one node for the first- and second-order equilibria, one
-// opposite pair (i, j) at a time: c_j = -c_i, so u.c, its square, the
-// second-order term and (TRT) the symmetric and antisymmetric parts of the
-// pair are formed once.  Rounding for rounding the values are those of
+// collide! of one node, one opposite pair (i, j) at a time: c_j = -c_i, so u.c,
+// its powers, the terms of the expansion (the odd ones change sign) and (TRT)
+// the symmetric and antisymmetric parts of the pair are formed once.  `before(i, ..)`
+// runs ahead of population i's part and may touch the velocity that the rest
+// depends on.  Rounding for rounding the values are those of
 // collide_seq (negation and scaling by 1/2 are exact); D2Q9 TRT FP64 takes
 // 137 arithmetic instructions instead of 224.
-template <int QID, int COLL, int... Is>
+template <int QID, int COLL, class F, class H, int... Is>
 __device__ __forceinline__ void collide_pairs(double (&f)[QT<QID>::Q], const StepParams<double> &p,
-                                              const MultiConsts<double> &mc, int x, int y,
+                                              const MultiConsts<double> &mc, F &&force, H &&before,
                                               std::integer_sequence<int, Is...>) {
     constexpr int FEQ = QT<QID>::FEQ;
-    static_assert(FEQ <= 2 && COLL <= 1, "pair form: orders one and two, SRT and TRT");
+    static_assert(COLL <= 1, "pair form: SRT and TRT");
     double rho, ux, uy;
     moments_div2<QID>(f, rho, ux, uy, LBM_SEQ);
     if (p.force_kind != 0) {
         double Fx, Fy;
-        node_force(p, x, y, Fx, Fy);
+        force(Fx, Fy);
         ux = ux + p.tau_force * Fx;  // srt.jl:54 / trt.jl:79
         uy = uy + p.tau_force * Fy;
     }
     const double usq = ux * ux + uy * uy;
     const double hq = mc.hns * usq;
+    // orders three and four: the factors are those of a3 / 6 and a4 / 24 with
+    // the 1/2 of s^2 (u.c)^2 / 2 carried into them
+    const double q3 = 0.5 * (p.three_s * usq), q4 = p.six_s3 * usq, k4 = p.three_s2 * (usq * usq);
     double rw[QT<QID>::Q];
     auto one = [&](auto Ic) {
         constexpr int i = decltype(Ic)::value;
         constexpr int j = QT<QID>::opp(i), wr = weight_rep<QID>(i);
+        before(Ic, ux, uy);
         if constexpr (wr == i) rw[i] = rho * p.w[i];
         if constexpr (i <= j) {
             const double ud = udot<QID, i>(ux, uy);
             double qi, qj;
             if constexpr (i == j) {
-                qi = FEQ == 2 ? rw[wr] * (1.0 + hq) : rw[wr];
+                double a0 = FEQ >= 2 ? 1.0 + hq : 1.0;
+                if constexpr (FEQ >= 4) a0 = a0 + (1.0 / 24.0) * k4;
+                qi = FEQ >= 2 ? rw[wr] * a0 : rw[wr];
                 qj = qi;
             } else {
                 const double a1 = p.s * ud;
                 double ai = 1.0 + a1, aj = 1.0 - a1;
-                if constexpr (FEQ == 2) {
-                    const double h2 = mc.hs2 * (ud * ud) + hq;
+                if constexpr (FEQ >= 2) {
+                    const double ud2 = ud * ud, m2 = mc.hs2 * ud2, h2 = m2 + hq;
                     ai = ai + h2;
                     aj = aj + h2;
+                    if constexpr (FEQ >= 3) {
+                        const double t3 = (2.0 * (1.0 / 6.0)) * (a1 * (m2 - q3));
+                        ai = ai + t3;
+                        aj = aj - t3;
+                    }
+                    if constexpr (FEQ >= 4) {
+                        const double t4 = (1.0 / 24.0) * ((p.s4 * pow4(ud) - q4 * ud2) + k4);
+                        ai = ai + t4;
+                        aj = aj + t4;
+                    }
                 }
                 qi = rw[wr] * ai;
                 qj = rw[wr] * aj;
@@ -149,12 +166,12 @@ __device__ __forceinline__ void collide_pairs(double (&f)[QT<QID>::Q], const Ste
 // equilibrium (ev, od as in collide_neq_pairs), ns = (g_i + g_j) - 2 w ev and
 // na = (g_i - g_j) - 2 w od are the relaxed parts: g_i - ns / (2 tau_s) -
 // na / (2 tau_a).  D2Q9 TRT: 66 instructions per node instead of 92.
-template <int QID, int COLL, int... Is>
+template <int QID, int COLL, class F, class H, int... Is>
 __device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const StepParams<float> &p,
-                                              const MultiConsts<float> &mc, int x, int y,
+                                              const MultiConsts<float> &mc, F &&force, H &&before,
                                               std::integer_sequence<int, Is...>) {
     constexpr int FEQ = QT<QID>::FEQ, Q = QT<QID>::Q;
-    static_assert(FEQ <= 2 && COLL <= 1, "pair form: orders one and two, SRT and TRT");
+    static_assert(COLL <= 1, "pair form: SRT and TRT");
     float s[Q], d[Q];  // pair sums and differences, at the smaller index
     auto sums = [&](auto Ic) {
         constexpr int i = decltype(Ic)::value, j = QT<QID>::opp(i);
@@ -179,23 +196,40 @@ __device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const Step
     float ux = mx * ir, uy = my * ir;
     if (p.force_kind != 0) {
         float Fx, Fy;
-        node_force(p, x, y, Fx, Fy);
+        force(Fx, Fy);
         ux = ux + p.tau_force * Fx;
         uy = uy + p.tau_force * Fy;
     }
-    // the record form of the equilibrium (make_rec)
-    const float sr = p.s * rho, ax = sr * ux, ay = sr * uy;
-    const float a0 = FEQ == 2 ? drho - 0.5f * (ax * ux + ay * uy) : drho;
-    const float a3 = 0.5f * ir;
+    // the record form of the equilibrium (make_rec); orders three and four: the
+    // even and odd powers of node_eq's polynomial in t = c.u
+    float ax = ux, ay = uy, a0, a3 = 0.0f;
+    NodeEq e;
+    if constexpr (FEQ <= 2) {
+        const float sr = p.s * rho;
+        ax = sr * ux;
+        ay = sr * uy;
+        a0 = FEQ == 2 ? drho - 0.5f * (ax * ux + ay * uy) : drho;
+        a3 = 0.5f * ir;
+    } else {
+        e = node_eq<QID>(drho, ux, uy, p);
+        a0 = e.k0;
+    }
     auto one = [&](auto Ic) {
         constexpr int i = decltype(Ic)::value;
         constexpr int j = QT<QID>::opp(i), wr = weight_rep<QID>(i);
+        before(Ic, ax, ay);
         if constexpr (i == j) {
             const float n = f[i] - p.w[wr] * a0;
             f[i] = f[i] - (COLL == 0 ? p.om : p.oms) * n;
         } else if constexpr (i < j) {
-            const float od = udot<QID, i>(ax, ay);
-            const float ev = FEQ == 2 ? a0 + a3 * (od * od) : a0;
+            float od = udot<QID, i>(ax, ay), ev = a0;
+            if constexpr (FEQ == 2) {
+                ev = a0 + a3 * (od * od);
+            } else if constexpr (FEQ > 2) {
+                const float t = od, t2 = t * t;
+                od = t * (e.k1 + t2 * e.k3);
+                ev = FEQ == 3 ? a0 + t2 * e.k2 : a0 + t2 * (e.k2 + t2 * e.k4);
+            }
             if constexpr (COLL == 0) {
                 const float w = p.w[wr];
                 f[i] = f[i] - p.om * (f[i] - w * (ev + od));
@@ -213,11 +247,11 @@ __device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const Step
 template <int QID, int COLL, class T>
 __device__ __forceinline__ void collide_multi(T (&f)[QT<QID>::Q], const StepParams<T> &p,
                                               const MultiConsts<T> &mc, int x, int y) {
-    static_assert(QT<QID>::FEQ <= 2, "one-speed stencils");
     if constexpr (COLL == 4) {  // SRT in the single-step kernels' own form
         collide_any<QID, 0>(f, p, x, y);
     } else if constexpr (COLL <= 1) {
-        collide_pairs<QID, COLL>(f, p, mc, x, y, LBM_SEQ);
+        collide_pairs<QID, COLL>(f, p, mc, [&](T &Fx, T &Fy) { node_force(p, x, y, Fx, Fy); },
+                                 [](auto, T &, T &) {}, LBM_SEQ);
     } else {
         double rho, ux, uy;
         moments_div2<QID>(f, rho, ux, uy, LBM_SEQ);

@@ -1,0 +1,71 @@
+"""Runs on the stencils that reach two or three nodes, several steps per pass
+(lbm_stage.h), against the oracle.
+
+The kernel writes 112 or 120 columns per block and at least 8 rows per chunk;
+the shapes sit at those edges: the smallest lattices it takes, one below, one
+block's columns and one more, lattices lower than a chunk's run-in, tall and
+long ones, and sizes of many blocks."""
+import numpy as np
+import pytest
+
+from lbm_cases import bc_dicts, force_for, to_lbmhip
+from test_gpu_multi import _L, _model, _oracle, _populations
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(64, 16), (63, 40), (70, 15), (112, 64), (113, 65), (120, 90), (121, 17), (65, 1201),
+          (3001, 19), (517, 261)]
+
+
+def _bcs(name, nx, ny):
+    if name != "bands":
+        return bc_dicts(name, nx, ny)
+    # ranges narrower than the walls, a later condition over an earlier one
+    return [dict(kind=0, direction=2, xs=(3, nx - 2), ys=(1, 2)),
+            dict(kind=1, direction=0, xs=(1, nx), ys=(1, ny), u=(0.04, 0.0), rho=1.0),
+            dict(kind=0, direction=0, xs=(5, nx // 2), ys=(ny - 1, ny)),
+            dict(kind=0, direction=2, xs=(nx // 2, nx), ys=(2, ny))]
+
+
+@pytest.mark.parametrize("qid", [13, 17, 21, 37])
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("coll,bcname,force,steps", [
+    (0, "periodic", "none", 7), (1, "bands", "field", 8), (0, "couette", "const", 5),
+    (1, "poiseuille", "const", 2), (1, "cavity", "none", 3)])
+def test_f64_bit_exact(oracle_lib, qid, shape, coll, bcname, force, steps):
+    nx, ny = shape
+    f0 = _populations(qid, nx, ny, seed=qid + coll)
+    F = force_for(force, nx, ny)
+    q, cm, taus = _model(qid, coll, F)
+    bcs = _bcs(bcname, nx, ny)
+    model = _L().LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs))
+    print(f"stages D2Q{qid} coll {coll} {nx}x{ny} {bcname} {force} {steps} steps", flush=True)
+    _L().simulate(model, range(steps))
+    S, C = _oracle(oracle_lib, qid, f0, coll, taus, steps, F, bcs)
+    assert np.array_equal(model.f_stream.to_numpy(), S)
+    assert np.array_equal(model.f_collision.to_numpy(), C)
+
+
+@pytest.mark.parametrize("qid", [13, 17, 21, 37])
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("coll,bcname,force,steps", [
+    (0, "periodic", "none", 7), (1, "bands", "field", 8), (1, "poiseuille", "const", 11)])
+def test_f32_error_no_larger_than_single_steps(oracle_lib, qid, shape, coll, bcname, force, steps):
+    """Every step rounds as the single-step kernels do (which the per-launch
+    timing entry point keeps): the populations' error against the oracle's
+    FP64 run is at most theirs, with a tenth for the scatter of roundings."""
+    L = _L()
+    nx, ny = shape
+    f0 = _populations(qid, nx, ny, seed=11, noise=1e-4)
+    F = force_for(force, nx, ny)
+    q, cm, taus = _model(qid, coll, F)
+    bcs = _bcs(bcname, nx, ny)
+    print(f"stages f32 D2Q{qid} coll {coll} {nx}x{ny} {bcname} {force}", flush=True)
+    many = L.LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs), storage="f32")
+    L.simulate(many, range(steps))
+    one = L.LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs), storage="f32")
+    L.simulate_launch_times(one, steps)
+    S, C = _oracle(oracle_lib, qid, f0, coll, taus, steps, F, bcs)
+    for a, b, ref in ((many.f_stream, one.f_stream, S), (many.f_collision, one.f_collision, C)):
+        ea, eb = (np.linalg.norm(x.to_numpy() - ref) for x in (a, b))
+        assert ea <= 1.1 * eb, (ea, eb)
