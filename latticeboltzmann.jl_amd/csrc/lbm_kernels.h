@@ -456,10 +456,6 @@ __device__ __forceinline__ void node_force(const StepParams<T> &p, int x, int y,
         const long long n = (long long)x + (long long)p.nx * y;
         Fx = static_cast<T>(p.Ffield[n]);
         Fy = static_cast<T>(p.Ffield[p.plane + n]);
-        // wait for the values here: waited for where the branches meet, a run
-        // without a field would wait there too, for all its loads and stores in
-        // flight
-        asm volatile("" : "+v"(Fx), "+v"(Fy));
     }
 }
 

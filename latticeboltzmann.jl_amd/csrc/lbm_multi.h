@@ -70,6 +70,21 @@ __device__ __forceinline__ void div2(double mx, double my, double r, double &ux,
     }
 }
 
+// node_force, a field's values waited for in the branch that loads them: waited
+// for where the branches meet, a run without a field would wait there too, for
+// all its loads and stores in flight (the single-step kernels, which have none
+// in flight there, are slower with it: FP16-DEV 64 x 1110 5.7 us a step for 5.3)
+template <class T>
+__device__ __forceinline__ void node_force_wait(const StepParams<T> &p, int x, int y, T &Fx, T &Fy) {
+    if (p.force_kind == 1) {
+        Fx = p.Fx;
+        Fy = p.Fy;
+    } else {
+        node_force(p, x, y, Fx, Fy);
+        asm volatile("" : "+v"(Fx), "+v"(Fy));
+    }
+}
+
 // node_moments with the shared reciprocal
 template <int QID, int... Is>
 __device__ __forceinline__ void moments_div2(const double (&f)[QT<QID>::Q], double &rho, double &ux,
@@ -250,7 +265,7 @@ __device__ __forceinline__ void collide_multi(T (&f)[QT<QID>::Q], const StepPara
     if constexpr (COLL == 4) {  // SRT in the single-step kernels' own form
         collide_any<QID, 0>(f, p, x, y);
     } else if constexpr (COLL <= 1) {
-        collide_pairs<QID, COLL>(f, p, mc, [&](T &Fx, T &Fy) { node_force(p, x, y, Fx, Fy); },
+        collide_pairs<QID, COLL>(f, p, mc, [&](T &Fx, T &Fy) { node_force_wait(p, x, y, Fx, Fy); },
                                  [](auto, T &, T &) {}, LBM_SEQ);
     } else {
         double rho, ux, uy;

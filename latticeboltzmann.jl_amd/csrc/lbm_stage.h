@@ -143,7 +143,7 @@ k_stages(const typename ST::store_t *__restrict__ C, typename ST::store_t *__res
     // next row are issued: read after them it would wait for them all.
     V Fx = V(0), Fy = V(0);
     auto read_force = [&] {
-        if (p.force_kind != 0) node_force(p, x, row, Fx, Fy);
+        if (p.force_kind != 0) node_force_wait(p, x, row, Fx, Fy);
     };
     auto collide = [&](V(&f)[Q]) {
         constexpr int P1 = (2 * Q / 5) | 1, P2 = P1 + 4;
