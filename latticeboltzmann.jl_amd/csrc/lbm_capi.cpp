@@ -13,6 +13,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -1682,14 +1683,25 @@ int lbm_mei_initialize(lbm_model m, lbm_field f_stream, lbm_field f_collision, d
 }
 
 // ---- on-device processing -----------------------------------------------------
+// Partial sums and results of k_track, kept with the handle that a program
+// holds for its rows: allocating and freeing them took most of a row's 50 us on
+// 256 x 256 nodes.  The results lie in host memory that the last kernel writes.
+struct TrackWork {
+    std::mutex mu;  // one row at a time
+    double *part = nullptr;
+    double *out = nullptr;
+};
+
 struct lbm_expected_s {
     int nx = 0, ny = 0;
     double *d = nullptr;  // 8 planes
+    TrackWork work;
 };
 
 struct lbm_velocity_tracker_s {
     int nx = 0, ny = 0;
     double *d = nullptr;  // u_x, u_y planes
+    TrackWork work;
 };
 
 static int planes_create(int nx, int ny, int nplanes, double **d, const char *what) {
@@ -1709,8 +1721,16 @@ static int planes_create(int nx, int ny, int nplanes, double **d, const char *wh
     return 0;
 }
 
+static void free_work(TrackWork &w) {
+    free_dev(reinterpret_cast<void *&>(w.part));
+    if (w.out) (void)hipHostFree(w.out);
+    w.out = nullptr;
+}
+
 // one pass of k_track over f; sums[kTrackCols] on the host
-static int track_sums(lbm_field f, const lbm::TrackArgs &a, double *sums, const char *what) {
+static int track_sums(lbm_field f, const lbm::TrackArgs &a, TrackWork &w, double *sums,
+                      const char *what) {
+    const std::lock_guard<std::mutex> lock(w.mu);
     const lbm::StepParams<double> p = field_params(f);
     const void *fdata;
     int fstorage;
@@ -1719,18 +1739,15 @@ static int track_sums(lbm_field f, const lbm::TrackArgs &a, double *sums, const 
     // fixed grid for a given lattice size: the summation order is reproducible
     const long long blocks = (p.plane + 255) / 256;
     const int npart = (int)(blocks < 2048 ? blocks : 2048);
-    double *part = nullptr, *out = nullptr;
-    hipError_t e = hipMalloc(&part, (size_t)npart * lbm::kTrackCols * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&out, lbm::kTrackCols * sizeof(double));
+    hipError_t e = hipSuccess;
+    if (!w.part) e = hipMalloc(&w.part, (size_t)npart * lbm::kTrackCols * sizeof(double));
+    if (e == hipSuccess && !w.out)
+        e = hipHostMalloc(&w.out, lbm::kTrackCols * sizeof(double), hipHostMallocDefault);
     int rc = 0;
     if (e == hipSuccess)
-        rc = lbm::dispatch_track(f->qid, fstorage, fdata, p, a, part, npart, out, g_stream);
-    if (e == hipSuccess && !rc)
-        e = hipMemcpyAsync(sums, out, lbm::kTrackCols * sizeof(double), hipMemcpyDeviceToHost,
-                           g_stream);
+        rc = lbm::dispatch_track(f->qid, fstorage, fdata, p, a, w.part, npart, w.out, g_stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
-    free_dev(reinterpret_cast<void *&>(part));
-    free_dev(reinterpret_cast<void *&>(out));
+    if (e == hipSuccess && !rc) std::memcpy(sums, w.out, lbm::kTrackCols * sizeof(double));
     free_dev(reinterpret_cast<void *&>(ftmp));
     if (e != hipSuccess) return fail(-3, "%s: %s", what, hipGetErrorString(e));
     if (rc) return fail(-4, "%s: processing kernel failed (%d)", what, rc);
@@ -1754,6 +1771,7 @@ int lbm_expected_destroy(lbm_expected e) {
     if (!e) return 0;
     if (g_stream) (void)hipStreamSynchronize(g_stream);
     free_dev(reinterpret_cast<void *&>(e->d));
+    free_work(e->work);
     delete e;
     return 0;
 }
@@ -1782,7 +1800,7 @@ int lbm_track_errors(lbm_field f, lbm_expected e, const lbm_track_params *prm, d
     a.sfac = 1.0 / (prm->u_max * prm->u_max);
     a.u_old = nullptr;
     double s[lbm::kTrackCols];
-    if (int rc = track_sums(f, a, s, "lbm_track_errors")) return rc;
+    if (int rc = track_sums(f, a, e->work, s, "lbm_track_errors")) return rc;
     // the norms of the pushed row (track_hydrodynamic_errors.jl:205-221)
     out[0] = std::sqrt(s[lbm::kErrRho]);
     out[1] = std::sqrt(s[lbm::kErrU] / s[lbm::kTotU2]);
@@ -1815,6 +1833,7 @@ int lbm_velocity_tracker_destroy(lbm_velocity_tracker t) {
     if (!t) return 0;
     if (g_stream) (void)hipStreamSynchronize(g_stream);
     free_dev(reinterpret_cast<void *&>(t->d));
+    free_work(t->work);
     delete t;
     return 0;
 }
@@ -1829,7 +1848,10 @@ int lbm_velocity_stats(lbm_field f, lbm_velocity_tracker t, double *out5) {
     a.exp = nullptr;
     a.u_old = t ? t->d : nullptr;
     double s[lbm::kTrackCols];
-    if (int rc = track_sums(f, a, s, "lbm_velocity_stats")) return rc;
+    TrackWork once;  // a call without a tracker has no handle to keep it in
+    const int rc = track_sums(f, a, t ? t->work : once, s, "lbm_velocity_stats");
+    free_work(once);
+    if (rc) return rc;
     // u_mean /= divide_by (stopping_criteria.jl:39), divide_by = nx * ny
     const double nodes = (double)f->nx * (double)f->ny;
     out5[0] = s[lbm::kSumUx] / nodes;
