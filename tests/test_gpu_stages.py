@@ -1,10 +1,11 @@
 """Runs on the stencils that reach two or three nodes, several steps per pass
 (lbm_stage.h), against the oracle.
 
-The kernel writes 112 or 120 columns per block and at least 8 rows per chunk;
-the shapes sit at those edges: the smallest lattices it takes, one below, one
-block's columns and one more, lattices lower than a chunk's run-in, tall and
-long ones, and sizes of many blocks."""
+The pipeline runs from 0.12 to 0.4 million nodes up and writes 112 or 120
+columns per block and at least 8 rows per chunk.  The shapes sit at those
+edges: whole strips and one column more, ragged sizes, long and low lattices
+(17 rows: below three steps' run-in), tall and narrow ones; (300, 200) and
+(3001, 15) stay with single steps."""
 import numpy as np
 import pytest
 
@@ -13,11 +14,14 @@ from test_gpu_multi import _L, _model, _oracle, _populations
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(64, 16), (63, 40), (70, 15), (112, 64), (113, 65), (120, 90), (121, 17), (65, 1201),
-          (3001, 19), (517, 261)]
+SHAPES = [(672, 800), (841, 640), (1021, 517), (30001, 17), (224, 4001), (300, 200), (3001, 15)]
 
 
 def _bcs(name, nx, ny):
+    if name == "south":
+        return [dict(kind=0, direction=2, xs=(1, nx), ys=(1, ny))]
+    if name == "north":
+        return [dict(kind=1, direction=0, xs=(1, nx), ys=(1, ny), u=(0.04, 0.0), rho=1.0)]
     if name != "bands":
         return bc_dicts(name, nx, ny)
     # ranges narrower than the walls, a later condition over an earlier one
@@ -31,7 +35,8 @@ def _bcs(name, nx, ny):
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("coll,bcname,force,steps", [
     (0, "periodic", "none", 7), (1, "bands", "field", 8), (0, "couette", "const", 5),
-    (1, "poiseuille", "const", 2), (1, "cavity", "none", 3)])
+    (1, "poiseuille", "const", 2), (1, "cavity", "none", 3), (1, "south", "none", 6),
+    (0, "north", "const", 7)])
 def test_f64_bit_exact(oracle_lib, qid, shape, coll, bcname, force, steps):
     nx, ny = shape
     f0 = _populations(qid, nx, ny, seed=qid + coll)
@@ -49,7 +54,8 @@ def test_f64_bit_exact(oracle_lib, qid, shape, coll, bcname, force, steps):
 @pytest.mark.parametrize("qid", [13, 17, 21, 37])
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("coll,bcname,force,steps", [
-    (0, "periodic", "none", 7), (1, "bands", "field", 8), (1, "poiseuille", "const", 11)])
+    (0, "periodic", "none", 7), (1, "bands", "field", 8), (1, "poiseuille", "const", 11), (0, "south", "none", 7),
+    (1, "north", "none", 7)])
 def test_f32_error_no_larger_than_single_steps(oracle_lib, qid, shape, coll, bcname, force, steps):
     """Every step rounds as the single-step kernels do (which the per-launch
     timing entry point keeps): the populations' error against the oracle's
