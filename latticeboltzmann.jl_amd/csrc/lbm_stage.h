@@ -10,9 +10,9 @@
 // 2048 x 1024 nodes between two walls, SRT, us a step, single steps / pipeline:
 //   FP64: D2Q13 91 / 38, D2Q17 121 / 55, D2Q21 184 / 100, D2Q37 255 / 158;
 //   FP32: D2Q13 46 / 29, D2Q17 61 / 39, D2Q21 90 / 49, D2Q37 130 / 65.
-// D2Q37 FP64 moves 3.9 TB/s: its two steps take 830 FP64 instructions a row
-// each and the rings leave room for two waves per SIMD, so what bounds it is the
-// issue of those waves between the barriers, not memory.
+// D2Q37 FP64 moves 3.9 TB/s: a row and step takes 830 FP64 instructions, and the
+// rings leave room for two waves per SIMD, which wait 59 % of their cycles for
+// loads and at the barriers: latency bounds it, not the rate of memory.
 //
 // SUB = 2 (FP64): two sub-groups take a group's rows in turn, each row over two
 // iterations, which doubles the waves that the same rings feed: D2Q13 42.9 -> 40.7,
