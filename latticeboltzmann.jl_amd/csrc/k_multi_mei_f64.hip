@@ -13,7 +13,7 @@ template <int QID>
 __global__ void __launch_bounds__(256)
 k_mei_step(const double *__restrict__ C, double *__restrict__ Cn, const StepParams<double> p,
            const MeiStop stop) {
-    if (mei_stopped(stop.watch) != 0) return;
+    if (mei_done(stop)) return;
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y;
     if (x >= p.nx) return;

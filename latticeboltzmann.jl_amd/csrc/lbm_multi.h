@@ -277,8 +277,8 @@ __device__ __forceinline__ void collide_multi(T (&f)[QT<QID>::Q], const StepPara
 // (nx, ny)), taken on the device: the thread that holds the corner compares the
 // density of each new state with the previous one's and records the first step
 // that converged; launches after that return at once, so the state before it
-// is still in its buffer.  Blocks of the recording launch may or may not see
-// the record: its output is not used once the record is set.
+// is still in its buffer.  The output of the recording launch is not used once
+// the record is set.
 template <int QID, int... Is>
 __device__ __forceinline__ double mei_density(const double (&f)[QT<QID>::Q],
                                               std::integer_sequence<int, Is...>) {
@@ -288,6 +288,13 @@ __device__ __forceinline__ double mei_density(const double (&f)[QT<QID>::Q],
 }
 __device__ __forceinline__ long long mei_stopped(const MeiWatch *w) {
     return __hip_atomic_load(&w->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Whether an earlier launch recorded the stop: a launch records steps from its
+// own first one up, so every thread of a launch gets the same answer, whenever
+// its corner's thread records (k_tile has barriers after this).
+__device__ __forceinline__ bool mei_done(const MeiStop &m) {
+    const long long stop = mei_stopped(m.watch);
+    return stop != 0 && stop < m.step;
 }
 template <int QID>
 __device__ __forceinline__ void mei_check(const MeiStop &m, const double (&f)[QT<QID>::Q], long long step) {
@@ -423,7 +430,7 @@ tile_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *__
     static_assert(M == 1 && !ST::kNeq, "one-speed stencils, one value per population");
     __shared__ T buf[Q * N];
     if constexpr (COLL == 3)
-        if (a.mei.watch && mei_stopped(a.mei.watch) != 0) return;
+        if (a.mei.watch && mei_done(a.mei)) return;
     const int tile = tile_of_block(a);
     if (tile >= a.tiles) return;
     const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;

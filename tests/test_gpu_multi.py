@@ -283,3 +283,45 @@ def test_adjoint_passes(qid, shape, coll, T):
     tol = 64 * (T + 1) * 2.0 ** -24
     assert np.linalg.norm(r["grad_u0"] - ref["grad_u0"]) <= tol * np.linalg.norm(ref["grad_u0"])
     assert abs(r["loss"] - ref["loss"]) <= tol * ref["loss"]
+
+
+def _corner_changes(oracle_lib, qid, u, steps, bcs):
+    """|rho_t - rho_(t-1)| at node (nx, ny), t = 1 .. steps, rho_0 = 0"""
+    rho, out = 0.0, []
+    for t in range(1, steps + 1):
+        S, _, _ = oracle_lib.mei_initialize(qid, u, 0.8, 0.0, t, bcs)
+        r = S[-1, -1, 0] + S[-1, -1, 1]
+        for i in range(2, S.shape[2]):
+            r = r + S[-1, -1, i]
+        out.append(abs(r - rho))
+        rho = r
+    return out
+
+
+@pytest.mark.parametrize("qid,nx,ny", [(9, 33, 20), (9, 5, 7), (9, 168, 160), (9, 169, 160),
+                                       (5, 24, 31), (13, 40, 17)])
+@pytest.mark.parametrize("bcname", ["periodic", "couette"])
+def test_mei_stop_at_every_step_that_can_hold_it(oracle_lib, qid, nx, ny, bcname):
+    """The recording launch is run by all its threads to its end (it has
+    barriers), the ones after it by none: wherever in a launch the stop falls,
+    steps, f_stream and f_collision are the oracle's."""
+    x, y = np.meshgrid(np.arange(nx) * 2 * np.pi / nx, np.arange(ny) * 2 * np.pi / ny,
+                       indexing="ij")
+    u = np.asfortranarray(np.stack([0.03 * np.cos(x) * np.sin(y), 0.02 * np.sin(x + y)], axis=-1))
+    bcd = bc_dicts(bcname, nx, ny)
+    d = _corner_changes(oracle_lib, qid, u, 26, bcd)
+    low, at = d[0], [1]
+    for t in range(2, len(d) + 1):
+        if d[t - 1] < low:
+            at.append(t)
+            low = d[t - 1]
+    print(f"mei stops D2Q{qid} {nx}x{ny} {bcname}: {at}", flush=True)
+    assert len(at) > 1
+    for t in at:
+        eps = 1.5 * d[0] if t == 1 else 0.5 * (min(d[:t - 1]) + d[t - 1])
+        S, C, n = oracle_lib.mei_initialize(qid, u, 0.8, eps, 200, bcd)
+        assert n == t
+        s, c, steps = _mei_run(qid, u, to_lbmhip(bcd), eps, 200)
+        assert steps == t
+        assert np.array_equal(s, S)
+        assert np.array_equal(c, C)
