@@ -1887,6 +1887,7 @@ struct lbm_batch_s {
     int region_mode = -1;
     lbm::BatchRegion *dRegions = nullptr;
     int nregions = 0;
+    std::mutex stage_mu;       // one host transfer at a time
     double *dStage = nullptr;  // host transfers: dense FP64 rows
     size_t stage_doubles = 0;
     hipGraphExec_t gexec = nullptr;
@@ -2147,6 +2148,8 @@ static int batch_xfer(lbm_batch b, int k, int buf, double *host, bool up) {
     const size_t rows = (size_t)L.ny * b->q.Q, nx = (size_t)L.nx;
     const size_t fit = kStageMax / nx > 0 ? kStageMax / nx : 1;
     const size_t step = rows < fit ? rows : fit;
+    // held until the last copy has ended: threads may move different lattices
+    const std::lock_guard<std::mutex> lock(b->stage_mu);
     if (step * nx > b->stage_doubles) {
         free_dev(reinterpret_cast<void *&>(b->dStage));
         b->stage_doubles = 0;

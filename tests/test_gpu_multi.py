@@ -325,3 +325,29 @@ def test_mei_stop_at_every_step_that_can_hold_it(oracle_lib, qid, nx, ny, bcname
         assert steps == t
         assert np.array_equal(s, S)
         assert np.array_equal(c, C)
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32"])
+def test_batch_transfers_from_several_threads(storage):
+    """Threads that move different lattices of one batch at a time share its
+    transfer buffer, which grows with the lattice: every thread gets back what
+    it put in."""
+    from concurrent.futures import ThreadPoolExecutor
+    L = _L()
+    sizes = [(8 + 37 * k, 5 + 23 * k) for k in range(12)]
+    b = L.LatticeBatch(L.D2Q9(), sizes, [0.8] * len(sizes), None, storage=storage)
+    f = [_populations(9, nx, ny, seed=k) for k, (nx, ny) in enumerate(sizes)]
+    if storage == "f32":  # values that FP32 holds, as deviations from the weights too
+        w = np.asarray(L.D2Q9().weights)
+        dev = [np.round((x - w) * 2.0 ** 20) * 2.0 ** -20 for x in f]
+        f = [np.asfortranarray(w.astype(np.float32).astype(float) + d) for d in dev]
+
+    def move(k):
+        for _ in range(20):
+            b.upload(k, f[k])
+            for role in ("f_stream", "f_collision"):
+                np.testing.assert_allclose(b.download(k, role), f[k], rtol=0,
+                                           atol=0 if storage == "f64" else 2.0 ** -26)
+
+    with ThreadPoolExecutor(4) as pool:
+        list(pool.map(move, range(len(sizes))))
