@@ -212,8 +212,8 @@ int lbm_stream_bc(lbm_model m, lbm_field f, lbm_field f_new);
  * nsteps x (collide! f_stream -> f_collision; stream! + apply!) with fused pull
  * collide-stream kernels.  With the automatic launch shape, D2Q4/5/9 models in
  * storage F64, F32, F16NEQ or BF16NEQ advance several steps per kernel (the
- * 16-bit storages on even widths from 800,000 nodes up; they then round to 16
- * bits once per pass instead of once per step), and so do SRT and TRT models of
+ * 16-bit storages on even widths from 0.8 to 1.8 million nodes up, by their
+ * walls; they then round to 16 bits once per pass instead of once per step), and so do SRT and TRT models of
  * D2Q13/17/21/37 in F64 and F32 whose walls are north and south ones, from
  * 0.12 to 0.4 million nodes up; everything else runs one
  * kernel per step.  On return both buffers hold exactly what the reference's

@@ -512,6 +512,7 @@ int run(lbm::Op op, lbm_model m, lbm_field src, lbm_field dst, bool with_bcs) {
 struct MultiPlan {
     int kernel = lbm::kMultiNone;
     int max_steps = 1;
+    int min_steps = 2;  // shorter runs keep single steps
     // relative cost of a pass of k steps (0: not available), k = 1 the single-step kernel
     double cost[9] = {};
 };
@@ -527,8 +528,19 @@ struct MultiPlan {
 //   FP32: 64^2 4.0 -> 0.8; 257^2 4.5 -> 1.6; 512^2 6.0 -> 2.3; 1024^2 17.6 ->
 //     6.1 (march 7.6); 2048^2 64 -> 18 (blocks 20.5); 4096^2 218 -> 57;
 //   FP16-NEQ: 4096^2 194 -> 71 (two columns per lane: even widths).
-// (below this the 16-bit storages keep the single-step row kernel)
-constexpr long long kNeqMarchNodes = 800000;
+// Below this many nodes the 16-bit storages keep the single-step row kernel: a
+// small lattice is a round of few waves, whose serial chain of rows bounds a
+// pass, and a wave at a wall has the longest.  Runs of 41 steps, time over
+// single steps' by walls (none / north and south / east too), the worst of
+// D2Q4/5/9, SRT and TRT, FP16 and BF16: 1000 x 810 0.96 / 1.23 / 1.70,
+// 1400 x 1200 0.70 / 0.80 / 1.05, 2000 x 1500 0.55 / 0.57 / 0.74.  Two steps:
+// 1.12 / 1.20 / 1.32, 1.01 / 1.08 / 1.15, 0.88 / 0.88 / 0.93; they need twice
+// the nodes.  The row kernel wastes most of its lanes below 256 columns: 64 x
+// 19000 0.28 without walls, 0.30 with north and south ones.
+long long neq_march_nodes(int nx, int walls) {
+    if (nx < 256 || !walls) return 800000;
+    return walls & (1 << LBM_EAST | 1 << LBM_WEST) ? 1800000 : 1200000;
+}
 
 // The register-block kernels: a pass takes a + b per further round of 256
 // blocks (one per CU), by its steps; microseconds, D2Q9 TRT, measured on 100^2
@@ -655,7 +667,11 @@ MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     // columns: blocks 7 us against 10 for 270,000 nodes; at 24 they lose)
     const bool wide = f->nx >= 32 && f->ny >= 12;
     if (rows_mode(f->storage)) {
-        if (f->nx % 2 || f->nx < 64 || !wide || nodes < kNeqMarchNodes) return pl;
+        int walls = 0;
+        for (const auto &b : m->bcs) walls |= 1 << b.direction;
+        const long long least = neq_march_nodes(f->nx, walls);
+        if (f->nx % 2 || f->nx < 64 || !wide || nodes < least) return pl;
+        if (nodes < 2 * least || f->nx < 256) pl.min_steps = 3;
         pl.kernel = lbm::kMultiMarch;
         pl.max_steps = 4;
         const double c[5] = {0, 194, 226, 254, 285};
@@ -1233,7 +1249,7 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
     // Runs that time every launch keep one fused step per launch; the others
     // advance several collisions per pass where a kernel for it exists.
     const MultiPlan plan = per_launch ? MultiPlan{} : multi_plan(m, S);
-    const bool multi = plan.kernel != lbm::kMultiNone && nsteps >= 2;
+    const bool multi = plan.kernel != lbm::kMultiNone && nsteps >= plan.min_steps;
     // step 1 starts from the canonical state S: the first pass collides S_0 in
     // place.  Without a several-step kernel, one-speed stencils on lattices of
     // whole 64 x 8 tiles take C_1 = collide(BC(stream(collide(S_0)))) in one

@@ -336,12 +336,13 @@ __device__ __forceinline__ bool at_wall(const StepParams<T> &p, int walls, int x
 }
 
 template <int QID, class T>
-__device__ __forceinline__ unsigned bc_mask(const StepParams<T> &p, int walls, int x, int y) {
+__device__ __forceinline__ unsigned bc_mask(const StepParams<T> &p, const BCDev *bcs, int walls, int x,
+                                            int y) {
     static_assert(QT<QID>::MAXC == 1 && QT<QID>::Q <= 16, "one-speed stencils");
     unsigned m = 0;
     if (at_wall(p, walls, x, y)) {
         for (int b = 0; b < p.nbc; ++b) {
-            const BCDev bc = p.bcs[b];
+            const BCDev bc = bcs[b];
             const bool at = bc.dir == 0   ? y == p.ny - 1
                             : bc.dir == 1 ? x == p.nx - 1
                             : bc.dir == 2 ? y == 0
@@ -445,7 +446,7 @@ tile_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *__
         const int ux = tx * TX - SH::H + hx, uy = ty * TY - SH::H + hy;
         xs[k] = wrap(ux, p.nx);
         ys[k] = wrap(uy, p.ny);
-        bcm[k] = BC ? bc_mask<QID>(p, a.wall.walls, xs[k], ys[k]) : 0u;
+        bcm[k] = BC ? bc_mask<QID>(p, p.bcs, a.wall.walls, xs[k], ys[k]) : 0u;
         // distance outside the tile (0 inside): level l needs ring <= levels - l
         const int dx = max(SH::H - hx, hx - (SH::H + TX - 1)), dy = max(SH::H - hy, hy - (SH::H + TY - 1));
         ring[k] = n < N ? max(0, max(dx, dy)) : TMAX;
@@ -650,7 +651,7 @@ block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *_
         ys[j] = __builtin_amdgcn_readfirstlane(wrap(cy0 - h + row0 + j, p.ny));
     unsigned bcm[R];
 #pragma unroll
-    for (int j = 0; j < R; ++j) bcm[j] = BC ? bc_mask<QID>(p, wall.walls, x, ys[j]) : 0u;
+    for (int j = 0; j < R; ++j) bcm[j] = BC ? bc_mask<QID>(p, p.bcs, wall.walls, x, ys[j]) : 0u;
     V g[R][Q];
     const bool mine_x = ux >= cx0 && ux < min(cx0 + outx, p.nx);
     // row j of a level to `dst`, where this block owns it
@@ -870,6 +871,13 @@ k_march(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
     constexpr int Q = QT<QID>::Q, COLS = SH::COLS + 2 * NC, LINES = SH::LINES;
     static_assert(QT<QID>::MAXC == 1, "one-speed stencils");
     __shared__ V rows[4][LINES][SH::LINE][COLS];
+    // The boundary list: a row that walks it must not wait for the next row's
+    // loads and the stores in flight, as reads of memory would.
+    __shared__ BCDev list[BC ? kMaxBC : 1];
+    if constexpr (BC) {
+        if ((int)threadIdx.x < p.nbc) list[threadIdx.x] = p.bcs[threadIdx.x];
+        __syncthreads();
+    }
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int wave = (int)blockIdx.x * 4 + wv;
@@ -890,6 +898,23 @@ k_march(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
     // LDS element of the lane's first column and of its neighbours' (rows are
     // padded by NC at both ends: what the end lanes read there is halo)
     const int e0 = lane * NC + NC, em = e0 - 1, ep = e0 + 1;
+    // A column's mask changes from row to row only where the lattice or a
+    // condition's range begins or ends: it is formed there (row mask_next, and
+    // row 0) and kept in between.  Formed at every row, an east or west column
+    // held its wave up by some 4,000 cycles a row.
+    int mask_next = -1;
+    unsigned mask[NC];
+    auto masks = [&](int y) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) mask[c] = bc_mask<QID>(p, list, a.wall.walls, xs[c], y);
+        int next = y < 1 ? 1 : (y < p.ny - 1 ? p.ny - 1 : p.ny);
+        for (int b = 0; b < p.nbc; ++b) {
+            const int lo = list[b].y0, hi = list[b].y1 + 1;
+            if (lo > y && lo < next) next = lo;
+            if (hi > y && hi < next) next = hi;
+        }
+        mask_next = __builtin_amdgcn_readfirstlane(next);
+    };
     // boundary masks of the row each level holds: they move down with the rows
     unsigned bcm[LINES + 1][NC];
 #pragma unroll
@@ -950,11 +975,12 @@ k_march(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
         r = __builtin_amdgcn_readfirstlane(r + 1 == p.ny ? 0 : r + 1);
         if (k + 1 < iters) fetch(r);
         if constexpr (BC) {
+            if (k == 0 || rl == 0 || rl == mask_next) masks(rl);
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
 #pragma unroll
                 for (int l = LINES; l > 0; --l) bcm[l][c] = bcm[l - 1][c];
-                bcm[0][c] = bc_mask<QID>(p, a.wall.walls, xs[c], rl);
+                bcm[0][c] = mask[c];
             }
         }
         if (SH::SHIFTED || a.first) {

@@ -351,3 +351,53 @@ def test_batch_transfers_from_several_threads(storage):
 
     with ThreadPoolExecutor(4) as pool:
         list(pool.map(move, range(len(sizes))))
+
+
+def _ranged_walls(nx, ny):
+    """East and west walls whose ranges begin and end at rows all over the
+    lattice, one row long too, a later condition over an earlier one."""
+    return [dict(kind=0, direction=1, xs=(1, nx), ys=(min(7, ny), max(min(7, ny), ny // 3))),
+            dict(kind=0, direction=1, xs=(1, nx), ys=(ny // 2, ny // 2)),
+            dict(kind=0, direction=3, xs=(1, nx), ys=(ny // 2, ny)),
+            dict(kind=0, direction=3, xs=(1, nx), ys=(1, 1)),
+            dict(kind=1, direction=0, xs=(1, nx), ys=(1, ny), u=(0.05, 0.0), rho=1.0),
+            dict(kind=0, direction=0, xs=(nx // 2, nx), ys=(2, ny)),
+            dict(kind=0, direction=2, xs=(2, nx // 3), ys=(1, ny))]
+
+
+@pytest.mark.parametrize("shape", [(2049, 1500), (47, 65001), (250001, 12)])
+@pytest.mark.parametrize("coll,steps", [(0, 5), (1, 13)])
+def test_march_ranged_walls_f64_bit_exact(oracle_lib, shape, coll, steps):
+    nx, ny = shape
+    f0 = _populations(9, nx, ny, seed=17)
+    q, cm, taus = _model(9, coll, None)
+    bcs = _ranged_walls(nx, ny)
+    model = _L().LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs))
+    print(f"march ranges {nx}x{ny} coll {coll} {steps} steps", flush=True)
+    _L().simulate(model, range(steps))
+    S, C = _oracle(oracle_lib, 9, f0, coll, taus, steps, None, bcs)
+    assert np.array_equal(model.f_stream.to_numpy(), S)
+    assert np.array_equal(model.f_collision.to_numpy(), C)
+
+
+@pytest.mark.parametrize("storage", ["f16neq", "bf16neq"])
+@pytest.mark.parametrize("qid", [4, 9])
+@pytest.mark.parametrize("shape,bcname", [((1500, 1204), "ranged"), ((1500, 1204), "cavity"),
+                                          ((1202, 1000), "couette"), ((64, 19001), "ranged"),
+                                          ((150002, 12), "partial")])
+def test_march_walls_neq_error_no_larger_than_single_steps(oracle_lib, storage, qid, shape, bcname):
+    """as test_neq_error_no_larger_than_single_steps, on lattices that their
+    walls leave to the several-step kernel"""
+    L = _L()
+    nx, ny = shape
+    f0 = _populations(qid, nx, ny, seed=7, noise=1e-4)
+    q, cm, taus = _model(qid, 1, None)
+    bcs = _ranged_walls(nx, ny) if bcname == "ranged" else bc_dicts(bcname, nx, ny)
+    many = L.LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs), storage=storage)
+    L.simulate(many, range(9))
+    one = L.LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs), storage=storage)
+    L.simulate_launch_times(one, 9)
+    S, C = _oracle(oracle_lib, qid, f0, 1, taus, 9, None, bcs)
+    for a, b, ref in ((many.f_stream, one.f_stream, S), (many.f_collision, one.f_collision, C)):
+        ea, eb = (np.linalg.norm(x.to_numpy() - ref) for x in (a, b))
+        assert ea <= 1.1 * eb, (ea, eb)
