@@ -638,6 +638,12 @@ MultiPlan plan_stages(const lbm_model_s *m, const lbm_field_s *f) {
     return pl;
 }
 
+// k_fused_first*: the first step of a run in one pass, collide! included
+bool first_in_one_pass(const lbm_model_s *m, const lbm_field_s *f) {
+    return (m->qid == 4 || m->qid == 5 || m->qid == 9) && f->nx % 64 == 0 && f->ny % 8 == 0 &&
+           (m->coll <= LBM_TRT || (f->storage == LBM_STORE_F64 && m->coll == LBM_MRT));
+}
+
 MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     MultiPlan pl;
     if (m->launch_block || m->launch_rows || m->launch_vec || m->launch_nt >= 0) {
@@ -700,6 +706,14 @@ MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
         const double c32[7] = {0, 218, 260, 280, 295, 0, 341};
         for (int k = 1; k <= pl.max_steps; ++k) pl.cost[k] = f64 ? c64[k] : c32[k];
     }
+    // A run of two steps is one pass and a stream either way where single steps
+    // can begin in one pass; that pass is the faster one on large lattices and
+    // on narrow or low ones (time of two steps over the single-step kernels',
+    // D2Q4/5/9: 4096^2 1.01 to 1.15, FP32 64 x 8000 1.07 to 1.24, 6400 x 64 1.02
+    // to 1.11, FP64 0.92 to 1.15; 1536 x 1024 0.84 to 0.98).
+    if (pl.kernel != lbm::kMultiTile && first_in_one_pass(m, f) &&
+        (nodes > 8000000 || f->nx < 128 || f->ny < 128))
+        pl.min_steps = 3;
     return pl;
 }
 
@@ -1256,10 +1270,7 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
     // pass (k_fused_first*); otherwise C_0 = collide(S_0) first.  Runs that
     // time every launch keep the two-pass start, so that their launches are
     // all of one kernel.
-    const bool first_fused =
-        nsteps >= 2 && !per_launch && !multi && (m->qid == 4 || m->qid == 5 || m->qid == 9) &&
-        S->nx % 64 == 0 && S->ny % 8 == 0 &&
-        (m->coll <= LBM_TRT || (S->storage == LBM_STORE_F64 && m->coll == LBM_MRT));
+    const bool first_fused = nsteps >= 2 && !per_launch && !multi && first_in_one_pass(m, S);
     int64_t k_first = 1;  // collisions done by the first pass
     if (multi && multi_next(plan, nsteps) > 1) {
         k_first = multi_next(plan, nsteps);

@@ -401,3 +401,11 @@ def test_march_walls_neq_error_no_larger_than_single_steps(oracle_lib, storage, 
     for a, b, ref in ((many.f_stream, one.f_stream, S), (many.f_collision, one.f_collision, C)):
         ea, eb = (np.linalg.norm(x.to_numpy() - ref) for x in (a, b))
         assert ea <= 1.1 * eb, (ea, eb)
+
+
+@pytest.mark.parametrize("shape", [(64, 8000), (6400, 64), (4096, 2048), (128, 8000)])
+@pytest.mark.parametrize("coll,bcname", [(1, "periodic"), (2, "cavity")])
+def test_two_steps_on_whole_tiles_f64_bit_exact(oracle_lib, shape, coll, bcname):
+    """a run of two steps keeps the single-step kernels' one-pass start on
+    large lattices and on narrow or low ones"""
+    _check_f64(oracle_lib, 9, coll, *shape, bcname, "const", 2)
