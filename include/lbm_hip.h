@@ -184,15 +184,17 @@ int lbm_model_set_bcs(lbm_model m, const lbm_bc *bcs, int n);
  * distinct Hermite components; periodic lattices with nx a multiple of 16,
  * other cases return an error; parity with the oracle to 1e-12 relative
  * instead of bit for bit).  It is opt-in: on MI355X it is slower than the
- * default vector kernel.  A shape other than the automatic one also selects
- * one fused step per launch (lbm_simulate).  No counterpart in the reference
- * (a CPU loop has no launch shape). */
+ * default vector kernel.  Setting a shape also selects one fused step per
+ * launch (lbm_simulate); with nontemporal < 0, the automatic numbers (0, or as
+ * lbm_autotune returns them) do not.  No counterpart in the reference (a CPU
+ * loop has no launch shape). */
 int lbm_model_set_launch(lbm_model m, int block_x, int rows_per_block, int nodes_per_thread,
                          int nontemporal);
 /* Autotuner: times every launch shape of the fused step for this model, and
  * the several-step kernels where lbm_simulate has them, on scratch copies of
  * f_stream (the caller's fields are not advanced), keeps the fastest in the
- * model and returns it (the automatic shape for the several-step kernels).  No counterpart in the reference. */
+ * model and returns it: for the several-step kernels the automatic numbers with
+ * *nontemporal = -1.  No counterpart in the reference. */
 int lbm_autotune(lbm_model m, lbm_field f_stream, int trial_steps, int *block_x,
                  int *rows_per_block, int *nodes_per_thread, int *nontemporal,
                  double *us_per_step);

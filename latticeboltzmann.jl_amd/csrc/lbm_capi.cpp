@@ -646,15 +646,17 @@ bool first_in_one_pass(const lbm_model_s *m, const lbm_field_s *f) {
 
 MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     MultiPlan pl;
-    if (m->launch_block || m->launch_rows || m->launch_vec || m->launch_nt >= 0) {
-        // a shape set by the caller names a single-step kernel, unless it is
-        // the automatic one (what lbm_autotune returns when this path wins)
+    // A shape set by the caller names a single-step kernel, with the automatic
+    // numbers too.  Only those numbers with the store kind left automatic are
+    // no shape of their own: lbm_autotune returns them when this path wins.
+    if (m->launch_nt >= 0) return pl;
+    if (m->launch_block || m->launch_rows || m->launch_vec) {
         lbm_model_s def;
         def.coll = m->coll;
-        int b, r, v, nt, b0, r0, v0, nt0;
+        int b, r, v, nt, b0, r0, v0;
         auto_launch(m, f, b, r, v, nt);
-        auto_launch(&def, f, b0, r0, v0, nt0);
-        if (b != b0 || r != r0 || v != v0 || nt != nt0) return pl;
+        auto_launch(&def, f, b0, r0, v0, nt);
+        if (b != b0 || r != r0 || v != v0) return pl;
     }
     if (m->qid != 4 && m->qid != 5 && m->qid != 9) return plan_stages(m, f);
     if (m->coll != LBM_SRT && m->coll != LBM_TRT &&
@@ -1426,6 +1428,7 @@ int lbm_autotune(lbm_model m, lbm_field f_stream, int trial_steps, int *block_x,
         }
     }
     // the several-step kernels (automatic shape): kept by returning that shape
+    // with the store kind automatic (see multi_plan)
     if (!rc) {
         m->launch_block = m->launch_rows = m->launch_vec = 0;
         m->launch_nt = -1;
@@ -1447,6 +1450,7 @@ int lbm_autotune(lbm_model m, lbm_field f_stream, int trial_steps, int *block_x,
             if (!rc && us < best) {
                 best = us;
                 auto_launch(m, A, bb, br, bv, bn);
+                bn = -1;
             }
         }
     }

@@ -163,9 +163,11 @@ def simulate_timed(model: LatticeBoltzmannModel, nsteps: int):
 
 
 def autotune(model: LatticeBoltzmannModel, trial_steps: int = 20) -> dict:
-    """Time every launch shape of the fused step on scratch copies of the
-    model's lattice (the model state is not advanced), keep the fastest in
-    ``model.launch`` and return it with its time per step."""
+    """Time every launch shape of the fused step, and the several-step kernels
+    where there are some, on scratch copies of the model's lattice (the model
+    state is not advanced), keep the fastest in ``model.launch`` and return it
+    with its time per step.  ``nontemporal`` is -1 for the several-step kernels:
+    the other numbers are the automatic ones then."""
     import ctypes
 
     m = native_model(model.quadrature).configure(model.collision_model, model.f_stream,

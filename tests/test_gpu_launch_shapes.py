@@ -1,0 +1,51 @@
+"""Which kernels a run takes by its launch shape: a shape set by the caller
+means one fused step per launch, the automatic setting several steps per pass.
+
+FP32 TRT on D2Q9 tells the two apart: the several-step kernels round a step
+differently.  ``simulate_launch_times`` runs one step per launch whatever the
+shape."""
+import numpy as np
+import pytest
+
+from lbm_cases import random_populations
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(shape, launch, steps, times=False):
+    import lbmhip as L
+    f0 = random_populations(9, *shape, seed=3, noise=1e-2)
+    m = L.LatticeBoltzmannModel.from_populations(L.D2Q9(), f0, L.TRT.fields(0.7, 1.3),
+                                                 storage="f32")
+    m.launch = launch
+    if times:
+        L.simulate_launch_times(m, steps)
+    else:
+        L.simulate(m, range(steps))
+    return m.f_stream.to_numpy()
+
+
+@pytest.mark.parametrize("shape", [(100, 90), (300, 250)])
+def test_a_shape_set_to_the_automatic_numbers_runs_single_steps(shape):
+    several = _run(shape, None, 9)
+    for launch in ((256, 1, 1, 1), (256, 1, 1, 0), (0, 0, 0, 1), (128, 1, 1, -1)):
+        single = _run(shape, launch, 9, times=True)
+        assert not np.array_equal(single, several)
+        assert np.array_equal(_run(shape, launch, 9), single), launch
+    for launch in ((0, 0, 0, -1), (256, 1, 1, -1)):
+        assert np.array_equal(_run(shape, launch, 9), several), launch
+
+
+@pytest.mark.parametrize("shape", [(100, 90), (300, 250)])
+def test_autotune_result_names_the_kernel_it_timed(shape):
+    import lbmhip as L
+    f0 = random_populations(9, *shape, seed=3, noise=1e-2)
+    m = L.LatticeBoltzmannModel.from_populations(L.D2Q9(), f0, L.TRT.fields(0.7, 1.3),
+                                                 storage="f32")
+    best = L.autotune(m, trial_steps=20)
+    L.simulate(m, range(9))
+    several = _run(shape, None, 9)
+    want = several if best["nontemporal"] < 0 else _run(shape, m.launch, 9, times=True)
+    assert np.array_equal(m.f_stream.to_numpy(), want)
+    # applied to another model
+    assert np.array_equal(_run(shape, m.launch, 9), want)
