@@ -255,20 +255,24 @@ int lbm_batch_upload(lbm_batch b, int k, const double *f);
 int lbm_batch_download(lbm_batch b, int k, int role, double *f);
 /* launch shape of the single-step kernel: threads per tile-block (64, 128,
  * 256; 0 = 128) and grid size (0 = one block per tile; smaller grids make the
- * blocks stride over the tile table).  The default, and again after (0, 0)
- * with one node per thread, is automatic: several steps per pass over blocks
+ * blocks stride over the tile table).  The default, and again after (0, 0) or
+ * with grid LBM_BATCH_GRID_AUTO and one node per thread, is automatic: several
+ * steps per pass over blocks
  * of 64 x 24 (FP64) or 64 x 32 (FP32) nodes, unless the lattices are much
  * smaller than such a block.  Results are the same bits in FP64; in FP32 the
  * passes round like lbm_simulate's. */
+#define LBM_BATCH_GRID_AUTO 0x7fffffff
 int lbm_batch_set_launch(lbm_batch b, int block, int grid);
 /* nodes per thread of the batch kernel (1, 2 or 4; default 1): a tile holds
  * block x nodes consecutive nodes of one lattice, a lane nodes of them that
  * lie block apart */
 int lbm_batch_set_nodes_per_thread(lbm_batch b, int nodes);
-/* the launch shape in use (after lbm_batch_autotune: the fastest one);
- * any output may be NULL */
+/* the launch shape in use (after lbm_batch_autotune: the fastest one), to be
+ * set again with the functions above: the automatic setting is block 128,
+ * grid LBM_BATCH_GRID_AUTO, one node per thread.  Any output may be NULL */
 int lbm_batch_get_launch(lbm_batch b, int *block, int *grid, int *nodes_per_thread);
-/* times launch shapes on the batch (state saved and restored), keeps the fastest */
+/* times launch shapes on the batch (state saved and restored), keeps the fastest
+ * and returns it (*grid = LBM_BATCH_GRID_AUTO for the several-step passes) */
 int lbm_batch_autotune(lbm_batch b, int trial_steps, int *block, int *grid, double *us_per_step);
 /* nsteps of every lattice; graph_chunk > 0 replays runs of graph_chunk fused
  * steps from one captured hipGraph (0: direct launches; several steps per

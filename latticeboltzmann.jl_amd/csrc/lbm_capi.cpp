@@ -2231,9 +2231,10 @@ int lbm_batch_set_launch(lbm_batch b, int block, int grid) {
     if (block != 0 && block != 64 && block != 128 && block != 256)
         return fail(-1, "block must be 0 (automatic), 64, 128 or 256");
     if (grid < 0) return fail(-1, "grid must be >= 0");
-    b->block = block ? block : 128;
-    b->grid = grid;
-    b->explicit_shape = block != 0 || grid != 0;
+    const bool automatic = grid == LBM_BATCH_GRID_AUTO || (block == 0 && grid == 0);
+    b->block = block && !automatic ? block : 128;
+    b->grid = automatic ? 0 : grid;
+    b->explicit_shape = !automatic;
     return 0;
 }
 
@@ -2248,7 +2249,7 @@ int lbm_batch_set_nodes_per_thread(lbm_batch b, int nodes) {
 int lbm_batch_get_launch(lbm_batch b, int *block, int *grid, int *nodes_per_thread) {
     if (!b) return fail(-1, "null batch");
     if (block) *block = b->block;
-    if (grid) *grid = b->grid;
+    if (grid) *grid = b->explicit_shape || b->vec != 1 ? b->grid : LBM_BATCH_GRID_AUTO;
     if (nodes_per_thread) *nodes_per_thread = b->vec;
     return 0;
 }
@@ -2375,9 +2376,8 @@ int lbm_batch_autotune(lbm_batch b, int trial_steps, int *block, int *grid, doub
             best = us;
             multi = true;
             bb = 128;
+            bg = 0;
             bv = 1;
-            rc = batch_tiles(b, bb * bv);
-            bg = b->ntiles;
         }
     }
     if (!rc) rc = lbm_field_copy_raw(b->pool, save, b->pool_bytes);
@@ -2395,8 +2395,7 @@ int lbm_batch_autotune(lbm_batch b, int trial_steps, int *block, int *grid, doub
     b->block = bb;
     b->grid = bg;
     b->vec = bv;
-    if (block) *block = bb;
-    if (grid) *grid = bg;
+    (void)lbm_batch_get_launch(b, block, grid, nullptr);
     if (us_per_step) *us_per_step = best;
     return 0;
 }

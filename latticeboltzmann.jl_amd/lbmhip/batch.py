@@ -1,7 +1,8 @@
 """Batches of independent periodic lattices advanced together.
 
-Every time step of every lattice is one persistent kernel launch over a tile
-table; runs of fused steps replay a captured hipGraph.  Each lattice follows
+Every launch advances all lattices, by several time steps over a table of blocks
+or, with a launch shape set, by one over a table of tiles, where runs of fused
+steps replay a captured hipGraph.  Each lattice follows
 simulate(model, time) (src/lattice_boltzmann_model.jl:60-77) exactly as a
 single-lattice model does; the batch has no counterpart in the reference.
 """
@@ -14,6 +15,9 @@ import numpy as np
 
 from . import _lib
 from .quadratures import Quadrature
+
+
+GRID_AUTO = 0x7fffffff  # LBM_BATCH_GRID_AUTO (include/lbm_hip.h)
 
 
 class LatticeBatch:
@@ -62,8 +66,9 @@ class LatticeBatch:
                        "lbm_batch_set_nodes_per_thread")
 
     def launch(self) -> dict:
-        """The launch shape in use: threads per block, grid (0 = one block per
-        tile) and nodes per thread."""
+        """The launch shape in use, as set_launch takes it: threads per block,
+        grid (0 = one block per tile, GRID_AUTO: the automatic setting) and
+        nodes per thread."""
         b, g, v = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         _lib.check(_lib.lib().lbm_batch_get_launch(self._h, ctypes.byref(b), ctypes.byref(g),
                                                    ctypes.byref(v)), "lbm_batch_get_launch")

@@ -49,3 +49,54 @@ def test_autotune_result_names_the_kernel_it_timed(shape):
     assert np.array_equal(m.f_stream.to_numpy(), want)
     # applied to another model
     assert np.array_equal(_run(shape, m.launch, 9), want)
+
+
+SIZES = [(200, 100), (64, 64), (90, 70), (130, 48)]
+
+
+def _batch():
+    import lbmhip as L
+    b = L.LatticeBatch(L.D2Q9(), SIZES, [0.7] * len(SIZES), [1.3] * len(SIZES), storage="f32")
+    for k, shape in enumerate(SIZES):
+        b.upload(k, random_populations(9, *shape, seed=k, noise=1e-2))
+    return b
+
+
+def _batch_run(launch):
+    b = _batch()
+    if launch is not None:
+        b.set_launch(launch["block"], launch["grid"], launch["nodes_per_thread"])
+    b.simulate(9)
+    return b, [b.download(k) for k in range(len(b))]
+
+
+def _equal(a, b):
+    return all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def test_batch_shape_read_and_set_again_names_the_same_kernel():
+    """the automatic setting, shapes with its numbers, and what the autotuner
+    returns"""
+    auto, several = _batch_run(None)
+    tiles = sum(-(-(-(-nx // 32) * 32 * ny) // 128) for nx, ny in SIZES)
+    shapes = [dict(block=128, grid=0, nodes_per_thread=1),
+              dict(block=128, grid=tiles, nodes_per_thread=1)]
+    single = _batch_run(shapes[0])[1]
+    assert not _equal(single, several)
+    assert _equal(_batch_run(auto.launch())[1], several)
+    for s in shapes:
+        b, got = _batch_run(s)
+        assert b.launch() == s
+        assert _equal(got, single), s
+    b = _batch()
+    best = b.autotune(5)
+    shape = {k: best[k] for k in ("block", "grid", "nodes_per_thread")}
+    b.simulate(9)
+    assert b.launch() == shape
+    got = [b.download(k) for k in range(len(b))]
+    import lbmhip.batch as batch
+    assert _equal(got, several if best["grid"] == batch.GRID_AUTO else single)
+    again, same = _batch_run(shape)
+    assert again.launch() == shape and _equal(same, got)
+    again.set_launch(0, 0)
+    assert again.launch() == auto.launch()
