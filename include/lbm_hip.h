@@ -222,12 +222,20 @@ int lbm_stream_bc(lbm_model m, lbm_field f, lbm_field f_new);
  * model.f_stream / model.f_collision hold. */
 int lbm_simulate(lbm_model m, lbm_field f_stream, lbm_field f_collision, int64_t nsteps);
 /* As lbm_simulate, also returning the time of the fused kernels (HIP events on
- * the library stream): *ms_total over the fused launches of the run after the
- * first, *nlaunch the number of steps they advance (nsteps less the steps of
- * the first pass, which starts from the canonical state: one, or as many as a
- * several-step pass holds). */
+ * the library stream): *ms_total over the fused launches of the run, *nlaunch
+ * the number of fused steps they advance.  A first pass of several steps is
+ * among them (nsteps - 1 steps in all, and the collide! that begins the run);
+ * single steps are timed after the first launch, which is collide! (nsteps - 1)
+ * or, on D2Q4/5/9 lattices of whole 64 x 8 tiles, collide! and the first fused
+ * step (nsteps - 2). */
 int lbm_simulate_timed(lbm_model m, lbm_field f_stream, lbm_field f_collision, int64_t nsteps,
                        double *ms_total, int64_t *nlaunch);
+/* Measurement support; no counterpart in the reference; needs no GPU.  What a run
+ * of nsteps does with the automatic launch shape: *kernel names the kernel that
+ * advances several steps per pass ("" for one step per launch), *passes is the
+ * number of launches that lbm_simulate_timed times. */
+int lbm_simulate_plan(int quadrature, int storage, int collision, int nx, int ny, const lbm_bc *bcs,
+                      int nbc, int64_t nsteps, const char **kernel, int64_t *passes);
 /* Measurement support; no counterpart in the reference.  As lbm_simulate with
  * one fused step per launch and a HIP event before every fused launch: launch_ms[k] (nsteps - 1
  * entries) is the time from the start of fused launch k to the start of the

@@ -737,6 +737,11 @@ int multi_next(const MultiPlan &pl, int64_t left) {
     return pass[left];
 }
 
+// whether a run of nsteps advances several steps per pass
+bool runs_multi(const MultiPlan &pl, int64_t nsteps) {
+    return pl.kernel != lbm::kMultiNone && nsteps >= pl.min_steps;
+}
+
 void boundary_walls(const lbm_model_s *m, lbm::MultiLaunch &L) {
     for (size_t b = 0; b < m->bcs.size(); ++b) {
         L.walls |= 1 << m->bcs[b].direction;
@@ -1265,7 +1270,7 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
     // Runs that time every launch keep one fused step per launch; the others
     // advance several collisions per pass where a kernel for it exists.
     const MultiPlan plan = per_launch ? MultiPlan{} : multi_plan(m, S);
-    const bool multi = plan.kernel != lbm::kMultiNone && nsteps >= plan.min_steps;
+    const bool multi = runs_multi(plan, nsteps);
     // step 1 starts from the canonical state S: the first pass collides S_0 in
     // place.  Without a several-step kernel, one-speed stencils on lattices of
     // whole 64 x 8 tiles take C_1 = collide(BC(stream(collide(S_0)))) in one
@@ -1274,8 +1279,17 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
     // all of one kernel.
     const bool first_fused = nsteps >= 2 && !per_launch && !multi && first_in_one_pass(m, S);
     int64_t k_first = 1;  // collisions done by the first pass
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (ms) {
+        HIP_TRY(hipEventCreate(&e0));
+        HIP_TRY(hipEventCreate(&e1));
+    }
+    // a first pass of several steps holds all fused steps of a short run: timed
+    bool timing = false;
     if (multi && multi_next(plan, nsteps) > 1) {
         k_first = multi_next(plan, nsteps);
+        if (ms) HIP_TRY(hipEventRecord(e0, g_stream));
+        timing = true;
         if (int rc = run_multi(plan, m, S, C, (int)k_first, true)) return rc;
     } else if (first_fused) {
         if (int rc = run(lbm::Op::FusedFirst, m, S, C, true)) return rc;
@@ -1283,12 +1297,7 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
     } else {
         if (int rc = run(lbm::Op::Collide, m, S, C, false)) return rc;
     }
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (ms) {
-        HIP_TRY(hipEventCreate(&e0));
-        HIP_TRY(hipEventCreate(&e1));
-        HIP_TRY(hipEventRecord(e0, g_stream));
-    }
+    if (ms && !timing) HIP_TRY(hipEventRecord(e0, g_stream));
     // per-launch events (measurement runs only): one before every fused launch
     std::vector<hipEvent_t> ev;
     if (per_launch) {
@@ -1338,7 +1347,7 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
         float t = 0.0f;
         HIP_TRY(hipEventElapsedTime(&t, e0, e1));
         *ms = (double)t;
-        if (nlaunch) *nlaunch = nsteps - k_first;
+        if (nlaunch) *nlaunch = nsteps - (timing ? 1 : k_first);
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
     }
@@ -1495,6 +1504,44 @@ int lbm_simulate_timed(lbm_model m, lbm_field f_stream, lbm_field f_collision, i
     if (ms_total) *ms_total = ms;
     if (nlaunch) *nlaunch = nl;
     return rc;
+}
+
+int lbm_simulate_plan(int quadrature, int storage, int collision, int nx, int ny, const lbm_bc *bcs,
+                      int nbc, int64_t nsteps, const char **kernel, int64_t *passes) {
+    if (kernel) *kernel = "";
+    if (passes) *passes = 0;
+    HostQuad q;
+    if (!host_quad(quadrature, q)) return fail(-1, "unknown quadrature D2Q%d", quadrature);
+    if (!storage_bytes(storage)) return fail(-1, "unknown storage %d", storage);
+    if (collision != LBM_SRT && collision != LBM_TRT && collision != LBM_MRT)
+        return fail(-1, "unknown collision model %d", collision);
+    if (nx < 1 || ny < 1) return fail(-1, "lattice size must be positive");
+    if (nbc < 0 || nbc > lbm::kMaxBC || (nbc > 0 && !bcs))
+        return fail(-1, "0 to %d boundary conditions", lbm::kMaxBC);
+    if (nsteps < 0) return fail(-1, "negative step count");
+    lbm_model_s m;
+    m.qid = quadrature;
+    m.coll = collision;
+    m.bcs.assign(bcs, bcs + nbc);
+    lbm_field_s f;
+    f.qid = quadrature;
+    f.nx = nx;
+    f.ny = ny;
+    f.Q = q.Q;
+    f.storage = storage;
+    const MultiPlan plan = multi_plan(&m, &f);
+    int64_t n = 0;
+    if (runs_multi(plan, nsteps)) {
+        static const char *const names[] = {"k_tile", "k_block", "k_block",
+                                            "k_block", "k_march", "k_stages"};
+        if (kernel) *kernel = names[plan.kernel];
+        for (int64_t left = nsteps; left > 0; ++n) left -= multi_next(plan, left);
+        if (multi_next(plan, nsteps) == 1) --n;  // the collide! that begins the run
+    } else {
+        n = nsteps - (nsteps >= 2 && first_in_one_pass(&m, &f) ? 2 : 1);
+    }
+    if (passes) *passes = n > 0 ? n : 0;
+    return 0;
 }
 
 // ---- moments ----------------------------------------------------------------

@@ -19,8 +19,8 @@ from .initial_conditions import (AnalyticalEquilibrium,  # noqa: F401
                                  initialize_mei)
 from .lattice import HipLattice  # noqa: F401
 from .model import (LatticeBoltzmannModel, ProcessingMethod, apply_boundary_conditions_,  # noqa: F401
-                    autotune, collide_model_, next_, simulate, simulate_launch_times, simulate_timed,
-                    stream_model_)
+                    autotune, collide_model_, next_, simulate, simulate_launch_times, simulate_plan,
+                    simulate_timed, stream_model_)
 from .moments import conserved_sums, density, moments, velocity  # noqa: F401
 from .problems import TGV, TaylorGreenVortex  # noqa: F401
 from .processing import (DensityConvergence, ExpectedFields, MeanVelocityStoppingCriteria,  # noqa: F401

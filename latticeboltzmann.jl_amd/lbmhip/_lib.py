@@ -30,7 +30,8 @@ EXPORTS = [
     "lbm_model_set_mrt", "lbm_model_set_force", "lbm_model_set_bcs", "lbm_model_set_launch",
     "lbm_autotune",
     "lbm_collide", "lbm_stream", "lbm_apply_bcs", "lbm_stream_bc", "lbm_simulate",
-    "lbm_simulate_timed", "lbm_simulate_launch_times", "lbm_moments", "lbm_reduce",
+    "lbm_simulate_timed", "lbm_simulate_plan", "lbm_simulate_launch_times", "lbm_moments",
+    "lbm_reduce",
     "lbm_reduce_noalloc",
     "lbm_batch_create", "lbm_batch_destroy", "lbm_batch_info", "lbm_batch_upload",
     "lbm_batch_download", "lbm_batch_set_launch", "lbm_batch_set_nodes_per_thread",
@@ -118,6 +119,8 @@ def lib() -> ctypes.CDLL:
         getattr(L, name).argtypes = [vp, vp, vp]
     L.lbm_simulate.argtypes = [vp, vp, vp, i64]
     L.lbm_simulate_timed.argtypes = [vp, vp, vp, i64, dp, ctypes.POINTER(i64)]
+    L.lbm_simulate_plan.argtypes = [i, i, i, i, i, ctypes.POINTER(LbmBC), i, i64,
+                                    ctypes.POINTER(ctypes.c_char_p), ctypes.POINTER(i64)]
     L.lbm_simulate_launch_times.argtypes = [vp, vp, vp, i64, dp, ctypes.POINTER(i64)]
     L.lbm_moments.argtypes = [vp, d, dp, dp, dp, dp, dp, dp]
     L.lbm_reduce.argtypes = [vp, dp]

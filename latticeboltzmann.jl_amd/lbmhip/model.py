@@ -147,8 +147,8 @@ def simulate(model: LatticeBoltzmannModel, time) -> LatticeBoltzmannModel:
 
 def simulate_timed(model: LatticeBoltzmannModel, nsteps: int):
     """As ``simulate(model, range(nsteps))`` without processing; returns
-    (milliseconds spent in the fused kernels after the first pass, number of
-    steps they advance), measured with HIP events on the library's stream."""
+    (milliseconds spent in the fused kernels, number of fused steps they
+    advance), measured with HIP events on the library's stream."""
     import ctypes
 
     m = native_model(model.quadrature).configure(model.collision_model, model.f_stream,
@@ -160,6 +160,23 @@ def simulate_timed(model: LatticeBoltzmannModel, nsteps: int):
                                              model.f_collision.handle, int(nsteps),
                                              ctypes.byref(ms), ctypes.byref(nl)), "simulate")
     return ms.value, nl.value
+
+
+def simulate_plan(model: LatticeBoltzmannModel, nsteps: int):
+    """What ``simulate_timed(model, nsteps)`` does with the automatic launch
+    shape: (kernel that advances several steps per pass, "" for one step per
+    launch; number of launches timed)."""
+    import ctypes
+
+    kinds = {"SRT": _lib.SRT_KIND, "TRT": _lib.TRT_KIND, "MRT": _lib.MRT_KIND}
+    f, bcs = model.f_stream, model.boundary_conditions
+    arr = (_lib.LbmBC * max(1, len(bcs)))(*[bc.to_abi() for bc in bcs])
+    kernel, passes = ctypes.c_char_p(), ctypes.c_int64()
+    _lib.check(_lib.lib().lbm_simulate_plan(model.quadrature.id, _lib.STORAGES[f.storage],
+                                            kinds[type(model.collision_model).__name__], f.nx, f.ny,
+                                            arr, len(bcs), int(nsteps), ctypes.byref(kernel),
+                                            ctypes.byref(passes)), "lbm_simulate_plan")
+    return kernel.value.decode(), passes.value
 
 
 def autotune(model: LatticeBoltzmannModel, trial_steps: int = 20) -> dict:

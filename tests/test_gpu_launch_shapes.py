@@ -100,3 +100,32 @@ def test_batch_shape_read_and_set_again_names_the_same_kernel():
     assert again.launch() == shape and _equal(same, got)
     again.set_launch(0, 0)
     assert again.launch() == auto.launch()
+
+
+@pytest.mark.parametrize("qid,shape,launch", [
+    (9, (100, 90), None), (9, (300, 250), None), (9, (1021, 517), None), (9, (2100, 1500), None),
+    (17, (512, 512), None), (9, (100, 90), (128, 1, 1, 1)), (9, (128, 64), (128, 1, 1, 1)),
+    (13, (40, 30), None)])
+def test_timed_runs_count_their_fused_steps(qid, shape, launch):
+    """Every step of a run but the collide! that begins it is counted and timed,
+    also where one pass holds the whole run; a single-step run that begins with
+    collide! and the first fused step in one pass (whole 64 x 8 tiles) leaves
+    that step out.  The state is the untimed run's."""
+    import lbmhip as L
+    q = L.Quadratures[f"D2Q{qid}"]()
+    f0 = random_populations(qid, *shape, seed=3)
+    one_pass = launch is not None and shape[0] % 64 == 0 and shape[1] % 8 == 0
+    for steps in (1, 2, 3, 5, 8, 9, 20):
+        a, b = (L.LatticeBoltzmannModel.from_populations(q, f0, L.TRT.fields(0.7, 1.3))
+                for _ in (0, 1))
+        a.launch = b.launch = launch
+        ms, n = L.simulate_timed(a, steps)
+        assert n == (max(steps - 2, 0) if one_pass else steps - 1)
+        assert ms > 0 or n == 0
+        if launch is None:
+            kernel, passes = L.simulate_plan(a, steps)
+            assert bool(kernel) == (qid != 13 and steps >= 2)
+            assert passes == n if not kernel else (steps + 7) // 8 <= passes <= steps - 1
+        L.simulate(b, range(steps))
+        assert np.array_equal(a.f_stream.to_numpy(), b.f_stream.to_numpy())
+        assert np.array_equal(a.f_collision.to_numpy(), b.f_collision.to_numpy())
