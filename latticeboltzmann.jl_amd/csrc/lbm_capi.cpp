@@ -646,6 +646,7 @@ bool first_in_one_pass(const lbm_model_s *m, const lbm_field_s *f) {
 
 MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     MultiPlan pl;
+    if (f->nx > lbm::kMultiMaxNx) return pl;
     // A shape set by the caller names a single-step kernel, with the automatic
     // numbers too.  Only those numbers with the store kind left automatic are
     // no shape of their own: lbm_autotune returns them when this path wins.

@@ -164,6 +164,8 @@ inline BlockShape block_shape(int nx, int ny, int steps, int rows, int elem_byte
     b.down = (ny + b.outy - 1) / b.outy;
     return b;
 }
+// the several-step kernels address a row by 32-bit byte offsets
+constexpr int kMultiMaxNx = (1 << 27) - 1;
 constexpr int kMarchRows = 16;  // fewest rows of a marching wave
 constexpr int kStageRows = 8;   // fewest rows of a pipeline's chunk
 // Most steps of a pipeline pass.  FP64 D2Q21/37: the rings of one hand-over

@@ -1222,7 +1222,7 @@ template <int QID, int COLL, class ST, int T, int NC, bool BC>
 int launch_march(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
     using S = typename ST::store_t;
     using SH = MarchShape<QID, ST, T, NC, BC>;
-    if (p.nx % NC != 0 || p.nx >= (1 << 27)) return -5;
+    if (p.nx % NC != 0 || p.nx > kMultiMaxNx) return -5;
     static const int slots = [] {
         int per_cu = 0, dev = 0, cus = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(

@@ -330,7 +330,7 @@ template <int QID, int COLL, class ST, int T, int SUB, bool BC>
 int launch_stages(const MultiLaunch &L, const StepParams<typename ST::T> &p, hipStream_t s) {
     using S = typename ST::store_t;
     using SH = StageShape<QID, ST, T, SUB>;
-    if (p.nx >= (1 << 27) || p.ny < 2 * SH::M || (L.walls & (2 | 8))) return -5;
+    if (p.nx > kMultiMaxNx || p.ny < 2 * SH::M || (L.walls & (2 | 8))) return -5;
     constexpr int threads = kStageCols * SUB * T;
     static const int slots = [] {
         int per_cu = 0, dev = 0, cus = 0;

@@ -69,3 +69,13 @@ def test_plan_errors():
     for args in ((10, 0, 0, 8, 8, bc, 0, 3), (9, 99, 0, 8, 8, bc, 0, 3), (9, 0, 3, 8, 8, bc, 0, 3),
                  (9, 0, 0, 0, 8, bc, 0, 3), (9, 0, 0, 8, 8, None, 1, 3), (9, 0, 0, 8, 8, bc, 0, -1)):
         assert L.lbm_simulate_plan(*args, None, None) < 0
+
+
+@pytest.mark.parametrize("qid,storage", [(4, "f64"), (5, "f32"), (9, "f32"), (9, "f16neq"),
+                                         (13, "f32")])
+def test_rows_beyond_32_bit_offsets_keep_single_steps(qid, storage):
+    """the several-step kernels refuse rows of 2^27 nodes; the single-step ones
+    take them"""
+    assert plan(qid, storage, TRT, 2 ** 27 - 2, 15 if qid < 13 else 16, 9)[0] != ""
+    assert plan(qid, storage, TRT, 2 ** 27, 15 if qid < 13 else 16, 9) == ("", 8)
+    assert plan(qid, storage, TRT, 2 ** 27, 1, 9) == ("", 8)
