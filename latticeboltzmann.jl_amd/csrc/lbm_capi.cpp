@@ -1270,7 +1270,8 @@ static int simulate_impl(lbm_model m, lbm_field S, lbm_field C, int64_t nsteps, 
     }
     // Runs that time every launch keep one fused step per launch; the others
     // advance several collisions per pass where a kernel for it exists.
-    const MultiPlan plan = per_launch ? MultiPlan{} : multi_plan(m, S);
+    // (a tracked run calls for one step at a time: no plan for those)
+    const MultiPlan plan = per_launch || nsteps < 2 ? MultiPlan{} : multi_plan(m, S);
     const bool multi = runs_multi(plan, nsteps);
     // step 1 starts from the canonical state S: the first pass collides S_0 in
     // place.  Without a several-step kernel, one-speed stencils on lattices of
