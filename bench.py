@@ -11,10 +11,11 @@ relative L2 velocity error against the FP64 run.
 
 ``roofline`` prices the fused kernel against MI355X's 8 TB/s: algorithmic
 bytes per launch = 2 * Q * sizeof(population) * nodes (one read and one write
-of every population per pass, however many steps the pass advances:
-``steps_per_pass``), divided by the kernel's average duration measured with
-HIP events on the library's stream.  The ``spread`` entries are of runs with
-one step per launch.
+of every population per pass, however many steps the pass advances), divided
+by the kernel's average duration: the time of the K steps' passes, measured
+with HIP events on the library's stream, over their number
+(``steps_per_pass`` = steps over passes).  The ``spread`` entries are of runs
+with one step per launch.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--n 4096]
 """
@@ -49,9 +50,6 @@ def tgv_populations(L, q, n, u0=0.02):
 # the Taylor-Green workload's length: the accuracy of every storage is taken
 # after this many steps, whatever --steps is
 ACCURACY_STEPS = 5000
-# time steps a kernel of the timed runs advances per pass over the lattice (the
-# library's several-step kernels at this size; the deviation storages: one)
-STEPS_PER_PASS = {"f64": 5, "f32": 6, "f16neq": 4, "bf16neq": 4, "f16dev": 1, "bf16dev": 1}
 # fused launches timed one by one for the spread of the kernel's duration
 SPREAD_LAUNCHES = 200
 # back-to-back device copies of the FP64 lattice for the copy-rate ceiling
@@ -87,7 +85,18 @@ def run_storage(L, q, f0, cm, storage, steps, warmup, accuracy_steps):
     c1 = L.clock_sample()
     m = L.moments(acc.f_stream, stress=False)
     del acc
-    return model, wall, kernel_ms, nlaunch, L.average_clock_mhz(c0, c1), (m.ux, m.uy)
+    return (model, wall, pass_figures(L, model, steps, kernel_ms, nlaunch),
+            L.average_clock_mhz(c0, c1), (m.ux, m.uy))
+
+
+def pass_figures(L, model, steps, kernel_ms, nlaunch):
+    """(several-step kernel or "", average milliseconds of a timed pass, steps
+    per pass) of a timed run.  A first pass of several steps holds the collide!
+    that begins the run, so all ``steps`` steps are in the passes then."""
+    kernel, passes = L.simulate_plan(model, steps)
+    if passes < 1:  # a run of one step: collide! and stream!, no fused pass
+        return kernel, 0.0, 0.0
+    return kernel, kernel_ms / passes, (steps if kernel else nlaunch) / passes
 
 
 def copy_rate(L, f, copies=COPY_LAUNCHES):
@@ -126,12 +135,19 @@ def _r(v, nd=1):
     return None if v is None else round(v, nd)
 
 
+def _rate(nbytes, ms):
+    """GB/s (0 where nothing was timed: a run of one step)"""
+    return nbytes / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
+
+
 def rel_l2(a, b):
     num = np.sqrt(np.sum((a[0] - b[0]) ** 2 + (a[1] - b[1]) ** 2))
     return float(num / np.sqrt(np.sum(b[0] ** 2 + b[1] ** 2)))
 
 
-def traffic_for(key):
+def traffic_for(storage, n, kernel):
+    """Measured HBM bytes of a pass at this size, or None"""
+    key = f"d2q9_trt_{storage}_{n}" + (f"_{kernel}" if kernel else "")
     try:
         with open(TRAFFIC_FILE) as fh:
             return json.load(fh).get(key)
@@ -564,12 +580,11 @@ def main():
     nodes = n * n
 
     acc_steps = a.accuracy_steps
-    m64, wall64, kms64, nl64, clk64, u64 = run_storage(L, q, f0, cm, "f64", K, W, acc_steps)
+    m64, wall64, (kernel64, kavg64, spp64), clk64, u64 = run_storage(L, q, f0, cm, "f64", K, W,
+                                                                     acc_steps)
     mlups64 = nodes * K / wall64 / 1e6
     bytes64 = 2 * q.Q * 8 * nodes
-    kavg64 = kms64 / max(nl64, 1)
-    spp64 = STEPS_PER_PASS["f64"]
-    gbs64 = bytes64 / (kavg64 * spp64 * 1e-3) / 1e9
+    gbs64 = _rate(bytes64, kavg64)
     spread64 = launch_spread(L, m64)
     copy_s = copy_rate(L, m64.f_stream)
     copy_gbs = bytes64 / copy_s / 1e9
@@ -603,10 +618,10 @@ def main():
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(gbs64 / HBM_PEAK_GBS, 4),
-            "traffic": traffic_for("d2q9_trt_f64_4096"),
-            "kernel": "k_march<9,TRT,F64> (marching waves, five steps per pass)",
-            "kernel_ms_avg": round(kavg64 * spp64, 5),
-            "steps_per_pass": spp64,
+            "traffic": traffic_for("f64", n, kernel64),
+            "kernel": f"{kernel64 or 'k_fused_v'}<9,TRT,F64>",
+            "kernel_ms_avg": round(kavg64, 5),
+            "steps_per_pass": round(spp64, 3),
             "bytes_per_launch": bytes64,
             "shader_clock_mhz": _r(clk64),
             "spread": spread64,
@@ -622,27 +637,20 @@ def main():
         # the reduced storages: non-equilibrium parts about a 16-bit equilibrium
         # record (*neq: 2 Q + 8 bytes per node), rest-state deviations (*dev),
         # and shifted FP32
-        kernels = {
-            "f16neq": "k_march<9,TRT,F16Neq> (marching waves, two columns per lane, four steps "
-                      "per pass)",
-            "bf16neq": "k_march<9,TRT,BF16Neq> (marching waves, two columns per lane, four "
-                       "steps per pass)",
-            "f16dev": "k_fused_v<9,TRT,F16Dev> (4 nodes/thread)",
-            "bf16dev": "k_fused_v<9,TRT,BF16Dev> (4 nodes/thread)",
-            "f32": "k_march<9,TRT,F32> (marching waves, six steps per pass)",
-        }
+        single = {"f16neq": "k_fused_neq_rows", "bf16neq": "k_fused_neq_rows",
+                  "f16dev": "k_fused_v", "bf16dev": "k_fused_v", "f32": "k_fused_v"}
+        names = {"f16neq": "F16Neq", "bf16neq": "BF16Neq", "f16dev": "F16Dev",
+                 "bf16dev": "BF16Dev", "f32": "F32"}
         for storage, key, per_node in (("f16neq", "fp16neq", 2 * q.Q + 8),
                                        ("f16dev", "fp16dev", 2 * q.Q),
                                        ("bf16neq", "bf16neq", 2 * q.Q + 8),
                                        ("bf16dev", "bf16dev", 2 * q.Q),
                                        ("f32", "fp32", 4 * q.Q)):
-            m16, wall16, kms16, nl16, clk16, u16 = run_storage(L, q, f0, cm, storage, K, W,
-                                                               acc_steps)
+            m16, wall16, (kernel16, kavg16, spp16), clk16, u16 = run_storage(L, q, f0, cm, storage,
+                                                                             K, W, acc_steps)
             mlups16 = nodes * K / wall16 / 1e6
             bytes16 = 2 * per_node * nodes
-            kavg16 = kms16 / max(nl16, 1)
-            spp16 = STEPS_PER_PASS[storage]
-            gbs16 = bytes16 / (kavg16 * spp16 * 1e-3) / 1e9
+            gbs16 = _rate(bytes16, kavg16)
             spread16 = launch_spread(L, m16)
             del m16
             result[key] = {
@@ -655,10 +663,10 @@ def main():
                 "ms_per_step": round(wall16 / K * 1e3, 5),
                 "roofline": {"bound": "hbm", "achieved": round(gbs16, 1), "peak": HBM_PEAK_GBS,
                              "unit": "GB/s", "frac": round(gbs16 / HBM_PEAK_GBS, 4),
-                             "traffic": traffic_for(f"d2q9_trt_{storage}_4096"),
-                             "kernel": kernels[storage],
-                             "kernel_ms_avg": round(kavg16 * spp16, 5),
-                             "steps_per_pass": spp16, "bytes_per_launch": bytes16,
+                             "traffic": traffic_for(storage, n, kernel16),
+                             "kernel": f"{kernel16 or single[storage]}<9,TRT,{names[storage]}>",
+                             "kernel_ms_avg": round(kavg16, 5),
+                             "steps_per_pass": round(spp16, 3), "bytes_per_launch": bytes16,
                              "shader_clock_mhz": _r(clk16), "spread": spread16},
             }
 

@@ -79,3 +79,33 @@ def test_rows_beyond_32_bit_offsets_keep_single_steps(qid, storage):
     assert plan(qid, storage, TRT, 2 ** 27 - 2, 15 if qid < 13 else 16, 9)[0] != ""
     assert plan(qid, storage, TRT, 2 ** 27, 15 if qid < 13 else 16, 9) == ("", 8)
     assert plan(qid, storage, TRT, 2 ** 27, 1, 9) == ("", 8)
+
+
+@pytest.mark.parametrize("n,storage,steps,kernel,passes,per_pass", [
+    (4096, "f64", 20, "k_march", 4, 5.0), (4096, "f32", 20, "k_march", 4, 5.0),
+    (4096, "f32", 5000, "k_march", 834, 5000 / 834), (1024, "f64", 20, "k_block", None, None),
+    (4096, "f16dev", 20, "", 18, 1.0), (4095, "f16dev", 20, "", 19, 1.0)])
+def test_bench_prices_the_passes_that_run(n, storage, steps, kernel, passes, per_pass):
+    """the benchmark's kernel, time of a pass and steps per pass follow the plan
+    of the run at hand"""
+    from types import SimpleNamespace
+
+    import bench
+    import lbmhip as L
+    model = SimpleNamespace(quadrature=L.D2Q9(), boundary_conditions=[],
+                            collision_model=L.TRT.fields(0.6, 1.3),
+                            f_stream=SimpleNamespace(storage=storage, nx=n, ny=n))
+    counted = passes if not kernel else steps - 1
+    got = bench.pass_figures(L, model, steps, 7.0, counted)
+    assert got[0] == kernel
+    if passes:
+        assert got[1:] == pytest.approx((7.0 / passes, per_pass))
+    assert got[1] * (steps if kernel else counted) / got[2] == pytest.approx(7.0)
+    assert bench.pass_figures(L, model, 1, 0.005, 0) == ("", 0.0, 0.0)
+
+
+def test_bench_traffic_belongs_to_the_kernel_and_size():
+    import bench
+    march = bench.traffic_for("f64", 4096, "k_march")
+    assert march > 1.1 * bench.traffic_for("f64", 4096, "") > 0
+    assert bench.traffic_for("f64", 1024, "k_block") is None
