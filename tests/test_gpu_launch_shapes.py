@@ -129,3 +129,69 @@ def test_timed_runs_count_their_fused_steps(qid, shape, launch):
         L.simulate(b, range(steps))
         assert np.array_equal(a.f_stream.to_numpy(), b.f_stream.to_numpy())
         assert np.array_equal(a.f_collision.to_numpy(), b.f_collision.to_numpy())
+
+
+def _first_step_model(qid, shape, coll, bcname, force, storage, seed, noise):
+    import lbmhip as L
+    from lbm_cases import bc_dicts, force_for, to_lbmhip
+    q = L.Quadratures[f"D2Q{qid}"]()
+    f0 = random_populations(qid, *shape, seed=seed, noise=noise)
+    F = force_for(force, *shape)
+    cm, taus = {0: (L.SRT(0.8, F), [0.8]), 1: (L.TRT.fields(0.7, 1.3, F), [0.7, 1.3]),
+                2: (L.MRT(q, [0.9, 0.75], force=F), [0.9, 0.75])}[coll]
+    bcs = bc_dicts(bcname, *shape)
+
+    def model():
+        return L.LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs), storage=storage)
+
+    return model, f0, taus, F, bcs
+
+
+# whole 64 x 8 tiles whose runs begin with k_fused_first*: with a shape set, and
+# without one too long and low for the several-step kernels
+FIRST = [((128, 16), (128, 1, 1, 1)), ((64, 8), (64, 4, 1, 1)), ((3392, 8), None)]
+
+
+@pytest.mark.parametrize("shape,launch", FIRST)
+@pytest.mark.parametrize("qid", [4, 5, 9])
+@pytest.mark.parametrize("coll", [0, 1, 2])
+@pytest.mark.parametrize("bcname,force", [("periodic", "none"), ("couette", "const"),
+                                          ("cavity", "field"), ("partial", "none")])
+def test_first_step_in_one_pass_bit_exact(oracle_lib, qid, shape, launch, coll, bcname, force):
+    """FP64: the run's first step as one pass (collide S_0 into an LDS tile with
+    a halo, stream, boundaries, collide) gives the oracle's bits."""
+    import lbmhip as L
+    model, f0, taus, F, bcs = _first_step_model(qid, shape, coll, bcname, force, "f64",
+                                                53 + qid + coll, 2e-3)
+    for steps in (2, 5):
+        m = model()
+        m.launch = launch
+        assert L.simulate_timed(m, steps)[1] == steps - 2  # its two steps are one launch
+        S, C = f0.copy(order="F"), f0.copy(order="F")
+        oracle_lib.simulate(qid, S, C, coll, taus, steps, force=F, bcs=bcs)
+        assert np.array_equal(m.f_stream.to_numpy(), S)
+        assert np.array_equal(m.f_collision.to_numpy(), C)
+
+
+@pytest.mark.parametrize("shape,launch", FIRST)
+@pytest.mark.parametrize("qid", [4, 5, 9])
+@pytest.mark.parametrize("coll", [0, 1])
+@pytest.mark.parametrize("bcname,force", [("periodic", "none"), ("couette", "const"),
+                                          ("cavity", "field"), ("partial", "none")])
+def test_first_step_in_one_pass_f32(qid, shape, launch, coll, bcname, force):
+    """FP32 against the two-pass start (collide!, then the fused step): the two
+    order a step's operations differently, so each of the two collisions may
+    differ by 16 half-ulps of the largest shifted population (the bound of
+    test_f32_tracks_oracle), for six steps; a wrong pull, halo or boundary value
+    differs by 1e-2 w."""
+    import lbmhip as L
+    model, f0, *_ = _first_step_model(qid, shape, coll, bcname, force, "f32", 61 + qid, 1e-4)
+    one, two = model(), model()
+    one.launch = two.launch = launch or (256, 1, 1, 1)
+    assert L.simulate_timed(one, 6)[1] == 4
+    L.simulate_launch_times(two, 6)
+    w = np.asarray(one.quadrature.weights)
+    for a, b in ((one.f_stream, two.f_stream), (one.f_collision, two.f_collision)):
+        a, b = a.to_numpy(), b.to_numpy()
+        G = max(np.abs(b - w).max(), np.abs(f0 - w).max())
+        assert np.abs(a - b).max() <= 16 * 7 * 2.0 ** -24 * G

@@ -75,3 +75,42 @@ def test_f32_error_no_larger_than_single_steps(oracle_lib, qid, shape, coll, bcn
     for a, b, ref in ((many.f_stream, one.f_stream, S), (many.f_collision, one.f_collision, C)):
         ea, eb = (np.linalg.norm(x.to_numpy() - ref) for x in (a, b))
         assert ea <= 1.1 * eb, (ea, eb)
+
+
+@pytest.mark.parametrize("qid", [13, 17, 21, 37])
+@pytest.mark.parametrize("shape", [(672, 800), (1021, 517), (30001, 17)])
+@pytest.mark.parametrize("coll,bcname,steps", [(0, "couette", 6), (1, "poiseuille", 8),
+                                               (1, "couette", 9)])
+def test_f64_later_passes_between_two_walls_bit_exact(oracle_lib, qid, shape, coll, bcname, steps):
+    """passes of three steps (D2Q13 and D2Q17) that pull their first one"""
+    nx, ny = shape
+    f0 = _populations(qid, nx, ny, seed=qid + 5 * coll)
+    q, cm, taus = _model(qid, coll, None)
+    bcs = _bcs(bcname, nx, ny)
+    model = _L().LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs))
+    print(f"stages later D2Q{qid} {nx}x{ny} {bcname} {steps} steps", flush=True)
+    _L().simulate(model, range(steps))
+    S, C = _oracle(oracle_lib, qid, f0, coll, taus, steps, None, bcs)
+    assert np.array_equal(model.f_stream.to_numpy(), S)
+    assert np.array_equal(model.f_collision.to_numpy(), C)
+
+
+@pytest.mark.parametrize("qid", [13, 17, 21, 37])
+@pytest.mark.parametrize("shape", [(672, 800), (1021, 517), (30001, 17)])
+@pytest.mark.parametrize("direction", [0, 2])
+@pytest.mark.parametrize("steps", [3, 8])
+def test_f64_one_ranged_wall_bit_exact(oracle_lib, qid, shape, direction, steps):
+    """one wall over a part of its row, a later condition of the same wall over
+    another part; passes of up to three steps"""
+    nx, ny = shape
+    f0 = _populations(qid, nx, ny, seed=qid + direction)
+    q, cm, taus = _model(qid, 1, None)
+    ys = (1, 2) if direction == 2 else (ny - 2, ny)
+    bcs = [dict(kind=0, direction=direction, xs=(5, nx // 2), ys=ys),
+           dict(kind=0, direction=direction, xs=(nx // 3, nx - 60), ys=(1, ny))]
+    model = _L().LatticeBoltzmannModel.from_populations(q, f0, cm, to_lbmhip(bcs))
+    print(f"stages one wall {direction} D2Q{qid} {nx}x{ny} {steps} steps", flush=True)
+    _L().simulate(model, range(steps))
+    S, C = _oracle(oracle_lib, qid, f0, 1, taus, steps, None, bcs)
+    assert np.array_equal(model.f_stream.to_numpy(), S)
+    assert np.array_equal(model.f_collision.to_numpy(), C)
