@@ -4,9 +4,11 @@
 // bound by 2 Q sizeof(population) n bytes per node.  The kernels here advance
 // a region by T steps per pass instead, recomputing a halo that shrinks by
 // the stencil's reach per step, so T steps cost one pass:
+//   * k_tile: a block keeps a tile of the lattice in LDS (small lattices);
+//   * k_block: a block of waves keeps 64 columns of rows in registers and
+//     exchanges the waves' edge rows through LDS (those in between);
 //   * k_march: a wave marches up a strip of columns with the rows of the T
-//     levels in registers and in its own LDS;
-//   * k_tile: a block keeps a tile of the lattice in LDS.
+//     levels in registers and in its own LDS (large ones).
 // Every node is updated by the operations of the single-step kernels in their
 // order, wrapped to its lattice position, boundary list included: FP64 results
 // are bit-identical to running the steps one by one.
@@ -101,8 +103,9 @@ __device__ __forceinline__ void moments_div2(const double (&f)[QT<QID>::Q], doub
 // the symmetric and antisymmetric parts of the pair are formed once.  `before(i, ..)`
 // runs ahead of population i's part and may touch the velocity that the rest
 // depends on.  Rounding for rounding the values are those of
-// collide_seq (negation and scaling by 1/2 are exact); D2Q9 TRT FP64 takes
-// 137 arithmetic instructions instead of 224.
+// collide_seq (negation and scaling by 1/2 are exact, short of overflow: a run
+// whose populations pass 2^1021 may reach infinity at another step); D2Q9 TRT
+// FP64 takes 137 arithmetic instructions instead of 224.
 template <int QID, int COLL, class F, class H, int... Is>
 __device__ __forceinline__ void collide_pairs(double (&f)[QT<QID>::Q], const StepParams<double> &p,
                                               const MultiConsts<double> &mc, F &&force, H &&before,
