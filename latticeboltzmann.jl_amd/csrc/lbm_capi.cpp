@@ -1977,6 +1977,7 @@ struct lbm_batch_s {
     // shape is automatic (region_mode: -1 undecided, 0 not worth it, 1 in use)
     bool explicit_shape = false;
     int region_mode = -1;
+    int region_min = 2;  // shorter runs keep single steps
     lbm::BatchRegion *dRegions = nullptr;
     int nregions = 0;
     std::mutex stage_mu;       // one host transfer at a time
@@ -2056,10 +2057,13 @@ int batch_launch(lbm_batch b, int op, int parity) {
 // small lattices computes mostly nodes that are not written, while the
 // single-step kernel packs a lattice's nodes densely.  us a step, several
 // steps / single steps: 512 lattices of 200 x 200 (2 computed nodes a written
-// one) 194 / 510 in FP64 and 90 / 303 in FP32, of 64 x 64 (3) 33 / 52 and
-// 14 / 29; the two would meet near 5, and the line is drawn at 4.  Up to one
-// block a CU the number of nodes computed does not matter (48 lattices of
-// 40 x 40: 3.2 / 5.8 and 2.1 / 5.0).
+// one) 194 / 510 in FP64 and 90 / 303 in FP32, of 64 x 64 (3) 25 / 52 and
+// 13 / 28, and at the line, drawn at 4: FP64 28 x 28 (3.9) 7.7 / 15.2, FP32
+// 32 x 32 (4.0) 5.4 / 9.1 (where the two meet beyond it was not measured).  Up
+// to one block a CU the number of nodes computed does not matter (48 lattices
+// of 40 x 40: 3.2 / 5.8 and 2.1 / 5.0).  A call of two steps saves one launch
+// only; FP32 near the line loses by it (512 of 32 x 32 47.8 / 42.8 us a call,
+// 56 x 56 (3.9) 91.8 / 91.5, 64 x 64 (3) 90 / 100; FP64 28 x 28 55 / 61).
 // Returns < 0 on error; otherwise b->region_mode says which.
 int batch_regions(lbm_batch b) {
     if (b->region_mode >= 0) return 0;
@@ -2075,10 +2079,12 @@ int batch_regions(lbm_batch b) {
         for (int y = 0; y < ny; y += outy)
             for (int x = 0; x < nx; x += outx) reg.push_back(lbm::BatchRegion{k, x, y, outx, outy});
     }
-    if (reg.size() > 256 && (double)reg.size() * 64.0 * rows > 4.0 * (double)b->nodes) {
+    const double written = (double)b->nodes, computed = (double)reg.size() * 64.0 * rows;
+    if (reg.size() > 256 && computed > 4.0 * written) {
         b->region_mode = 0;
         return 0;
     }
+    b->region_min = !f64 && reg.size() > 256 && computed > 3.5 * written ? 3 : 2;
     HIP_TRY(hipMalloc(&b->dRegions, reg.size() * sizeof(lbm::BatchRegion)));
     HIP_TRY(hipMemcpyAsync(b->dRegions, reg.data(), reg.size() * sizeof(lbm::BatchRegion),
                            hipMemcpyHostToDevice, g_stream));
@@ -2311,7 +2317,7 @@ int lbm_batch_simulate(lbm_batch b, int64_t nsteps, int graph_chunk, double *ms_
     const bool automatic = !b->explicit_shape && b->vec == 1;
     if (automatic)
         if (int rc = batch_regions(b)) return rc;
-    const bool multi = automatic && b->region_mode == 1 && nsteps >= 2;
+    const bool multi = automatic && b->region_mode == 1 && nsteps >= b->region_min;
     const int tmax = b->storage == LBM_STORE_F64 ? lbm::kBatchStepsF64 : lbm::kBatchStepsF32;
     // equal passes: the last ones are not left with a single step
     auto pass = [&](int64_t left) {

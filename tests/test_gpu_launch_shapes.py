@@ -195,3 +195,21 @@ def test_first_step_in_one_pass_f32(qid, shape, launch, coll, bcname, force):
         a, b = a.to_numpy(), b.to_numpy()
         G = max(np.abs(b - w).max(), np.abs(f0 - w).max())
         assert np.abs(a - b).max() <= 16 * 7 * 2.0 ** -24 * G
+
+
+@pytest.mark.parametrize("steps,several", [(2, False), (3, True)])
+def test_short_runs_of_batches_of_small_lattices(steps, several):
+    """FP32, 512 lattices of 32 x 32 (four nodes computed for one written): two
+    steps run one per launch, three in a pass"""
+    import lbmhip as L
+    f = [random_populations(9, 32, 32, seed=k, noise=1e-2) for k in range(2)]
+    out = []
+    for launch in (None, (128, 0)):
+        b = L.LatticeBatch(L.D2Q9(), [(32, 32)] * 512, [0.7] * 512, [1.3] * 512, storage="f32")
+        for k in range(512):
+            b.upload(k, f[k % 2])
+        if launch:
+            b.set_launch(*launch)
+        b.simulate(steps)
+        out.append([b.download(k) for k in (0, 1, 510, 511)])
+    assert _equal(*out) == (not several)
