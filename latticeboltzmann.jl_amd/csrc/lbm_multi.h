@@ -188,7 +188,7 @@ __device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const Step
                                               const MultiConsts<float> &mc, F &&force, H &&before,
                                               std::integer_sequence<int, Is...>) {
     constexpr int FEQ = QT<QID>::FEQ, Q = QT<QID>::Q;
-    static_assert(COLL <= 1, "pair form: SRT and TRT");
+    static_assert(COLL <= 1 || COLL == 6 || COLL == 7, "pair form: SRT and TRT");
     float s[Q], d[Q];  // pair sums and differences, at the smaller index
     auto sums = [&](auto Ic) {
         constexpr int i = decltype(Ic)::value, j = QT<QID>::opp(i);
@@ -237,7 +237,8 @@ __device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const Step
         before(Ic, ax, ay);
         if constexpr (i == j) {
             const float n = f[i] - p.w[wr] * a0;
-            f[i] = f[i] - (COLL == 0 ? p.om : p.oms) * n;
+            if constexpr (COLL == 6) f[i] = p.omo * f[i] + p.om * (p.w[wr] * a0);
+            else f[i] = f[i] - (COLL == 0 ? p.om : p.oms) * n;
         } else if constexpr (i < j) {
             float od = udot<QID, i>(ax, ay), ev = a0;
             if constexpr (FEQ == 2) {
@@ -247,27 +248,60 @@ __device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const Step
                 od = t * (e.k1 + t2 * e.k3);
                 ev = FEQ == 3 ? a0 + t2 * e.k2 : a0 + t2 * (e.k2 + t2 * e.k4);
             }
-            if constexpr (COLL == 0) {
+            if constexpr (COLL == 6) {  // the single-step kernels' relaxation (srt.jl:57-59)
+                const float w = p.w[wr];
+                f[i] = p.omo * f[i] + p.om * (w * (ev + od));
+                f[j] = p.omo * f[j] + p.om * (w * (ev - od));
+            } else if constexpr (COLL == 0) {
                 const float w = p.w[wr];
                 f[i] = f[i] - p.om * (f[i] - w * (ev + od));
                 f[j] = f[j] - p.om * (f[j] - w * (ev - od));
             } else {
                 const float ns = s[i] + mc.w2[wr] * ev, na = d[i] + mc.w2[wr] * od;
-                f[i] = (f[i] - mc.homs * ns) - mc.homa * na;
-                f[j] = (f[j] - mc.homs * ns) + mc.homa * na;
+                if constexpr (COLL == 7) {  // one rounding at f's size instead of two
+                    const float t = mc.homa * na;
+                    f[i] = f[i] - (mc.homs * ns + t);
+                    f[j] = f[j] - (mc.homs * ns - t);
+                } else {
+                    f[i] = (f[i] - mc.homs * ns) - mc.homa * na;
+                    f[j] = (f[j] - mc.homs * ns) + mc.homa * na;
+                }
             }
         }
     };
     (one(std::integral_constant<int, Is>{}), ...);
 }
 
-template <int QID, int COLL, class T>
+// The form of a collision (COLL 0 SRT, 1 TRT, 2 MRT; 4 SRT in the single-step
+// kernels' own form): 4 and 5 that form, 6 and 7 pair forms of FP32.
+//
+// FP32 momentum drifts by the rounding of the weights, s sum w c^2 = 1 + d, and,
+// with SRT as omo f + om feq, by that of omo = 1 - 1/tau and om: two errors that
+// cancel at some tau and add up at others.  The pair form as f - om (f - feq) has
+// the first only: over tau in 0.6 .. 1.0 and 200 steps its error against 64 bits
+// was 0.3 to 6.4 times the single-step kernels' on D2Q9 (geometric mean 1.07), up
+// to 8.6 on D2Q5 (1.9).  So SRT relaxes as they do (D2Q9 60 steps on 1500 x 1300
+// 530 -> 603 us, single steps 1,754).  TRT on D2Q9 takes both relaxed parts off
+// at once (at tau 0.6, where the drifts cancel, 1.05 before), on D2Q4/5, up to 1.8
+// before, it runs the single-step form (5 %).  The ratio is 1.00 with each.  The
+// 16-bit storages, whose single steps relax f - feq, keep the plain pairs (0.6
+// to 1.02 of the single-step kernels' error) but for TRT on D2Q4/5 (up to 1.5
+// before, 0.6 to 1.01).
+template <int QID, int COLL, class ST>
+LBM_HD constexpr int multi_form() {
+    if (COLL > 1 || !ST::kShift) return COLL;
+    if (COLL == 1 && QID < 9) return 5;
+    return ST::kNeq ? COLL : (COLL == 0 ? 6 : 7);
+}
+
+template <int QID, int COLL, class ST, class T>
 __device__ __forceinline__ void collide_multi(T (&f)[QT<QID>::Q], const StepParams<T> &p,
                                               const MultiConsts<T> &mc, int x, int y) {
-    if constexpr (COLL == 4) {  // SRT in the single-step kernels' own form
-        collide_any<QID, 0>(f, p, x, y);
-    } else if constexpr (COLL <= 1) {
-        collide_pairs<QID, COLL>(f, p, mc, [&](T &Fx, T &Fy) { node_force_wait(p, x, y, Fx, Fy); },
+    constexpr int FORM = multi_form<QID, COLL, ST>();
+    if constexpr (FORM == 4 || FORM == 5) {
+        collide_any<QID, FORM - 4>(f, p, x, y);
+    } else if constexpr (FORM != 2) {
+        collide_pairs<QID, FORM>(f, p, mc, [&](T &Fx, T &Fy) { node_force_wait(p, x, y, Fx, Fy); },
                                  [](auto, T &, T &) {}, LBM_SEQ);
     } else {
         double rho, ux, uy;
@@ -483,7 +517,7 @@ tile_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *__
             };
             adj_each_node<QID>(one);
         } else {
-            collide_multi<QID, COLL, T>(f[k], p, mc, xs[k], ys[k]);
+            collide_multi<QID, COLL, ST, T>(f[k], p, mc, xs[k], ys[k]);
         }
     };
     auto store = [&](S *dst, int k) {
@@ -698,7 +732,7 @@ block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *_
                     return ld_pop<QID, decltype(Jc)::value, ST>(C, p, (long long)x + (long long)p.nx * y);
                 });
         }
-        collide_multi<QID, COLL, V>(g[j], p, mc, x, y);
+        collide_multi<QID, COLL, ST, V>(g[j], p, mc, x, y);
         if constexpr (ALL) store(static_cast<S *>(all->out[0]), j, g[j]);
     }
     for (int l = 2; l <= L; ++l) {
@@ -743,7 +777,7 @@ block_region(const typename ST::store_t *__restrict__ C, typename ST::store_t *_
                 bc_apply<QID, V>(p, wall.moving, bcm[j], f,
                                  [&](auto Jc) { return g[j][decltype(Jc)::value]; });
             }
-            collide_multi<QID, COLL, V>(f, p, mc, x, y);
+            collide_multi<QID, COLL, ST, V>(f, p, mc, x, y);
             auto cp = [&](auto Ic) {
                 constexpr int i = decltype(Ic)::value;
                 g[j][i] = f[i];
@@ -995,7 +1029,7 @@ k_march(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
                     });
             }
 #pragma unroll
-            for (int c = 0; c < NC; ++c) collide_multi<QID, COLL, V>(n[c], p, mc, xs[c], rl);
+            for (int c = 0; c < NC; ++c) collide_multi<QID, COLL, ST, V>(n[c], p, mc, xs[c], rl);
         }
         const int par = k & 1;
         Rec16 orec[NC];
@@ -1069,7 +1103,7 @@ k_march(const typename ST::store_t *__restrict__ C, typename ST::store_t *__rest
                         continue;
                     }
                 }
-                collide_multi<QID, COLL, V>(f[c], p, mc, xs[c], rl);
+                collide_multi<QID, COLL, ST, V>(f[c], p, mc, xs[c], rl);
                 auto cp = [&](auto Ic) {
                     constexpr int i = decltype(Ic)::value;
                     n[c][i] = f[c][i];

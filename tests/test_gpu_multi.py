@@ -471,3 +471,81 @@ def test_f64_non_finite_populations(oracle_lib, qid, shape, coll, value):
     assert np.isnan(S).any() or np.isinf(S).any()
     assert np.array_equal(model.f_stream.to_numpy(), S, equal_nan=True)
     assert np.array_equal(model.f_collision.to_numpy(), C, equal_nan=True)
+
+
+def _vortices(nx, ny, seed):
+    rng = np.random.default_rng(seed)
+    x, y = np.meshgrid(np.arange(nx) * 2 * np.pi / nx, np.arange(ny) * 2 * np.pi / ny,
+                       indexing="ij")
+    ux, uy = (sum(0.01 * rng.normal() * np.sin(k * c + rng.uniform(0, 6)) for k in (1, 2, 3))
+              for c in (y, x))
+    return 1 + 0.01 * np.sin(x + y), ux, uy
+
+
+@pytest.mark.parametrize("qid", [4, 5, 9])
+@pytest.mark.parametrize("shape", [(100, 90), (300, 250), (1021, 517), (4099, 2500)])
+@pytest.mark.parametrize("coll,tau", [(0, 0.6), (0, 0.678), (0, 0.728), (0, 0.87), (0, 0.949),
+                                      (0, 0.969), (1, 0.6), (1, 0.668), (1, 0.8)])
+def test_f32_drift_no_larger_than_single_steps(qid, shape, coll, tau):
+    """FP32 over 200 steps: what a step's rounding adds up to (the drift of the
+    momentum, which depends on how a form rounds the weights and rates) is at
+    most the single-step kernels', with a twentieth for scatter."""
+    L = _L()
+    q = L.Quadratures[f"D2Q{qid}"]()
+    f0 = L.equilibrium_populations(q, *_vortices(*shape, seed=qid))
+    cm = L.SRT(tau) if coll == 0 else L.trt_magic(tau)
+
+    def run(storage, fn):
+        m = L.LatticeBoltzmannModel.from_populations(q, f0, cm, storage=storage)
+        fn(m)
+        return m.f_stream.to_numpy()
+
+    steps = 200 if shape[0] < 4000 else 40
+    ref = run("f64", lambda m: L.simulate(m, range(steps)))
+    many = np.linalg.norm(run("f32", lambda m: L.simulate(m, range(steps))) - ref)
+    one = np.linalg.norm(run("f32", lambda m: L.simulate_launch_times(m, steps)) - ref)
+    assert many <= 1.05 * one, (many / one)
+
+
+@pytest.mark.parametrize("trt", [False, True])
+def test_batch_f32_drift_no_larger_than_single_steps(trt):
+    L = _L()
+    sizes = [(100 + 10 * k, 90) for k in range(8)]
+    taus = [0.6, 0.643, 0.678, 0.728, 0.8, 0.87, 0.949, 0.969]
+    ta = [0.5 + 0.25 / (t - 0.5) for t in taus] if trt else None
+    f0 = [L.equilibrium_populations(L.D2Q9(), *_vortices(*s, seed=k)) for k, s in enumerate(sizes)]
+
+    def run(storage, shape):
+        b = L.LatticeBatch(L.D2Q9(), sizes, taus, ta, storage=storage)
+        for k, f in enumerate(f0):
+            b.upload(k, f)
+        b.set_launch(*shape)
+        b.simulate(200)
+        return [b.download(k) for k in range(len(sizes))]
+
+    ref, many, one = run("f64", (0, 0)), run("f32", (0, 0)), run("f32", (128, 0))
+    for k in range(len(sizes)):
+        e = [np.linalg.norm(x[k] - ref[k]) for x in (many, one)]
+        assert e[0] <= 1.05 * e[1], (taus[k], e)
+
+
+@pytest.mark.parametrize("storage", ["f16neq", "bf16neq"])
+@pytest.mark.parametrize("qid", [4, 5, 9])
+@pytest.mark.parametrize("coll,tau", [(0, 0.6), (0, 0.643), (0, 0.8), (1, 0.6), (1, 0.678),
+                                      (1, 0.728), (1, 0.9)])
+def test_neq_drift_no_larger_than_single_steps(storage, qid, coll, tau):
+    """the same for the 16-bit storages, 200 steps on 1000 x 900"""
+    L = _L()
+    q = L.Quadratures[f"D2Q{qid}"]()
+    f0 = L.equilibrium_populations(q, *_vortices(1000, 900, seed=qid))
+    cm = L.SRT(tau) if coll == 0 else L.trt_magic(tau)
+
+    def run(st, fn):
+        m = L.LatticeBoltzmannModel.from_populations(q, f0, cm, storage=st)
+        fn(m)
+        return m.f_stream.to_numpy()
+
+    ref = run("f64", lambda m: L.simulate(m, range(200)))
+    many = np.linalg.norm(run(storage, lambda m: L.simulate(m, range(200))) - ref)
+    one = np.linalg.norm(run(storage, lambda m: L.simulate_launch_times(m, 200)) - ref)
+    assert many <= 1.05 * one, (many / one)
