@@ -89,8 +89,8 @@ __device__ __forceinline__ void adj_moments(const typename ST::T (&f)[QT<QID>::Q
 // opposite pair (i, o) at a time: with ud = u . c_i, q = s^2/2 ud^2 - s/2 u^2,
 // feq_i +- feq_o = 2 w rho (1 + q), 2 w rho s ud, and the sums and differences
 // of nu give the pair's terms of A and B at once (B is divided by rho, which
-// cancels rho in dfeq/du).  D2Q9 SRT FP64: 230 arithmetic instructions instead
-// of 342.
+// cancels rho in dfeq/du).  D2Q9 SRT FP64: 238 arithmetic instructions instead
+// of 339.
 template <int QID, class ST, int COLL>
 __device__ __forceinline__ void adj_node_pairs(const typename ST::T (&f)[QT<QID>::Q],
                                                const typename ST::T (&mu)[QT<QID>::Q],
@@ -286,10 +286,12 @@ k_adj_step(const typename ST::T *__restrict__ lam_next, const typename ST::store
 // writes lambda, 27 populations a node; here lambda moves once per launch.
 // Same operations in the same order per node and step: in FP64 the bits of
 // single steps (FP32: another contraction of products and sums).
-// Bound by the pulls of the state: a tile's 22 columns touch three 128-byte
-// lines a row, so neighbouring tiles share most lines and run on one XCD, with
-// one L2 (consecutive workgroups go to the 8 XCDs in turn; the tiles are dealt
-// in 8 contiguous chunks).  D2Q9 SRT FP64 / FP32, us a step, single steps with
+// Bound by the pulls of the state (512^2 FP64, four steps: 103 MB in 26 us, waves
+// waiting 44 % of their cycles, the vector ALU issuing 45 % of the time): a tile's
+// 22 columns touch three 128-byte lines a row, so neighbouring tiles share most
+// lines and run on one XCD, with one L2 (consecutive workgroups go to the 8 XCDs
+// in turn; the tiles are dealt in 8 contiguous chunks).  D2Q9 SRT FP64 / FP32, us
+// a step, single steps with
 // the plain node sum 12.9 in FP64: single steps 11.3 / 9.6 on 512^2, 5.2 / 4.9
 // on 128^2; four steps, tiles dealt in turn 11.0 / 7.5 and 2.5 / 1.7; in chunks
 // 7.5 / 4.4 and 2.4 / 1.7.  Two blocks fit a CU (128 registers); 26 x 26 tiles

@@ -521,13 +521,14 @@ struct MultiPlan {
 // F64, F32 and the non-equilibrium ones, automatic launch shape (a launch
 // shape set by the caller names a single-step kernel).  Measured on MI355X,
 // D2Q9 TRT, us per step (single-step kernel -> the one chosen):
-//   FP64: 64^2 4.5 -> 1.1 and 128^2 4.8 -> 1.3 (8 x 8 tiles, 8 steps);
-//     257^2 5.4 -> 2.6 (64 x 16 blocks); 512^2 10.3 -> 4.1 (64 x 32 blocks);
-//     1024^2 33.8 -> 12.3 (wide blocks; marching waves 16.1);
-//     2048^2 116 -> 41 (marching waves; wide blocks 50); 4096^2 413 -> 130;
-//   FP32: 64^2 4.0 -> 0.8; 257^2 4.5 -> 1.6; 512^2 6.0 -> 2.3; 1024^2 17.6 ->
-//     6.1 (march 7.6); 2048^2 64 -> 18 (blocks 20.5); 4096^2 218 -> 57;
-//   FP16-NEQ: 4096^2 194 -> 71 (two columns per lane: even widths).
+//   FP64: 64^2 4.6 -> 1.2 and 128^2 4.9 -> 1.2 (8 x 8 tiles, 8 steps); 257^2
+//     6.4 -> 1.9 (64 x 16 blocks); 512^2 10.4 -> 3.5 (64 x 32 blocks); 1024^2
+//     33.6 -> 10.0 (wide blocks); 2048^2 116 -> 34 (marching waves); 4096^2
+//     415 -> 121;
+//   FP32: 64^2 4.0 -> 0.8; 257^2 5.6 -> 1.2; 512^2 6.2 -> 1.8; 1024^2 17.2 ->
+//     6.1; 2048^2 62 -> 16 (blocks); 4096^2 203 -> 57;
+//   FP16-NEQ (two columns per lane: even widths): 1024^2 18.7 -> 14.1, 2048^2
+//     51 -> 25, 4096^2 167 -> 77.
 // Below this many nodes the 16-bit storages keep the single-step row kernel: a
 // small lattice is a round of few waves, whose serial chain of rows bounds a
 // pass, and a wave at a wall has the longest.  Runs of 41 steps, time over
@@ -546,8 +547,9 @@ long long neq_march_nodes(int nx, int walls) {
 // blocks (one per CU), by its steps; microseconds, D2Q9 TRT, measured on 100^2
 // .. 1400^2 and 2000 x 150.  The first round's slope within it is small, so a
 // lattice wants the kernel and the steps that just fill a whole number of
-// rounds: 300^2 FP64 has 300 blocks of 64 x 16 at 6 steps (3.5 us a step) and
-// 228 at 5 (2.25); 560^2 273 of 64 x 32 at 6 (6.8) and 252 at 5 (4.3).
+// rounds: 300^2 FP64 has 300 blocks of 64 x 16 at 6 steps (3.75 us a step by the
+// table) and 228 at 5 (2.24; 2.08 measured), 560^2 286 of 64 x 32 at 6 (7.3) and
+// 240 at 5 (4.24; 3.75 measured).
 struct BlockCost {
     int kernel, rows, tmax;
     double a[9], b[9];
@@ -582,7 +584,7 @@ void plan_blocks(MultiPlan &pl, const BlockCost &c, const lbm_field_s *f, bool f
     }
 }
 
-// lattices for the 8 x 8 tiles (420 of them: 164 x 164; us a step on 160^2
+// lattices for the 8 x 8 tiles (420 of them: 168 x 160; us a step on 160^2
 // against the 64 x 16 blocks: 1.66 / 1.79 in FP64, 0.95 / 1.09 in FP32)
 bool small_tiles(const lbm_field_s *f) {
     return (long long)((f->nx + 7) / 8) * ((f->ny + 7) / 8) <= 420;
@@ -673,7 +675,7 @@ MultiPlan multi_plan(const lbm_model_s *m, const lbm_field_s *f) {
     // waves and blocks are 64 columns wide and recompute a halo of rows: a
     // lattice much narrower or lower than that spends its time on nodes that
     // are not written, and the single-step kernel is faster (FP64 at 32
-    // columns: blocks 7 us against 10 for 270,000 nodes; at 24 they lose)
+    // columns: blocks 5 us against 13 for 270,000 nodes; at 24 they lose)
     const bool wide = f->nx >= 32 && f->ny >= 12;
     if (rows_mode(f->storage)) {
         int walls = 0;

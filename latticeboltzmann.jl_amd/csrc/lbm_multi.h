@@ -182,7 +182,8 @@ __device__ __forceinline__ void collide_pairs(double (&f)[QT<QID>::Q], const Ste
 // relaxation uses again; with the even and odd parts of the pair's
 // equilibrium (ev, od as in collide_neq_pairs), ns = (g_i + g_j) - 2 w ev and
 // na = (g_i - g_j) - 2 w od are the relaxed parts: g_i - ns / (2 tau_s) -
-// na / (2 tau_a).  D2Q9 TRT: 66 instructions per node instead of 92.
+// na / (2 tau_a).  D2Q9 TRT: 71 arithmetic instructions per node instead of 102,
+// SRT 76 instead of 89 (form 7 and 6, see multi_form).
 template <int QID, int COLL, class F, class H, int... Is>
 __device__ __forceinline__ void collide_pairs(float (&f)[QT<QID>::Q], const StepParams<float> &p,
                                               const MultiConsts<float> &mc, F &&force, H &&before,
@@ -441,6 +442,9 @@ unsigned deal_tiles(A &a, int tiles_y) {
 // keeps its place: a thread pulls its nodes into registers, the block meets,
 // and the results overwrite the buffer.  `first`: the run's first step, level
 // 1 collides the canonical state S_0 of its own node instead of pulling.
+// 64^2 FP64, eight steps: 9 to 10 us on 64 of 256 CUs, whose waves wait 54 % of
+// their cycles at the two barriers of a level and for LDS; the vector ALU issues
+// a quarter of the time.
 struct TileArgs {
     int levels;
     int tiles_x, tiles, chunk;
@@ -640,6 +644,9 @@ __device__ __forceinline__ double lane_shift(double v) {
 // buffers, one barrier per level).  Every level computes the whole region; its
 // outermost ring of valid nodes is lost each time, so T levels write the inner
 // 64 - 2 (T - 1) columns and NW R - 2 (T - 1) rows.
+// 1024^2 FP64, five steps: 57 us for 158 MB, the vector ALU issuing 63 % of the
+// time; 1021 x 517 FP32, six steps: 22 us in 456 blocks of 16 waves, 60 %, the
+// waves waiting 44 % of their cycles, at the levels' barriers above all.
 struct BlockArgs {
     int levels;
     int tiles_x, tiles, chunk;
@@ -824,7 +831,8 @@ k_block_all(const typename ST::store_t *__restrict__ C, const LevelOut o,
 
 // Batched lattices: one region per block from a table; the lattice record is
 // read in place with a wave-uniform index (scalar loads).  Bound by FP
-// arithmetic like k_block; 512 lattices of 200 x 200, us a step against the
+// arithmetic (the vector ALU issues 87 % of the time, 48 lattices of 32^2 ..
+// 512^2 in FP32); 512 lattices of 200 x 200, us a step against the
 // single-step kernel's: 194 / 510 in FP64, 90 / 303 in FP32 (single steps are
 // bound by the passes over the pool, 2.9 and 2.4 TB/s there).
 template <int QID, int COLL, class ST, int NW, int R>
@@ -892,6 +900,12 @@ struct MarchShape {
     static constexpr int LINE = slot0(QT<QID>::Q);  // slots per kept level
 };
 
+// 4096^2, a pass: FP64 five steps 2.81 GB (1.16 times one read and one write) at
+// 4.2 TB/s, the vector ALU issuing 74 % of the time: either alone would take
+// two thirds to three quarters of it, and the waves of the one resident round
+// end at different times (1.9 of 3 a SIMD on average).  FP32 six steps 1.57 GB,
+// FP16-NEQ four steps 1.05 GB: the ALU issues all the time (91 % and more).
+//
 // The kept rows of a level, y - 1 (and y - 2 for the populations that moved
 // up), while row y arrives: populations with c_x = 0 in registers (they are
 // read by the same lane), the others in the wave's own LDS, where the reader
