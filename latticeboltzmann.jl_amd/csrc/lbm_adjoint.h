@@ -286,9 +286,9 @@ k_adj_step(const typename ST::T *__restrict__ lam_next, const typename ST::store
 // writes lambda, 27 populations a node; here lambda moves once per launch.
 // Same operations in the same order per node and step: in FP64 the bits of
 // single steps (FP32: another contraction of products and sums).
-// Bound by the pulls of the state (512^2 FP64, four steps: 103 MB in 26 us, waves
-// waiting 44 % of their cycles, the vector ALU issuing 45 % of the time): a tile's
-// 22 columns touch three 128-byte lines a row, so neighbouring tiles share most
+// Bound by the pulls of the state (512^2 FP64, launches of three and four steps:
+// 103 MB in 26 us, waves waiting 44 % of their cycles, the vector ALU issuing 45 %
+// of the time): a tile's 22 columns touch three 128-byte lines a row, so neighbouring tiles share most
 // lines and run on one XCD, with one L2 (consecutive workgroups go to the 8 XCDs
 // in turn; the tiles are dealt in 8 contiguous chunks).  D2Q9 SRT FP64 / FP32, us
 // a step, single steps with

@@ -224,7 +224,7 @@ processing_view(pm, f::HipLattice) =
 # the processing method (0 without one), and is followed by next!(model, t + 1);
 # the loop ends with the reference's closing next!(model, last(time) + 1).
 # Runs of steps between the points where next! reads the state go to one
-# lbm_simulate call (one fused collide-stream kernel per step).  A model with
+# lbm_simulate call (fused kernels of one or several steps).  A model with
 # a force closure advances one step per call instead, the closure evaluated at
 # that step's time, as the reference's per-node force(x, y, t * Δt)
 # (srt.jl:52, trt.jl:77, mrt.jl:92) is.
