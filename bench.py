@@ -99,6 +99,12 @@ def pass_figures(L, model, steps, kernel_ms, nlaunch):
     return kernel, kernel_ms / passes, (steps if kernel else nlaunch) / passes
 
 
+def step_us(L, model, steps):
+    """Kernel microseconds (of a step, of a pass) over a timed run"""
+    _, ms, per_pass = pass_figures(L, model, steps, *L.simulate_timed(model, steps))
+    return (1e3 * ms / per_pass if per_pass else 0.0), 1e3 * ms
+
+
 def copy_rate(L, f, copies=COPY_LAUNCHES):
     """Rate of a plain device copy of the same bytes on the same GPU
     (``lbm_field_copy``: 16-byte lanes, non-temporal stores), ``copies``
@@ -402,8 +408,8 @@ def mrt_leg(L, steps=20):
     """Regularised MRT (mrt.jl:56-118) in FP64 on the periodic Taylor-Green
     vortex, D2Q9 at 4096^2 and D2Q17 / D2Q37 at 8192 x 2048, all relaxation
     times 0.8, beside SRT(0.8) on the same lattice: kernel time per step from
-    HIP events and the fraction of 8 TB/s at 2 Q 8 bytes per node and step (more
-    than what moves where a pass advances several steps)."""
+    HIP events and the fraction of 8 TB/s at 2 Q 8 bytes per node and pass (of
+    one or several steps)."""
     rows = []
     for qid, nx, ny in ((9, 4096, 4096), (17, 8192, 2048), (37, 8192, 2048)):
         q = L.Quadratures[f"D2Q{qid}"]()
@@ -423,9 +429,8 @@ def mrt_leg(L, steps=20):
             if name == "MRT-MFMA":
                 m.launch = (256, 1, 16, 1)
             L.simulate(m, range(3))
-            ms, nl = L.simulate_timed(m, steps)
-            us = ms / max(nl, 1) * 1e3
-            gbs = 2 * q.Q * 8 * nx * ny / (us * 1e-6) / 1e9
+            us, pass_us = step_us(L, m, steps)
+            gbs = _rate(2 * q.Q * 8 * nx * ny, pass_us * 1e-3)
             rows.append({"quadrature": f"D2Q{qid}", "lattice": [nx, ny], "collision": name,
                          "us_per_step": round(us, 1), "mlups": round(nx * ny / us, 1),
                          "achieved_GBps": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4)})
@@ -437,8 +442,8 @@ def mrt_leg(L, steps=20):
 def sizes_leg(L, sizes, steps=20):
     """D2Q9 TRT(0.8, 1.1) on periodic n x n lattices (uniform flow 0.01 along
     x, equilibrium start) in FP64 and FP32: kernel time per step from HIP
-    events and algorithmic GB/s (2 Q sizeof per node and step; several steps
-    share a pass)."""
+    events and algorithmic GB/s (2 Q sizeof per node and pass of one or several
+    steps)."""
     q = L.D2Q9()
     rows = []
     for n in sizes:
@@ -449,9 +454,8 @@ def sizes_leg(L, sizes, steps=20):
             m = L.LatticeBoltzmannModel.from_populations(q, f0, L.TRT.fields(0.8, 1.1),
                                                          storage=storage)
             L.simulate(m, range(3))
-            ms, nl = L.simulate_timed(m, steps)
-            us = ms / max(nl, 1) * 1e3
-            gbs = 2 * q.Q * eb * n * n / (us * 1e-6) / 1e9
+            us, pass_us = step_us(L, m, steps)
+            gbs = _rate(2 * q.Q * eb * n * n, pass_us * 1e-3)
             rows.append({"lattice": [n, n], "storage": storage,
                          "us_per_step": round(us, 1), "achieved_GBps": round(gbs, 1),
                          "frac": round(gbs / HBM_PEAK_GBS, 4)})
@@ -491,7 +495,7 @@ def precision_leg(L, steps, nx=8192, ny=2048, tau=0.8, qids=(9, 17, 37),
                 m = L.LatticeBoltzmannModel.from_populations(q, f0, cm, bcs, storage=st)
                 L.synchronize()
                 t0 = time.perf_counter()
-                kms, nl = L.simulate_timed(m, steps)
+                kus, _ = step_us(L, m, steps)
                 L.synchronize()
                 wall = time.perf_counter() - t0
                 mom = L.moments(m.f_stream, stress=False)
@@ -505,7 +509,7 @@ def precision_leg(L, steps, nx=8192, ny=2048, tau=0.8, qids=(9, 17, 37),
                 row = {"quadrature": f"D2Q{qid}", "flow": flow, "storage": st, "steps": steps,
                        "rel_l2_vs_f64": e64, "rel_l2_vs_analytic": ea,
                        "mlups": round(nx * ny * steps / wall / 1e6, 1),
-                       "fused_kernel_ms": round(kms / max(nl, 1), 5),
+                       "fused_kernel_ms": round(kus * 1e-3, 5),
                        "u_max": float(np.abs(ux).max())}
                 rows.append(row)
                 print(json.dumps(row), flush=True)

@@ -231,11 +231,13 @@ int lbm_simulate(lbm_model m, lbm_field f_stream, lbm_field f_collision, int64_t
 int lbm_simulate_timed(lbm_model m, lbm_field f_stream, lbm_field f_collision, int64_t nsteps,
                        double *ms_total, int64_t *nlaunch);
 /* Measurement support; no counterpart in the reference; needs no GPU.  What a run
- * of nsteps does with the automatic launch shape: *kernel names the kernel that
- * advances several steps per pass ("" for one step per launch), *passes is the
- * number of launches that lbm_simulate_timed times. */
+ * of nsteps does with a launch shape (lbm_model_set_launch's numbers; 0, 0, 0, -1:
+ * automatic): *kernel names the kernel that advances several steps per pass (""
+ * for one step per launch), *passes is the number of launches that
+ * lbm_simulate_timed times. */
 int lbm_simulate_plan(int quadrature, int storage, int collision, int nx, int ny, const lbm_bc *bcs,
-                      int nbc, int64_t nsteps, const char **kernel, int64_t *passes);
+                      int nbc, int block_x, int rows_per_block, int nodes_per_thread,
+                      int nontemporal, int64_t nsteps, const char **kernel, int64_t *passes);
 /* Measurement support; no counterpart in the reference.  As lbm_simulate with
  * one fused step per launch and a HIP event before every fused launch: launch_ms[k] (nsteps - 1
  * entries) is the time from the start of fused launch k to the start of the

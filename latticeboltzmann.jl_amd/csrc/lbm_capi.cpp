@@ -1511,7 +1511,8 @@ int lbm_simulate_timed(lbm_model m, lbm_field f_stream, lbm_field f_collision, i
 }
 
 int lbm_simulate_plan(int quadrature, int storage, int collision, int nx, int ny, const lbm_bc *bcs,
-                      int nbc, int64_t nsteps, const char **kernel, int64_t *passes) {
+                      int nbc, int block_x, int rows_per_block, int nodes_per_thread,
+                      int nontemporal, int64_t nsteps, const char **kernel, int64_t *passes) {
     if (kernel) *kernel = "";
     if (passes) *passes = 0;
     HostQuad q;
@@ -1527,6 +1528,8 @@ int lbm_simulate_plan(int quadrature, int storage, int collision, int nx, int ny
     m.qid = quadrature;
     m.coll = collision;
     m.bcs.assign(bcs, bcs + nbc);
+    if (int rc = lbm_model_set_launch(&m, block_x, rows_per_block, nodes_per_thread, nontemporal))
+        return rc;
     lbm_field_s f;
     f.qid = quadrature;
     f.nx = nx;

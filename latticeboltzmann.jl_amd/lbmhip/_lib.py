@@ -119,7 +119,7 @@ def lib() -> ctypes.CDLL:
         getattr(L, name).argtypes = [vp, vp, vp]
     L.lbm_simulate.argtypes = [vp, vp, vp, i64]
     L.lbm_simulate_timed.argtypes = [vp, vp, vp, i64, dp, ctypes.POINTER(i64)]
-    L.lbm_simulate_plan.argtypes = [i, i, i, i, i, ctypes.POINTER(LbmBC), i, i64,
+    L.lbm_simulate_plan.argtypes = [i, i, i, i, i, ctypes.POINTER(LbmBC), i, i, i, i, i, i64,
                                     ctypes.POINTER(ctypes.c_char_p), ctypes.POINTER(i64)]
     L.lbm_simulate_launch_times.argtypes = [vp, vp, vp, i64, dp, ctypes.POINTER(i64)]
     L.lbm_moments.argtypes = [vp, d, dp, dp, dp, dp, dp, dp]

@@ -28,7 +28,7 @@ from . import _lib
 from .boundary_conditions import BoundaryCondition
 from .collision_models import CollisionModel
 from .lattice import HipLattice
-from .operators import apply_, collide_, native_model, stream_
+from .operators import apply_, collide_, launch_key, native_model, stream_
 from .quadratures import Quadrature
 
 
@@ -163,9 +163,9 @@ def simulate_timed(model: LatticeBoltzmannModel, nsteps: int):
 
 
 def simulate_plan(model: LatticeBoltzmannModel, nsteps: int):
-    """What ``simulate_timed(model, nsteps)`` does with the automatic launch
-    shape: (kernel that advances several steps per pass, "" for one step per
-    launch; number of launches timed)."""
+    """What ``simulate_timed(model, nsteps)`` does: (kernel that advances
+    several steps per pass, "" for one step per launch; number of launches
+    timed)."""
     import ctypes
 
     kinds = {"SRT": _lib.SRT_KIND, "TRT": _lib.TRT_KIND, "MRT": _lib.MRT_KIND}
@@ -174,8 +174,9 @@ def simulate_plan(model: LatticeBoltzmannModel, nsteps: int):
     kernel, passes = ctypes.c_char_p(), ctypes.c_int64()
     _lib.check(_lib.lib().lbm_simulate_plan(model.quadrature.id, _lib.STORAGES[f.storage],
                                             kinds[type(model.collision_model).__name__], f.nx, f.ny,
-                                            arr, len(bcs), int(nsteps), ctypes.byref(kernel),
-                                            ctypes.byref(passes)), "lbm_simulate_plan")
+                                            arr, len(bcs), *launch_key(model.launch), int(nsteps),
+                                            ctypes.byref(kernel), ctypes.byref(passes)),
+               "lbm_simulate_plan")
     return kernel.value.decode(), passes.value
 
 

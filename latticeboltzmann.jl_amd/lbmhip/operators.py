@@ -26,6 +26,17 @@ from .lattice import HipLattice
 from .quadratures import Quadrature
 
 
+def launch_key(launch) -> tuple:
+    """(threads per block along x, rows per block, nodes per thread,
+    non-temporal) of the fused step; None = automatic.  A 3-tuple omits the rows
+    (one row per block)."""
+    if launch is None:
+        return (0, 0, 0, -1)
+    if len(launch) == 3:
+        launch = (launch[0], 1, launch[1], launch[2])
+    return tuple(int(k) for k in launch)
+
+
 class NativeModel:
     """An ``lbm_model`` handle (collision model + force + BC list) that is
     reconfigured only when the requested configuration changes."""
@@ -117,12 +128,8 @@ class NativeModel:
         self._bcs_key = key
 
     def set_launch(self, launch) -> None:
-        """(threads per block along x, rows per block, nodes per thread,
-        non-temporal) of the fused step; None = automatic.  A 3-tuple omits
-        the rows (one row per block)."""
-        if launch is not None and len(launch) == 3:
-            launch = (launch[0], 1, launch[1], launch[2])
-        key = tuple(launch) if launch is not None else (0, 0, 0, -1)
+        """see launch_key"""
+        key = launch_key(launch)
         if key != self._launch_key:
             _lib.check(_lib.lib().lbm_model_set_launch(self._h, *[int(k) for k in key]),
                        "lbm_model_set_launch")

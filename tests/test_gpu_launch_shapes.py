@@ -122,10 +122,9 @@ def test_timed_runs_count_their_fused_steps(qid, shape, launch):
         ms, n = L.simulate_timed(a, steps)
         assert n == (max(steps - 2, 0) if one_pass else steps - 1)
         assert ms > 0 or n == 0
-        if launch is None:
-            kernel, passes = L.simulate_plan(a, steps)
-            assert bool(kernel) == (qid != 13 and steps >= 2)
-            assert passes == n if not kernel else (steps + 7) // 8 <= passes <= steps - 1
+        kernel, passes = L.simulate_plan(a, steps)
+        assert bool(kernel) == (qid != 13 and steps >= 2 and launch is None)
+        assert passes == n if not kernel else (steps + 7) // 8 <= passes <= steps - 1
         L.simulate(b, range(steps))
         assert np.array_equal(a.f_stream.to_numpy(), b.f_stream.to_numpy())
         assert np.array_equal(a.f_collision.to_numpy(), b.f_collision.to_numpy())

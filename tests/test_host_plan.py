@@ -9,7 +9,7 @@ import lbmhip._lib as lib
 SRT, TRT, MRT = 0, 1, 2
 
 
-def plan(qid, storage, coll, nx, ny, nsteps, walls=()):
+def plan(qid, storage, coll, nx, ny, nsteps, walls=(), launch=(0, 0, 0, -1)):
     """walls: directions (0 N, 1 E, 2 S, 3 W) of bounce-back walls"""
     arr = (lib.LbmBC * max(1, len(walls)))()
     for k, d in enumerate(walls):
@@ -17,7 +17,7 @@ def plan(qid, storage, coll, nx, ny, nsteps, walls=()):
         arr[k].x0, arr[k].x1, arr[k].y0, arr[k].y1 = 1, nx, 1, ny
     kernel, passes = ctypes.c_char_p(), ctypes.c_int64()
     rc = lib.lib().lbm_simulate_plan(qid, lib.STORAGES[storage], coll, nx, ny, arr, len(walls),
-                                     nsteps, ctypes.byref(kernel), ctypes.byref(passes))
+                                     *launch, nsteps, ctypes.byref(kernel), ctypes.byref(passes))
     assert rc == 0, lib.lib().lbm_last_error()
     return kernel.value.decode(), passes.value
 
@@ -66,9 +66,18 @@ def test_two_steps_on_whole_tiles():
 
 def test_plan_errors():
     L, bc = lib.lib(), (lib.LbmBC * 1)()
-    for args in ((10, 0, 0, 8, 8, bc, 0, 3), (9, 99, 0, 8, 8, bc, 0, 3), (9, 0, 3, 8, 8, bc, 0, 3),
-                 (9, 0, 0, 0, 8, bc, 0, 3), (9, 0, 0, 8, 8, None, 1, 3), (9, 0, 0, 8, 8, bc, 0, -1)):
-        assert L.lbm_simulate_plan(*args, None, None) < 0
+    for *args, steps in ((10, 0, 0, 8, 8, bc, 0, 3), (9, 99, 0, 8, 8, bc, 0, 3),
+                         (9, 0, 3, 8, 8, bc, 0, 3), (9, 0, 0, 0, 8, bc, 0, 3),
+                         (9, 0, 0, 8, 8, None, 1, 3), (9, 0, 0, 8, 8, bc, 0, -1)):
+        assert L.lbm_simulate_plan(*args, 0, 0, 0, -1, steps, None, None) < 0
+    assert L.lbm_simulate_plan(9, 0, 0, 8, 8, bc, 0, 96, 0, 0, -1, 3, None, None) < 0
+
+
+def test_plan_of_a_launch_shape():
+    assert plan(9, "f32", TRT, 300, 250, 9, launch=(256, 1, 1, 1)) == ("", 8)
+    assert plan(9, "f32", TRT, 320, 240, 9, launch=(256, 1, 1, 0)) == ("", 7)
+    assert plan(9, "f32", TRT, 300, 250, 9, launch=(128, 1, 1, -1)) == ("", 8)
+    assert plan(9, "f32", TRT, 300, 250, 9, launch=(256, 1, 1, -1))[0] == "k_block"
 
 
 @pytest.mark.parametrize("qid,storage", [(4, "f64"), (5, "f32"), (9, "f32"), (9, "f16neq"),
@@ -92,7 +101,7 @@ def test_bench_prices_the_passes_that_run(n, storage, steps, kernel, passes, per
 
     import bench
     import lbmhip as L
-    model = SimpleNamespace(quadrature=L.D2Q9(), boundary_conditions=[],
+    model = SimpleNamespace(quadrature=L.D2Q9(), boundary_conditions=[], launch=None,
                             collision_model=L.TRT.fields(0.6, 1.3),
                             f_stream=SimpleNamespace(storage=storage, nx=n, ny=n))
     counted = passes if not kernel else steps - 1
